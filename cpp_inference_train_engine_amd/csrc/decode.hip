@@ -13,6 +13,8 @@
 // decode_page_kernel -- the production kernel (H <= 16, kv_rank 128, rope 16,
 //   64-token tiled pages): one wave per page with all of the page's loads in
 //   flight at once, MFMA scores and PV.
+// Other tiled shapes: decode_wide_kernel (decode_wide.hip), attend_tile_kernel
+//   (attend_tile.hip).
 // decode_generic_kernel -- any H / kv_rank / rope / page size / layout: one
 //   256-thread block per (work item, head), VALU fp32.
 // merge_kernel -- log-sum-exp combine of the split partials of either kernel, one
@@ -740,6 +742,8 @@ hipError_t launch_decode_partials(const DecodeArgs& a, int dtype, bool force_gen
         return dtype == 0 ? launch_page<F16>(a, grid, stream) : launch_page<BF16>(a, grid, stream);
     if (!force_generic && decode_wide_supported(a.H, a.kv_rank, a.rope_dim, a.page_size))
         return launch_decode_wide(a, dtype, stream);
+    if (!force_generic && attend_tile_supported(a.kv_rank, a.rope_dim, a.page_size))
+        return launch_decode_tile(a, dtype, stream);
     const size_t shmem = (a.kv_rank + a.rope_dim + kGenChunk + 8) * sizeof(float);
     const dim3 g(grid, a.H);
     if (dtype == 0)

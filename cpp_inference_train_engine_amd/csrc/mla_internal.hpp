@@ -130,6 +130,12 @@ inline bool decode_fuses_merge(const DecodeArgs& a, bool generic) {
 // The DeepSeek-like shape (16 < H <= 128, kv_rank 512, rope 64, 64-token pages).
 bool decode_wide_supported(int H, int kv_rank, int rope_dim, int page_size);
 hipError_t launch_decode_wide(const DecodeArgs& a, int dtype, hipStream_t stream);
+// Any tiled record with kv_rank <= 512 and rope_dim <= 64 (attend_tile.hip): the shapes the
+// kernels above do not cover.
+bool attend_tile_supported(int kv_rank, int rope_dim, int page_size);
+hipError_t launch_decode_tile(const DecodeArgs& a, int dtype, hipStream_t stream);
+hipError_t launch_prefill_tile(const PrefillArgs& a, int max_q_len, int dtype,
+                               hipStream_t stream);
 // Prefill attention for the sessions with q_len > 1 (max_q_len >= their q_len).
 hipError_t launch_prefill(const PrefillArgs& a, int max_q_len, int dtype, bool force_generic,
                           hipStream_t stream);

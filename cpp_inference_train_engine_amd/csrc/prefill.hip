@@ -34,6 +34,7 @@
 //                       a+8, a+12)
 //   This work is MFMA-bound (512 queries x 8 heads over a 2k context is ~6k flop per
 //   cached byte).
+// Other tiled shapes: attend_tile_kernel (attend_tile.hip).
 // prefill_generic_kernel -- any H / kv_rank / rope / page size / layout: one
 //   256-thread block per (query row, head), VALU fp32.
 #include "mla_common.hpp"
@@ -521,6 +522,8 @@ hipError_t launch_prefill(const PrefillArgs& a, int max_q_len, int dtype, bool f
     if (!force_generic && prefill_mfma_supported(a.H, a.kv_rank, a.rope_dim, a.page_size))
         return dtype == 0 ? launch_prefill_page<F16>(a, max_q_len, stream)
                           : launch_prefill_page<BF16>(a, max_q_len, stream);
+    if (!force_generic && attend_tile_supported(a.kv_rank, a.rope_dim, a.page_size))
+        return launch_prefill_tile(a, max_q_len, dtype, stream);
     const size_t shmem = (a.kv_rank + a.rope_dim + kPgChunk + 8) * sizeof(float);
     const dim3 grid(max_q_len, a.B, a.H);
     if (dtype == 0)
