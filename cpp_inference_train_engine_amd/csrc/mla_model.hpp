@@ -26,11 +26,10 @@ struct ModelDims {
     int max_seq;   // max_sequence_length: RoPE table rows
     // padded sizes (K dimensions to 32, N dimensions to 16; see above)
     int d_pad;      // d_model -> 32
-    int q_pad;      // q_rank -> 32 (N of w_dq, K of w_uq)
+    int q_pad;      // q_rank -> 32 (N of w_dq, K of w_q)
     int kvw_pad;    // kv_rank + rope -> 16 (N of w_dkv)
-    int qk_pad;     // qk -> 16 (per-head N of w_uq)
-    int nope_pad;   // nope -> 32 (K of the absorption)
-    int kv_pad;     // kv_rank -> 16 (N of the absorption)
+    int kv_pad;     // kv_rank -> 16 (a head's latent columns of w_q)
+    int hq_pad;     // kv_pad + (rope -> 16): a head's columns of w_q
     int ctx_pad;    // H * kv_rank -> 32 (K of the output projection)
     int ff_pad;     // d_ff -> 32 (N of gate/up, K of down)
     int vocab_pad;  // vocab -> 16 (N of the tied logits)
@@ -39,8 +38,8 @@ struct ModelDims {
 struct LayerWeights {
     const float *attn_norm, *q_norm, *kv_norm, *ffn_norm;
     const uint16_t* w_dq_dkv;   // [d x (q_pad + kvw_pad)] tiled: q columns, then kv columns
-    const uint16_t* w_uq;       // [q_rank x H*qk_pad] tiled, head h at columns h*qk_pad..
-    const uint16_t* w_uk;       // H blocks [nope x kv_rank] tiled (W_uk_h^T)
+    const uint16_t* w_q;        // [q_rank x H*hq_pad] tiled, head h at columns h*hq_pad..: the
+                                // kv_pad latent columns (W_uq_nope . W_uk_h^T), then rope
     const uint16_t* w_out;      // [H*kv_rank x d] tiled: combined W_uv.W_o
     const uint16_t* w_gate_up;  // [d x 2*ff_pad] tiled, gate/up tiles interleaved
     const uint16_t* w_down;     // [d_ff x d] tiled
@@ -55,10 +54,13 @@ struct StepArgs {
     int num_pool_pages;
     const uint16_t* embed;     // token_embedding [V x d] tiled as the logits W (K=d, N=V)
     const float* final_norm;
+    const uint16_t* zeros;     // 512 fp16 zeros: the weights of k-steps past a K
     const float2* rope_tab;    // [max_seq x rope/2] (cos, sin) of pos * theta^(-j/rope)
     float2* rope_rows;         // [m_pad x rope/2] the table rows of this step's positions
     // activations (rows padded to m_pad)
     float *x, *res, *ctx;       // [m_pad x d_pad], [m_pad x d_pad], [m_pad x H*kv_rank]
+    uint16_t *cqw;              // [m_pad x q_pad] fp16 cq o q_norm
+    float* ckv;                 // [m_pad x kvw_pad] latent o kv_norm, then the key before RoPE
     uint16_t *xw, *resw;        // fp16 x o (next norm weight), res o ffn_norm [m_pad x d_pad]
     uint16_t *u;                // [m_pad x ff_pad] fp16
     uint16_t *q_latent, *q_rope;  // [B x H x kv_rank], [B x H x rope] in the cache dtype
@@ -69,29 +71,22 @@ struct StepArgs {
     int32_t* next_tokens;       // [B]
     // Per-row sums of squares of each 16-column tile of an activation, written by its
     // producer and summed (in tile order) into 1/rms by the RMSNorm-ing consumer.
-    float* ss_x;    // [m_pad x d_pad/16] of x (embed, g6) -> attn_norm (qkv), final_norm (g7)
+    float *ss_cq, *ss_kv;  // [m_pad x q_pad/16], [m_pad x kvw_pad/16] of cq, latent (g1) -> g2
+    float* ss_x;    // [m_pad x d_pad/16] of x (embed, g6) -> attn_norm (g1), final_norm (g7)
     float* ss_res;  // [m_pad x d_pad/16] of res (g4) -> ffn_norm (g5)
-};
-
-// The decode attention's pages, read ahead into L2 by extra workgroups of the qkv launch
-// that precedes it on the stream (page_prefetch, model.hip).  max_work = 0: none.
-struct PagePrefetch {
-    const int32_t *work_desc, *work_pages;  // the attention's work list
-    int max_work;   // work items (the attention's grid), 0 = no read-ahead
-    int pages;      // leading pages of each work item read ahead, <= kWorkPages
-    int page_size;  // tokens per page
-    int record;     // 16-bit words per page record
 };
 
 int g7_parts(const ModelDims& m);
 size_t qkv_lds_bytes(const ModelDims& m);
 hipError_t model_kernel_attributes(const ModelDims& m);
+// Launches of launch_layer_pre for a batch of `rows` rows: 1 (qkv) or 2 (g1, g2).
+int layer_pre_launches(int rows);
 // first_norm: attn_norm of layer 0
 hipError_t launch_embed(const StepArgs& s, const float* first_norm, hipStream_t st);
 hipError_t launch_layer_pre(const StepArgs& s, const LayerWeights& w, uint16_t* pool,
-                            const PagePrefetch& pf, hipStream_t st);  // qkv_kernel (which appends to `pool`)
+                            hipStream_t st);  // qkv, or g1 and g2; appends to `pool`
 // next_norm: attn_norm of the next layer, or final_norm after the last one; next: the
-// next layer's weights (their qkv blocks are prefetched into L2), or null
+// next layer's weights (their g1 blocks are prefetched into L2), or null
 hipError_t launch_layer_post(const StepArgs& s, const LayerWeights& w, const float* next_norm,
                              const LayerWeights* next, hipStream_t st);
 hipError_t launch_logits(const StepArgs& s, hipStream_t st);

@@ -3,12 +3,12 @@
 // each.
 //
 // Per layer, in launch order (y = x.W for every projection, as in ops.cpp:8-18):
-//   qkv_kernel  per 16 rows: RMSNorm(x, attn_norm) . [w_dq | w_dkv], then per head q_norm
-//               -> w_uq -> RoPE of the rope columns (q_rope, stored in the cache dtype)
-//               -> absorption q_latent = W_uk_h^T q_nope (inference.cpp:85-90,121-124;
-//               the MPS graph keeps q_latent in the storage dtype, mps_backend.mm:561);
-//               one more workgroup kv_norms the latent, RoPEs the key, rounds both and
-//               appends them to the paged cache (inference.cpp:91-103)
+//   g1_kernel   RMSNorm(x, attn_norm) . [w_dq | w_dkv]  (inference.cpp:85-95)
+//   g2_kernel   per head, q_norm(cq) . [W_uq_nope . W_uk_h^T | W_uq_rope]: q_latent with the
+//               absorption folded into the weight (inference.cpp:85-90,121-124) and, after
+//               RoPE, q_rope, both stored in the cache dtype as the MPS graph does
+//               (mps_backend.mm:561); one more workgroup kv_norms the latent, RoPEs the key,
+//               rounds both and appends them to the paged cache (inference.cpp:91-103)
 //   (decode attention partials + merge: decode.hip)
 //   g4_kernel   latent_ctx [H*kv_rank] . out_proj + x  (inference.cpp:154-156; out_proj
 //               is the combined W_uv.W_o of prepare_projections, inference.cpp:28-46)
@@ -85,49 +85,6 @@ __device__ __forceinline__ void l2_prefetch(int n, F&& addr, uint16_t* scratch, 
         copy_block_to_lds(addr(k), lane * 16, scratch);
 }
 
-// ---- the decode attention's pages, read ahead during qkv_kernel ----------------------
-// qkv_kernel occupies a few dozen CUs for several microseconds, and the attention that
-// follows it on the stream starts its 40 MB page stream only when qkv ends.  The attention
-// runs work item w with residue w % 8 (decode_page_kernel: one workgroup per item), so the
-// qkv launch gets one more block of 8 columns, and its workgroups of residue x copy the
-// leading pf.pages pages of the items x, x + 8, ... into LDS scratch: the lines land in
-// that XCD's L2, where the attention's page loads then hit.  The page that a decode
-// session's new token is appended to in this same launch (index (k_len - 1) / page_size)
-// is skipped: a copy taken before the append lands would be stale.  Items of prefill
-// sessions (q_len > 1), whose chunk is appended here too, are skipped whole.  Each wave
-// reads the descriptors of its items once (one vector load round), then issues the
-// copies of each valid page, 1 KB per instruction; nothing waits for them.
-__device__ void page_prefetch(const PagePrefetch& pf, const uint16_t* pool, int npool,
-                              uint16_t* scratch, int x, int gw, int nw) {
-    const int lane = threadIdx.x & 63;
-    const int items = x < pf.max_work ? (pf.max_work - 1 - x) / kXcds + 1 : 0;
-    const int pairs = items * pf.pages, bytes = pf.record * 2;
-    const uint32_t lds = lds_u32(scratch + (threadIdx.x >> 6) * 512);
-    for (int r0 = gw; r0 < pairs; r0 += 64 * nw) {
-        const int p = r0 + nw * lane;  // this lane's (item, page) pair of the round
-        bool ok = false;
-        int page = 0;
-        if (p < pairs) {
-            const int t = p / pf.pages, j = p % pf.pages, w = x + kXcds * t;
-            const int32_t* d = pf.work_desc + (long long)w * kWorkDescInts;
-            const int sess = d[0], kl = d[2], first = d[3], end = d[4], q_len = d[7];
-            page = pf.work_pages[(long long)w * kWorkPages + j];
-            ok = sess >= 0 && q_len == 1 && first + j < end &&
-                 first + j != (kl - 1) / pf.page_size && (unsigned)page < (unsigned)npool;
-        }
-        // The ids are read here, once: a wait for them inside the loop below would also
-        // wait for the copies already issued (vmcnt retires in order).
-        asm volatile("" ::"v"(page));
-        for (uint64_t m = __ballot(ok); m; m &= m - 1) {
-            const int pg = __builtin_amdgcn_readlane(page, __builtin_ctzll(m));
-            const uint16_t* base = pool + (long long)pg * pf.record;
-            for (int b = 0; b * 1024 < bytes; ++b)
-                if (b * 1024 + lane * 16 < bytes)
-                    copy_block_to_lds_at(base + b * 512, lane * 16, lds);
-        }
-    }
-}
-
 // Sums over aligned groups of G = 4, 8 or 16 lanes of a 16-lane row, left in every lane
 // of the group, on DPP lane moves (VALU) instead of LDS permutes: the two quad swaps give
 // every lane its quad's sum, then the half-row mirror pairs the quads of each half and the
@@ -163,71 +120,77 @@ __device__ __forceinline__ void zero(floatx4 (&acc)[MT][NT]) {
 
 // ---- operand prefetch ----------------------------------------------------------
 // A wave's k-steps are kt0, kt0 + ks, kt0 + 2ks, ... (KW of them; kt0 = the wave's
-// K group and ks = the number of K groups, so uneven K spreads evenly); k-steps past KT
-// load zeros and add nothing.
+// K group and ks = the number of K groups, so uneven K spreads evenly).
 //
-// Weight (B operand) registers of one wave: its k-steps of tiles [nt0, nt0+NT); tiles
-// past `ntv` stay zero.  Tile (nt, kt) of a tiled W (mla_model.hpp) is 512 contiguous
-// fp16 words; lane l reads 16 bytes at 8l.
+// Every load of a step kernel's operands and side inputs is unconditional: k-steps past
+// KT read the zero block as their weights (and add nothing), other out-of-range indices are
+// clamped, and what a clamped load read is dropped where it would be used.  A load behind a
+// condition becomes a branch, at whose join the compiler waits for loads in flight (the
+// conditional form of qkv_kernel waited for nearly all of its weights, and only then issued the
+// last two loads): every such wait is one more memory round trip of the kernel.  The wave
+// index is made scalar (wave_index), so the weight addresses and the choices are scalar too.
+__device__ __forceinline__ int wave_index() {
+    return __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+}
+
+// operands_issued() keeps the compiler from moving loads below it, behind the MFMAs (it does,
+// to save registers, and the loads it moved then start a round trip of their own).
+__device__ __forceinline__ void operands_issued() { __builtin_amdgcn_sched_barrier(0); }
+
+// Weight (B operand) registers of one wave: its k-steps of tiles [nt0, nt0+NT), of which
+// ntv >= 1 exist (the others repeat the last one).  Tile (nt, kt) of a tiled W
+// (mla_model.hpp) is 512 contiguous fp16 words; lane l reads 16 bytes at 8l.
+__device__ __forceinline__ V8 load_w(const uint16_t* w, const uint16_t* zeros, int nt, int kt,
+                                     int KT, int lane) {
+    const uint16_t* p = kt < KT ? w + ((long long)nt * KT + kt) * 512 : zeros;
+    return *reinterpret_cast<const V8*>(p + lane * 8);
+}
 template <int NT, int KW>
 struct BPre {
     V8 b[KW][NT];
-    __device__ __forceinline__ void load(const uint16_t* w, int nt0, int ntv, int KT, int kt0,
-                                         int ks, int lane) {
+    __device__ __forceinline__ void load(const uint16_t* w, const uint16_t* zeros, int nt0,
+                                         int ntv, int KT, int kt0, int ks, int lane) {
 #pragma unroll
         for (int kk = 0; kk < KW; ++kk)
 #pragma unroll
-            for (int j = 0; j < NT; ++j) {
-                const int kt = kt0 + kk * ks;
-                b[kk][j] = V8{};
-                if (kt < KT && j < ntv)
-                    b[kk][j] = *reinterpret_cast<const V8*>(
-                        w + ((long long)(nt0 + j) * KT + kt) * 512 + lane * 8);
-            }
+            for (int j = 0; j < NT; ++j)
+                b[kk][j] = load_w(w, zeros, nt0 + min(j, ntv - 1), kt0 + kk * ks, KT, lane);
     }
 };
 
 // Activation (A operand) registers: lane (g, n) needs rows 16mt + n (mt < MT) and
-// columns 32kt + 8g .. +7 of each of its k-steps.
+// columns 32kt + 8g .. +7 of each of its k-steps.  Rows past `rows` (>= 1) repeat the last one:
+// their products are dropped, and the lanes that share its address add no traffic.
 template <int KW, int MT>
 struct APre16 {  // fp16 rows, zero-padded to KT*32 columns
     V8 x[KW][MT];
-    __device__ __forceinline__ void load(const uint16_t* X, int ld, int KT, int kt0, int ks,
+    __device__ __forceinline__ void load(const uint16_t* X, int ld, int rows, int KT, int kt0,
+                                         int ks, int lane) {
+        const int g = lane >> 4, n = lane & 15;
+#pragma unroll
+        for (int kk = 0; kk < KW; ++kk)
+#pragma unroll
+            for (int mt = 0; mt < MT; ++mt)
+                x[kk][mt] = *reinterpret_cast<const V8*>(X + (long long)min(16 * mt + n, rows - 1) * ld +
+                                                         32 * min(kt0 + kk * ks, KT - 1) + 8 * g);
+    }
+};
+template <int KW, int MT>
+struct AHalf32 {  // fp32 rows (K % 8 == 0; the weights of columns past K are 0), rounded to fp16
+    floatx4 x[KW][MT][2];
+    __device__ __forceinline__ void load(const float* X, int ld, int rows, int K, int kt0, int ks,
                                          int lane) {
         const int g = lane >> 4, n = lane & 15;
 #pragma unroll
         for (int kk = 0; kk < KW; ++kk)
 #pragma unroll
             for (int mt = 0; mt < MT; ++mt) {
-                const int kt = kt0 + kk * ks;
-                x[kk][mt] = V8{};
-                if (kt < KT)
-                    x[kk][mt] = *reinterpret_cast<const V8*>(X + (long long)(16 * mt + n) * ld +
-                                                             32 * kt + 8 * g);
+                const floatx4* p = reinterpret_cast<const floatx4*>(
+                    X + (long long)min(16 * mt + n, rows - 1) * ld +
+                    min(32 * (kt0 + kk * ks) + 8 * g, K - 8));
+                x[kk][mt][0] = p[0];
+                x[kk][mt][1] = p[1];
             }
-    }
-};
-template <int KW, int MT>
-struct AHalf32 {  // fp32 rows (K % 8 == 0; columns past K read as zero), rounded to fp16
-    V8 x[KW][MT];
-    __device__ __forceinline__ void load(const float* X, int ld, int K, int KT, int kt0, int ks,
-                                         int lane) {
-        const int g = lane >> 4, n = lane & 15;
-#pragma unroll
-        for (int kk = 0; kk < KW; ++kk) {
-            const int kt = kt0 + kk * ks;
-            const int k = 32 * kt + 8 * g;
-            const bool ok = kt < KT && k < K;
-#pragma unroll
-            for (int mt = 0; mt < MT; ++mt) {
-                x[kk][mt] = V8{};
-                if (ok) {
-                    const floatx4* p =
-                        reinterpret_cast<const floatx4*>(X + (long long)(16 * mt + n) * ld + k);
-                    x[kk][mt] = to_half8(p[0], p[1]);
-                }
-            }
-        }
     }
 };
 
@@ -258,20 +221,17 @@ struct RmsPrefetch {
     float v[kPer];
     __device__ __forceinline__ void issue(const float* ss, int n_tiles, int row0, int rows) {
         const int t = threadIdx.x;
-        const bool mine = t < TPR * rows;
-        const float* p = ss + (long long)(row0 + (mine ? t / TPR : 0)) * n_tiles;
+        const float* p = ss + (long long)(row0 + min(t / TPR, rows - 1)) * n_tiles;
 #pragma unroll
-        for (int i = 0; i < kPer; ++i) {
-            const int tile = t % TPR + TPR * i;
-            v[i] = mine && tile < n_tiles ? p[tile] : 0.0f;
-        }
+        for (int i = 0; i < kPer; ++i)
+            v[i] = p[min(t % TPR + TPR * i, n_tiles - 1)];
     }
-    __device__ __forceinline__ void finish(int K, float eps, float* inv_s, int rows) {
+    __device__ __forceinline__ void finish(int n_tiles, int K, float eps, float* inv_s, int rows) {
         const int t = threadIdx.x;
         float sum = 0.0f;
 #pragma unroll
         for (int i = 0; i < kPer; ++i)
-            sum += v[i];
+            sum += t % TPR + TPR * i < n_tiles ? v[i] : 0.0f;
         sum = group_sum<TPR>(sum);
         if (t < TPR * rows && t % TPR == 0)
             inv_s[t / TPR] = 1.0f / sqrtf(sum / (float)K + eps);
@@ -285,7 +245,7 @@ struct RmsPrefetch {
 template <int MT, int NTW, int KG>
 __device__ __forceinline__ bool splitk_reduce(floatx4 (&acc)[MT][NTW], floatx4* part, int& mt,
                                               floatx4 (&v)[NTW * (kWaves / KG)]) {
-    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    const int wave = wave_index(), lane = threadIdx.x & 63;
 #pragma unroll
     for (int m = 0; m < MT; ++m)
 #pragma unroll
@@ -361,24 +321,215 @@ __global__ __launch_bounds__(256) void embed_kernel(StepArgs s, const float* nor
     }
 }
 
-// -------------------------------------------------------------------- qkv ----
-// Everything between the residual stream x and the attention, for 16 rows per
-// workgroup (inference.cpp:85-103): workgroup h < H computes head h's queries,
-// workgroup H the cache append.  Both start with the same split-K GEMM
-//     y = RMSNorm(x, attn_norm) . [w_dq | w_dkv]        (their column ranges)
-// (8 waves, wave w taking k-steps w, w+8, ..; the partial tiles meet in LDS), so no
-// other workgroup's output is waited for: each head workgroup recomputes the whole cq
-// row it needs for q_norm (w_dq is L2-resident, read once per workgroup).  Then
-//   head h:  q_norm(cq) -> . w_uq[:, head h] -> RoPE of the rope columns (q_rope in the
-//            cache dtype) -> q_latent = q_nope . W_uk_h^T (the MPS graph keeps q_latent
-//            in the storage dtype, mps_backend.mm:561)
-//   kv:      kv_norm of the latent columns, RoPE of the key, rounding, paged append
-// The norms are RMSNorm(v)_c = v_c * inv * w_c with one inv per row, and everything after
-// them is linear, so the split-K reduction writes v o w straight away, with the rows'
-// sums of squares per 16-column tile, and inv is applied later: to the w_uq products
-// (head) or at the append (kv).  No pass over the rows waits for a row norm.
-constexpr int kQkvWaves = 8;
+// --------------------------------------------------------------- g1 and g2 ----
+// Between the residual stream x and the attention (inference.cpp:85-103).  g1: per 16 rows and
+// 16-column tile, y = RMSNorm(x, attn_norm) . [w_dq | w_dkv], 8 waves splitting K.  The norms
+// that follow are RMSNorm(v)_c = v_c * inv * w_c with one inv per row, and what follows them is
+// linear, so g1 leaves v o w (cq: fp16, g2's A operand; latent: fp32) with the rows' sums of
+// squares per tile, and g2 applies inv to its products.  g2: wave w of workgroup b owns column
+// tile 4b + w of the H x hq_pad columns of w_q for 16 rows: no split of K (q_rank <= 256), no
+// exchange between waves.
+// Batches of up to 16 rows run both in one launch (qkv_kernel, below), with the same results
+// bit for bit (the same K groups, summed in the same order).
+template <int KW>
+__global__ __launch_bounds__(64 * kWaves) void g1_kernel(StepArgs s, LayerWeights L) {
+    __shared__ __attribute__((aligned(16))) floatx4 part[kWaves * 64];
+    __shared__ __attribute__((aligned(16))) uint16_t scratch[512];
+    __shared__ float inv_s[16];
+    const ModelDims& m = s.dims;
+    const int wave = wave_index(), lane = threadIdx.x & 63, g = lane >> 4, n = lane & 15;
+    const int q_tiles = m.q_pad / 16, tiles = q_tiles + m.kvw_pad / 16, nt = blockIdx.x;
+    const int row0 = blockIdx.y * 16, KT = m.d_pad / 32;
+    if (nt >= tiles)
+        return;  // columns are padded to a multiple of 8 (see l2_prefetch)
+    RmsPrefetch<16> rms;
+    rms.issue(s.ss_x, m.d_pad / 16, row0, 16);
+    BPre<1, KW> bw;
+    bw.load(L.w_dq_dkv, s.zeros, nt, 1, KT, wave, kWaves, lane);
+    APre16<KW, 1> a;
+    a.load(s.xw + (long long)row0 * m.d_pad, m.d_pad, s.B - row0, KT, wave, kWaves, lane);
+    // column c of cq (c < q_rank counts in its norm) or of [latent | key] (c < kv_rank)
+    const bool kv = nt >= q_tiles;
+    const int c = 16 * (kv ? nt - q_tiles : nt) + n, norm_cols = kv ? m.kv_rank : m.q_rank;
+    const float wn = (kv ? L.kv_norm : L.q_norm)[min(c, norm_cols - 1)];
+    operands_issued();
+    floatx4 acc[1][1];
+    zero(acc);
+    mma_steps(acc, bw, [&](int kk, int mt) { return a.x[kk][mt]; });
+    rms.finish(m.d_pad / 16, m.d_model, m.eps, inv_s, 16);
+    int mt;
+    floatx4 v[1];
+    if (!splitk_reduce<1, 1, kWaves>(acc, part, mt, v)) {
+        // g2 (next on the stream) runs workgroup b with residue b % 8: its four tiles are
+        // 4 * KTQ contiguous blocks of w_q
+        const int x = block_xcd(), KTQ = m.q_pad / 32, all = m.H * (m.hq_pad / 16) * KTQ;
+        const int wgs = (m.H * (m.hq_pad / 16) + 3) / 4, per = 4 * KTQ;
+        l2_prefetch(x < wgs ? (wgs - x + kXcds - 1) / kXcds * per : 0, [&](int k) {
+            return L.w_q + (long long)min((x + kXcds * (k / per)) * per + k % per, all - 1) * 512;
+        }, scratch, 1);
+        return;
+    }
+    floatx4 y;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const int row = row0 + 4 * g + i;
+        y[i] = v[0][i] * inv_s[4 * g + i];
+        if (row < s.B) {
+            if (kv)
+                s.ckv[(long long)row * m.kvw_pad + c] = y[i] * (c < m.kv_rank ? wn : 1.0f);
+            else
+                s.cqw[(long long)row * m.q_pad + c] = F16::from_float(c < m.q_rank ? y[i] * wn : 0.0f);
+        }
+    }
+    if (kv)
+        write_ss(y, c < m.kv_rank, s.ss_kv, m.kvw_pad / 16, nt - q_tiles, row0, s.B);
+    else
+        write_ss(y, c < m.q_rank, s.ss_cq, q_tiles, nt, row0, s.B);
+}
+
+// RoPE of the adjacent columns (a0, a1) (ops.cpp:88-108).  One form for every kernel: the
+// kernels that a row can go through, depending on the batch, give the same bits.
+__device__ __forceinline__ float rope_even(float a0, float a1, float2 cs) {
+    return fmaf(a0, cs.x, -(a1 * cs.y));
+}
+__device__ __forceinline__ float rope_odd(float a0, float a1, float2 cs) {
+    return fmaf(a0, cs.y, a1 * cs.x);
+}
+
+// The appended rows row0 .. row0 + 15: kv_norm of the latent, RoPE of the key, rounding, and the
+// paged store.  Everything comes from LDS: y (rows of ld: v o kv_norm, then the key), the rows'
+// kv_norm factors, slots (-1: none) and rotations [16][rope / 2].
+__device__ __forceinline__ void append_rows(const StepArgs& s, uint16_t* pool, const float* y,
+                                            int ld, const float* inv_s, const int32_t* slot_s,
+                                            const float2* cs_s) {
+    const ModelDims& m = s.dims;
+    const bool tiled = page_tiled(m.page_size, m.kv_rank, m.rope);
+    const int width = m.kv_rank + m.rope, per = blockDim.x / 16;  // threads of a row
+    const int r = threadIdx.x / per;
+    const int slot = slot_s[r];
+    const int page = slot / m.page_size, off = slot % m.page_size;
+    if (slot < 0 || page >= s.num_pool_pages)
+        return;
+    const float* yr = y + r * ld;
+    const float inv = inv_s[r];
+    uint16_t* base = pool + (long long)page * m.page_size * width;
+    for (int c = threadIdx.x % per; c < width; c += per) {
+        if (c < m.kv_rank) {
+            base[latent_word(tiled, off, c, m.page_size, m.kv_rank)] = F16::from_float(yr[c] * inv);
+        } else {
+            const int j = c - m.kv_rank;
+            const float2 cs = cs_s[r * (m.rope / 2) + j / 2];
+            const float a = yr[m.kv_rank + (j & ~1)], b = yr[m.kv_rank + (j | 1)];
+            base[rope_word(tiled, off, j, m.page_size, m.kv_rank, m.rope)] =
+                F16::from_float(j & 1 ? rope_odd(a, b, cs) : rope_even(a, b, cs));
+        }
+    }
+}
+constexpr int kMaxHalfRope = 32;  // rope <= 64 (mla_model_create checks)
+
+// One 16x16 tile of g2's products (rows row0 + 4g + i, column 16t + n of head h's columns),
+// times the rows' q_norm factors: q_latent, or q_rope after RoPE.
+__device__ __forceinline__ void store_q_tile(const StepArgs& s, floatx4 q, int h, int t, int row0,
+                                             const float2 (&cs)[4]) {
+    const ModelDims& m = s.dims;
+    const int lane = threadIdx.x & 63, g = lane >> 4, n = lane & 15, kv_tiles = m.kv_pad / 16;
+    const bool rope = t >= kv_tiles;
+    const int c = 16 * (rope ? t - kv_tiles : t) + n;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const int row = row0 + 4 * g + i;
+        if (!rope) {
+            if (row < s.B && c < m.kv_rank)
+                s.q_latent[((long long)row * m.H + h) * m.kv_rank + c] = F16::from_float(q[i]);
+            continue;
+        }
+        const float o = dpp_mov<0xB1>(q[i]);  // quad_perm [1,0,3,2]: the pair's other column
+        const float y = n & 1 ? rope_odd(o, q[i], cs[i]) : rope_even(q[i], o, cs[i]);
+        if (row < s.B && c < m.rope)
+            s.q_rope[((long long)row * m.H + h) * m.rope + c] = F16::from_float(y);
+    }
+}
+
+constexpr int kG2Waves = 4;
+
+template <int KW>
+__global__ __launch_bounds__(64 * kG2Waves) void g2_kernel(StepArgs s, LayerWeights L,
+                                                           uint16_t* pool) {
+    __shared__ __attribute__((aligned(16))) float inv_s[16];
+    __shared__ float y_s[16 * (192 + 4)];  // the append workgroup's (kvw_pad <= 192)
+    __shared__ int32_t slot_s[16];
+    __shared__ float2 cs_s[16 * kMaxHalfRope];
+    const ModelDims& m = s.dims;
+    const int wave = wave_index(), lane = threadIdx.x & 63, g = lane >> 4, n = lane & 15;
+    const int row0 = blockIdx.y * 16, KTQ = m.q_pad / 32, hq_tiles = m.hq_pad / 16;
+    const int all = m.H * hq_tiles, wgs = (all + kG2Waves - 1) / kG2Waves;
+    if ((int)blockIdx.x > wgs)
+        return;  // columns are padded to a multiple of 8 (see l2_prefetch)
+    RmsPrefetch<16> rms;
+    if ((int)blockIdx.x == wgs) {  // the append workgroup
+        // every load in flight at once (a thread: 12 columns of row tid / 16, one slot, two
+        // rotations), then from LDS: element by element from memory this workgroup took 9 us
+        rms.issue(s.ss_kv, m.kvw_pad / 16, row0, 16);
+        const int tid = threadIdx.x, row = row0 + tid / 16, ld = m.kvw_pad + 4, rh = m.rope / 2;
+        float v[12];
+#pragma unroll
+        for (int k = 0; k < 12; ++k)
+            v[k] = s.ckv[(long long)row * m.kvw_pad + min(16 * k + tid % 16, m.kvw_pad - 1)];
+        const int32_t slot = s.slot_mapping[min(row, s.B - 1)];
+        float2 r2[2];
+#pragma unroll
+        for (int k = 0; k < 2; ++k)
+            r2[k] = s.rope_rows[(long long)row0 * rh + min(tid + 256 * k, 16 * rh - 1)];
+        operands_issued();
+        rms.finish(m.kvw_pad / 16, m.kv_rank, m.eps, inv_s, 16);
+#pragma unroll
+        for (int k = 0; k < 12; ++k)
+            if (16 * k < m.kvw_pad)
+                y_s[tid / 16 * ld + 16 * k + tid % 16] = v[k];
+        if (tid % 16 == 0)
+            slot_s[tid / 16] = row < s.B ? slot : -1;
+#pragma unroll
+        for (int k = 0; k < 2; ++k)
+            if (tid + 256 * k < 16 * rh)
+                cs_s[tid + 256 * k] = r2[k];
+        __syncthreads();
+        append_rows(s, pool, y_s, ld, inv_s, slot_s, cs_s);
+        return;
+    }
+    rms.issue(s.ss_cq, m.q_pad / 16, row0, 16);
+    const int T = min(kG2Waves * (int)blockIdx.x + wave, all - 1), h = T / hq_tiles, t = T % hq_tiles;
+    BPre<1, KW> bw;
+    bw.load(L.w_q, s.zeros, T, 1, KTQ, 0, 1, lane);
+    APre16<KW, 1> a;
+    a.load(s.cqw + (long long)row0 * m.q_pad, m.q_pad, s.B - row0, KTQ, 0, 1, lane);
+    float2 cs[4];
+    const int rhalf = m.rope / 2, j2 = min((16 * max(t - m.kv_pad / 16, 0) + n) / 2, rhalf - 1);
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+        cs[i] = s.rope_rows[(long long)(row0 + 4 * g + i) * rhalf + j2];
+    operands_issued();
+    floatx4 acc[1][1];
+    zero(acc);
+    mma_steps(acc, bw, [&](int kk, int mt) { return a.x[kk][mt]; });
+    rms.finish(m.q_pad / 16, m.q_rank, m.eps, inv_s, 16);
+    __syncthreads();
+    if (kG2Waves * (int)blockIdx.x + wave >= all)
+        return;
+    store_q_tile(s, acc[0][0] * *reinterpret_cast<const floatx4*>(inv_s + 4 * g), h, t, row0, cs);
+}
+
+// qkv_kernel -- g1 and g2 in one launch for up to 16 rows: workgroup h < H computes head h's
+// queries, workgroup H the cache append.  Both start with g1's split-K GEMM over their column
+// range, so no other workgroup's output is waited for: each head workgroup recomputes the whole
+// cq row it needs for q_norm.  Each of the 9 workgroups (at 8 heads) then pulls 250 KB of
+// weights through one CU's load path, so from 17 rows on two launches, whose workgroups pull
+// 32 KB each, are faster.  A whole step, one launch against two: 278 / 279 us (1 session), 307 /
+// 310 (8), 317 / 325 (16), 314 / 310 (32), 321 / 315 (48), 328 / 322 (64).  Copying the first
+// page of each attention work item into L2 from idle workgroups of these launches, which paid
+// when one slower kernel did all of this (8.9 us at 64 rows; g1 and g2: 4.2 each), now costs
+// more than it saves (399 us without, 416 with every fourth item, 473 with all).
 constexpr int kQkvRows = 16;
+constexpr int kQkvMaxRows = 16;
 constexpr int kQkvMaxTiles = 16;  // q_pad <= 256, kvw_pad <= 192: at most 16 column tiles
 constexpr int kQkvPad = 8;        // fp16 pad of the LDS A-operand rows
 // fp32 pad of the LDS y rows: with a pitch of 36 mod 64 words, the split-K reduction's
@@ -387,247 +538,171 @@ constexpr int kQkvYPad = 36;
 
 // LDS layout of qkv_kernel (bytes), from the model dims.
 struct QkvLds {
-    int part, y, ya, qf, qn, total;
+    int part, y, ya, total;
 };
 __host__ __device__ inline QkvLds qkv_lds(const ModelDims& m) {
     const int nt = max(m.q_pad, m.kvw_pad) / 16;
     const int ncol = max(m.q_pad, m.kvw_pad);
-    // The split-K partials are dead once they are summed, so qf / qn reuse them; a head
-    // workgroup writes ya where the append workgroup keeps y (neither needs the other).
+    // A head workgroup writes ya where the append workgroup keeps y (neither needs the other).
     QkvLds l;
-    l.part = 0;                                             // [8 waves][nt][64] floatx4
-    l.qf = 0;                                               // [16][qk_pad + 4] fp32
-    l.qn = l.qf + kQkvRows * (m.qk_pad + 4) * 4;            // [16][nope_pad + pad] fp16
-    const int end = l.qn + kQkvRows * (m.nope_pad + kQkvPad) * 2;
-    l.y = max(kQkvWaves * nt * 64 * 16, end);               // [16][ncol + kQkvYPad] fp32
-    l.ya = l.y;                                             // [16][q_pad + pad] fp16
+    l.part = 0;                      // [8 waves][nt][64] floatx4
+    l.y = kWaves * nt * 64 * 16;     // [16][ncol + kQkvYPad] fp32
+    l.ya = l.y;                      // [16][q_pad + pad] fp16
     l.total = l.y + kQkvRows * (ncol + kQkvYPad) * 4;
     return l;
 }
 
-// KC: chunks of two k-steps per wave (KT <= 16 * KC); NT >= the workgroup's column tiles.
+// KC: chunks of two k-steps per wave (KT <= 16 * KC); NT >= the workgroup's column tiles
+// (q_pad <= 16 NT).
 template <int KC, int NT>
-__global__ __launch_bounds__(64 * kQkvWaves) void qkv_kernel(StepArgs s, LayerWeights L,
-                                                             uint16_t* pool, PagePrefetch pf) {
+__global__ __launch_bounds__(64 * kWaves) void qkv_kernel(StepArgs s, LayerWeights L,
+                                                          uint16_t* pool) {
     extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
+    constexpr int KQ = NT / 2;  // k-steps of w_q
     const ModelDims& m = s.dims;
     const QkvLds lay = qkv_lds(m);
     floatx4* part = reinterpret_cast<floatx4*>(smem + lay.part);
     float* y = reinterpret_cast<float*>(smem + lay.y);
     _Float16* ya = reinterpret_cast<_Float16*>(smem + lay.ya);
-    float* qf = reinterpret_cast<float*>(smem + lay.qf);
-    _Float16* qn = reinterpret_cast<_Float16*>(smem + lay.qn);
     __shared__ float inv_x[kQkvRows];
+    __shared__ __attribute__((aligned(16))) float inv_n[kQkvRows];  // kv_norm factor per row
+    __shared__ float ss_part[kQkvRows][kQkvMaxTiles];  // row sums of squares per column tile
+    __shared__ int32_t slot_s[kQkvRows];
+    __shared__ float2 cs_s[kQkvRows * kMaxHalfRope];
 
     const int h = blockIdx.x, row0 = blockIdx.y * kQkvRows;
-    if (h > m.H) {  // the heads' columns are padded to a multiple of 8 (head h: residue h % 8)
-        if (h >= (m.H + kXcds) / kXcds * kXcds)  // the read-ahead block past them
-            page_prefetch(pf, pool, s.num_pool_pages, reinterpret_cast<uint16_t*>(smem),
-                          block_xcd(), blockIdx.y * kQkvWaves + (threadIdx.x >> 6),
-                          gridDim.y * kQkvWaves);
-        return;
-    }
+    const int tid = threadIdx.x, wave = wave_index(), lane = tid & 63, g = lane >> 4, n = lane & 15;
+    if (h > m.H)
+        return;  // the heads' columns are padded to a multiple of 8 (head h: residue h % 8)
     const bool kv = h == m.H;
-    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, g = lane >> 4, n = lane & 15;
     const int KT = m.d_pad / 32, q_tiles = m.q_pad / 16;
     const int nt0 = kv ? q_tiles : 0, ntv = kv ? m.kvw_pad / 16 : q_tiles;
-    const int ncol = 16 * ntv, ldy = max(m.q_pad, m.kvw_pad) + kQkvYPad;
-    __shared__ int32_t slot_s[kQkvRows];
+    const int ldy = max(m.q_pad, m.kvw_pad) + kQkvYPad;
     RmsPrefetch<16> rms;
     rms.issue(s.ss_x, m.d_pad / 16, row0, kQkvRows);
-    // Side inputs of the later phases travel with the GEMM operands: the norm weight of
-    // the two columns this thread reduces (16 * (wave + 8k) + n: 1 for the key's RoPE
-    // columns, 0 past q_rank), the RoPE rotation of its first RoPE element, and (kv
-    // workgroup) the rows' cache slots.
+    // The norm weights of the two columns this thread reduces (16 * (wave + 8k) + n), the rows'
+    // slots and rotations travel with the GEMM operands.
     const int ncols = kv ? m.kv_rank : m.q_rank;
     const float* nwp = kv ? L.kv_norm : L.q_norm;
     float nw[2];
 #pragma unroll
-    for (int k = 0; k < 2; ++k) {
-        const int c = 16 * (wave + kQkvWaves * k) + n;
-        nw[k] = c < ncols ? nwp[c] : kv ? 1.0f : 0.0f;
-    }
+    for (int k = 0; k < 2; ++k)
+        nw[k] = nwp[min(16 * (wave + kWaves * k) + n, ncols - 1)];
     const int rhalf = m.rope / 2;
-    float2 rcs = {0.0f, 0.0f};
-    if (tid < kQkvRows * rhalf && row0 + tid / rhalf < s.B)
-        rcs = s.rope_rows[(long long)(row0 + tid / rhalf) * rhalf + tid % rhalf];
-    int32_t slot_pf = -1;
-    if (kv && tid < kQkvRows && row0 + tid < s.B)
-        slot_pf = s.slot_mapping[row0 + tid];
+    const int32_t slot_pf = s.slot_mapping[min(row0 + tid, s.B - 1)];
+    const float2 rcs = s.rope_rows[(long long)row0 * rhalf + min(tid, kQkvRows * rhalf - 1)];
 
     // ---- GEMM 1: every operand of this wave in flight at once, chunk by chunk ----
     floatx4 acc[NT];
 #pragma unroll
     for (int j = 0; j < NT; ++j)
         acc[j] = floatx4{0, 0, 0, 0};
-    const uint16_t* xw = s.xw + (long long)(row0 + n) * m.d_pad;
-    // head workgroups also prefetch their w_uq / W_uk tiles (used after the reduction)
-    const int qk_tiles = m.qk_pad / 16, KTQ = m.q_pad / 32;
-    const int kv_tiles = m.kv_pad / 16, KTU = m.nope_pad / 32;
-    V8 bq[8], bu[4];
+    const uint16_t* xw = s.xw + (long long)min(row0 + n, s.B - 1) * m.d_pad;
+    // Head workgroups also prefetch their w_q tiles (used after the reduction; wave w owns
+    // tiles w and w + 8 of the head's kv_tiles latent and then rope tiles) and the RoPE
+    // rotations of the rows and columns they hold of a rope tile.
+    const int KTQ = m.q_pad / 32, kv_tiles = m.kv_pad / 16, hq_tiles = m.hq_pad / 16;
+    V8 bq[2][KQ];
+    float2 qcs[2][4];
 #pragma unroll
     for (int c = 0; c < KC; ++c) {
         V8 a[2], b[2][NT];
 #pragma unroll
         for (int kk = 0; kk < 2; ++kk) {
-            const int kt = wave + kQkvWaves * (2 * c + kk);
-            a[kk] = kt < KT ? *reinterpret_cast<const V8*>(xw + 32 * kt + 8 * g) : V8{};
+            const int kt = wave + kWaves * (2 * c + kk);
+            a[kk] = *reinterpret_cast<const V8*>(xw + 32 * min(kt, KT - 1) + 8 * g);
 #pragma unroll
             for (int j = 0; j < NT; ++j)
-                b[kk][j] = kt < KT && j < ntv
-                               ? *reinterpret_cast<const V8*>(
-                                     L.w_dq_dkv + ((long long)(nt0 + j) * KT + kt) * 512 + lane * 8)
-                               : V8{};
+                b[kk][j] = load_w(L.w_dq_dkv, s.zeros, nt0 + min(j, ntv - 1), kt, KT, lane);
         }
         if (c == 0 && !kv) {
 #pragma unroll
-            for (int k = 0; k < 8; ++k)
-                bq[k] = wave < qk_tiles && k < KTQ
-                            ? *reinterpret_cast<const V8*>(
-                                  L.w_uq + ((long long)(h * qk_tiles + wave) * KTQ + k) * 512 +
-                                  lane * 8)
-                            : V8{};
+            for (int t = 0; t < 2; ++t) {
+                const int tile = wave + kWaves * t;
+                if (tile < hq_tiles) {  // scalar, and nothing else writes the registers
+                    const int j2 = (16 * max(tile - kv_tiles, 0) + n) / 2;
 #pragma unroll
-            for (int k = 0; k < 4; ++k)
-                bu[k] = wave < kv_tiles && k < KTU
-                            ? *reinterpret_cast<const V8*>(
-                                  L.w_uk + (long long)h * kv_tiles * KTU * 512 +
-                                  ((long long)wave * KTU + k) * 512 + lane * 8)
-                            : V8{};
+                    for (int k = 0; k < KQ; ++k)
+                        bq[t][k] = load_w(L.w_q, s.zeros, h * hq_tiles + tile, k, KTQ, lane);
+#pragma unroll
+                    for (int i = 0; i < 4; ++i)
+                        qcs[t][i] =
+                            s.rope_rows[(long long)(row0 + 4 * g + i) * rhalf + min(j2, rhalf - 1)];
+                }
+            }
         }
+        operands_issued();
 #pragma unroll
         for (int kk = 0; kk < 2; ++kk)
 #pragma unroll
             for (int j = 0; j < NT; ++j)
                 acc[j] = mma(a[kk], b[kk][j], acc[j]);
     }
-    rms.finish(m.d_model, m.eps, inv_x, kQkvRows);
-    if (kv && tid < kQkvRows)
-        slot_s[tid] = slot_pf;
+    rms.finish(m.d_pad / 16, m.d_model, m.eps, inv_x, kQkvRows);
 #pragma unroll
     for (int j = 0; j < NT; ++j)
         if (j < ntv)
             part[(wave * ntv + j) * 64 + lane] = acc[j];
-    __shared__ float ss_part[kQkvRows][kQkvMaxTiles];  // row sums of squares per column tile
-    __shared__ float inv_n[kQkvRows];                  // q_norm / kv_norm factor per row
+    if (tid < kQkvRows)
+        slot_s[tid] = row0 + tid < s.B ? slot_pf : -1;
+    if (tid < kQkvRows * rhalf)
+        cs_s[tid] = rcs;
+    if (tid < kQkvRows * kQkvMaxTiles && tid % kQkvMaxTiles >= ntv)
+        ss_part[tid / kQkvMaxTiles][tid % kQkvMaxTiles] = 0.0f;
     __syncthreads();
     // v[r][c] = inv_x[r] * sum over the waves (rows 4g+i, column 16j+n of lane group e);
     // head: ya = v o q_norm weight (fp16 A operand); kv: y = v o kv_norm weight (1 for the
     // key's RoPE columns).  ss_part[r][j] = sum of v^2 over tile j's norm columns.
-    for (int e = tid, k = 0; e < ntv * 64; e += 64 * kQkvWaves, ++k) {
-        const int j = e >> 6, l = e & 63, col = 16 * j + (l & 15);
+#pragma unroll
+    for (int k = 0; k < 2; ++k) {
+        const int j = wave + kWaves * k, col = 16 * j + n;
+        if (j >= ntv)
+            break;
         floatx4 v = {0, 0, 0, 0};
 #pragma unroll
-        for (int w = 0; w < kQkvWaves; ++w)
-            v += part[(w * ntv + j) * 64 + l];
-        const float wc = k == 0 ? nw[0] : nw[1];
+        for (int w = 0; w < kWaves; ++w)
+            v += part[(w * ntv + j) * 64 + lane];
+        const float wc = col < ncols ? nw[k] : kv ? 1.0f : 0.0f;
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-            const int r = 4 * (l >> 4) + i;
+            const int r = 4 * g + i;
             const float yv = v[i] * inv_x[r];
             if (kv)
                 y[r * ldy + col] = yv * wc;
             else
                 ya[r * (m.q_pad + kQkvPad) + col] = (_Float16)(yv * wc);
             const float sq = sum16(col < ncols ? yv * yv : 0.0f);
-            if ((l & 15) == 0)
+            if (n == 0)
                 ss_part[r][j] = sq;
         }
     }
     __syncthreads();
-    // inv of each row (ops.cpp:37-44: 1/sqrt(mean(v^2) + eps)) by the last wave's first
-    // lanes, visible after the next barrier
-    if (wave == kQkvWaves - 1 && lane < kQkvRows) {
-        float ss = 0.0f;
-        for (int j = 0; j * 16 < ncols; ++j)
-            ss += ss_part[lane][j];
-        inv_n[lane] = 1.0f / sqrtf(ss / (float)ncols + m.eps);
-    }
+    // the norm factors of this lane group's rows 4g + i (ops.cpp:37-44: 1/sqrt(mean(v^2) + eps))
+    floatx4 inv;
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+        inv[i] = 1.0f / sqrtf(sum16(ss_part[4 * g + i][n]) / (float)ncols + m.eps);
 
-    if (kv) {  // ---- RoPE of the key (in place), then rounding and the paged append ----
-        {
-            for (int e = tid; e < kQkvRows * rhalf; e += 64 * kQkvWaves) {
-                const int rr = e / rhalf, jp = 2 * (e % rhalf);
-                const float2 cs =
-                    e == tid ? rcs : s.rope_rows[(long long)(row0 + rr) * rhalf + e % rhalf];
-                float* yk = y + rr * ldy + m.kv_rank + jp;
-                const float a0 = yk[0], a1 = yk[1];
-                yk[0] = a0 * cs.x - a1 * cs.y;
-                yk[1] = a0 * cs.y + a1 * cs.x;
-            }
-        }
+    if (kv) {  // ---- kv_norm, RoPE of the key, rounding and the paged append ----
+        if (wave == 0 && n == 0)
+            *reinterpret_cast<floatx4*>(inv_n + 4 * g) = inv;
         __syncthreads();
-        const bool tiled = page_tiled(m.page_size, m.kv_rank, m.rope);
-        const int width = m.kv_rank + m.rope;
-        for (int e = tid; e < kQkvRows * width; e += 64 * kQkvWaves) {
-            const int r = e / width, c = e % width, row = row0 + r;
-            if (row >= s.B)
-                continue;
-            const int slot = slot_s[r];
-            const int page = slot / m.page_size, off = slot % m.page_size;
-            if (slot < 0 || page >= s.num_pool_pages)
-                continue;
-            uint16_t* base = pool + (long long)page * m.page_size * width;
-            const uint16_t v = F16::from_float(c < m.kv_rank ? y[r * ldy + c] * inv_n[r]
-                                                             : y[r * ldy + c]);
-            if (c < m.kv_rank)
-                base[latent_word(tiled, off, c, m.page_size, m.kv_rank)] = v;
-            else
-                base[rope_word(tiled, off, c - m.kv_rank, m.page_size, m.kv_rank, m.rope)] = v;
-        }
+        append_rows(s, pool, y, ldy, inv_n, slot_s, cs_s);
         return;
     }
-    (void)ncol;
-
-    // ---- q_h = (cq o q_norm weight) . w_uq[:, head h], times the row's inv below: wave
-    // w < qk_tiles owns column tile w ----
-    if (wave < qk_tiles) {
+    // ---- (cq o q_norm weight) . w_q[head h], times the row's inv ----
+#pragma unroll
+    for (int t = 0; t < 2; ++t) {
+        const int tile = wave + kWaves * t;
+        if (tile >= hq_tiles)
+            break;
         floatx4 q = {0, 0, 0, 0};
 #pragma unroll
-        for (int k = 0; k < 8; ++k)
+        for (int k = 0; k < KQ; ++k)
             if (k < KTQ)
                 q = mma(*reinterpret_cast<const V8*>(ya + n * (m.q_pad + kQkvPad) + 32 * k + 8 * g),
-                        bq[k], q);
-#pragma unroll
-        for (int i = 0; i < 4; ++i)
-            qf[(4 * g + i) * (m.qk_pad + 4) + 16 * wave + n] = q[i];
-    }
-    __syncthreads();
-    {   // RoPE of the rope columns (pairs adjacent, ops.cpp:88-108) -> q_rope; q_nope -> fp16
-        const int half = rhalf, ldq = m.nope_pad + kQkvPad;
-        for (int e = tid; e < kQkvRows * half; e += 64 * kQkvWaves) {
-            const int r = e / half, j2 = e % half, jp = 2 * j2, row = row0 + r;
-            if (row >= s.B)
-                continue;
-            const float2 cs = e == tid ? rcs : s.rope_rows[(long long)row * half + j2];
-            const float a0 = qf[r * (m.qk_pad + 4) + m.nope + jp] * inv_n[r];
-            const float a1 = qf[r * (m.qk_pad + 4) + m.nope + jp + 1] * inv_n[r];
-            uint16_t* qr = s.q_rope + ((long long)row * m.H + h) * m.rope;
-            qr[jp] = F16::from_float(a0 * cs.x - a1 * cs.y);
-            qr[jp + 1] = F16::from_float(a0 * cs.y + a1 * cs.x);
-        }
-        for (int e = tid; e < kQkvRows * m.nope_pad; e += 64 * kQkvWaves) {
-            const int r = e / m.nope_pad, c = e % m.nope_pad;
-            qn[r * ldq + c] = (_Float16)(c < m.nope ? qf[r * (m.qk_pad + 4) + c] * inv_n[r] : 0.0f);
-        }
-    }
-    __syncthreads();
-    // ---- q_latent_h = q_nope . W_uk_h^T: wave w < kv_tiles owns latent tile w ----
-    if (wave < kv_tiles) {
-        const int ldq = m.nope_pad + kQkvPad;
-        floatx4 ql = {0, 0, 0, 0};
-#pragma unroll
-        for (int k = 0; k < 4; ++k)
-            if (k < KTU)
-                ql = mma(*reinterpret_cast<const V8*>(qn + n * ldq + 32 * k + 8 * g), bu[k], ql);
-        const int c = 16 * wave + n;
-        if (c < m.kv_rank)
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                const int row = row0 + 4 * g + i;
-                if (row < s.B)
-                    s.q_latent[((long long)row * m.H + h) * m.kv_rank + c] = F16::from_float(ql[i]);
-            }
+                        bq[t][k], q);
+        store_q_tile(s, q * inv, h, tile, row0, qcs[t]);
     }
 }
 
@@ -637,23 +712,24 @@ __global__ __launch_bounds__(64 * kQkvWaves) void qkv_kernel(StepArgs s, LayerWe
 // y's per-tile sums of squares.  The residual and norm columns are fetched with the
 // operands.
 template <int KW, typename ALoad, typename Pf>
-__device__ __forceinline__ void splitk_residual(ALoad&& aload, const uint16_t* w, int KT, int N,
+__device__ __forceinline__ void splitk_residual(ALoad&& aload, const uint16_t* w,
+                                                const uint16_t* zeros, int KT, int N,
                                                 const float* residual, const float* wnorm,
                                                 float* out, uint16_t* outw, float* ss,
                                                 int n_tiles, int ld, int row0, int B,
                                                 Pf&& prefetch) {
     __shared__ __attribute__((aligned(16))) floatx4 part[kWaves * 64];
-    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, g = lane >> 4, n = lane & 15;
+    const int wave = wave_index(), lane = threadIdx.x & 63, g = lane >> 4, n = lane & 15;
     const int nt = blockIdx.x, col = nt * 16 + n;
     BPre<1, KW> bw;
-    bw.load(w, nt, 1, KT, wave, kWaves, lane);
-    floatx4 res = {0, 0, 0, 0};
-    float wn = 0.0f;
-    if (wave == 0 && col < N) {
+    bw.load(w, zeros, nt, 1, KT, wave, kWaves, lane);
+    floatx4 res;
+    float wn;
+    if (wave == 0) {  // the wave that uses them
 #pragma unroll
         for (int i = 0; i < 4; ++i)
-            res[i] = residual[(long long)(row0 + 4 * g + i) * ld + col];
-        wn = wnorm[col];
+            res[i] = residual[(long long)(row0 + 4 * g + i) * ld + min(col, N - 1)];
+        wn = wnorm[min(col, N - 1)];
     }
     floatx4 acc[1][1];
     zero(acc);
@@ -686,10 +762,12 @@ __global__ __launch_bounds__(64 * kWaves) void g4_kernel(StepArgs s, LayerWeight
     splitk_residual<KW>(
         [&](floatx4(&acc)[1][1], const BPre<1, KW>& bw, int kt0, int lane) {
             AHalf32<KW, 1> a;
-            a.load(s.ctx + (long long)row0 * ctx_w, ctx_w, ctx_w, KT, kt0, kWaves, lane);
-            mma_steps(acc, bw, [&](int kk, int mt) { return a.x[kk][mt]; });
+            a.load(s.ctx + (long long)row0 * ctx_w, ctx_w, s.B - row0, ctx_w, kt0, kWaves, lane);
+            operands_issued();
+            mma_steps(acc, bw,
+                      [&](int kk, int mt) { return to_half8(a.x[kk][mt][0], a.x[kk][mt][1]); });
         },
-        L.w_out, KT, m.d_model, s.x, L.ffn_norm, s.res, s.resw, s.ss_res, m.d_pad / 16, m.d_pad,
+        L.w_out, s.zeros, KT, m.d_model, s.x, L.ffn_norm, s.res, s.resw, s.ss_res, m.d_pad / 16, m.d_pad,
         row0, s.B, [&]() {
             // g5 (next on the stream) runs column pair p with residue p % 8: its two tiles of
             // every k-step are 2 * KT5 contiguous blocks
@@ -703,46 +781,52 @@ __global__ __launch_bounds__(64 * kWaves) void g4_kernel(StepArgs s, LayerWeight
 }
 
 // next_norm: the norm weight of x's next consumer (attn_norm of the next layer, or
-// final_norm after the last layer).  next: the next layer's weights (qkv_kernel runs
+// final_norm after the last layer).  next: the next layer's weights (qkv_kernel or g1_kernel runs
 // next on the stream), or null after the last layer.
 template <int KW>
 __global__ __launch_bounds__(64 * kWaves) void g6_kernel(StepArgs s, LayerWeights L,
                                                          const float* next_norm,
                                                          const uint16_t* next_dq_dkv,
-                                                         const uint16_t* next_uq,
-                                                         const uint16_t* next_uk) {
+                                                         const uint16_t* next_q) {
     __shared__ __attribute__((aligned(16))) uint16_t pf_scratch[512];
     const ModelDims& m = s.dims;
     const int row0 = blockIdx.y * 16, KT = m.ff_pad / 32;
     splitk_residual<KW>(
         [&](floatx4(&acc)[1][1], const BPre<1, KW>& bw, int kt0, int lane) {
             APre16<KW, 1> a;
-            a.load(s.u + (long long)row0 * m.ff_pad, m.ff_pad, KT, kt0, kWaves, lane);
+            a.load(s.u + (long long)row0 * m.ff_pad, m.ff_pad, s.B - row0, KT, kt0, kWaves, lane);
+            operands_issued();
             mma_steps(acc, bw, [&](int kk, int mt) { return a.x[kk][mt]; });
         },
-        L.w_down, KT, m.d_model, s.res, next_norm, s.x, s.xw, s.ss_x, m.d_pad / 16, m.d_pad,
+        L.w_down, s.zeros, KT, m.d_model, s.res, next_norm, s.x, s.xw, s.ss_x, m.d_pad / 16, m.d_pad,
         row0, s.B, [&]() {
             if (!next_dq_dkv)
                 return;
-            // qkv_kernel runs head h with residue h % 8 and the append workgroup (h = H) with H % 8:
-            // head workgroups read the w_dq tiles, the append one the w_dkv tiles, and head h
-            // its w_uq and W_uk blocks (contiguous per head)
-            const int x = block_xcd(), KTq = m.d_pad / 32, q_tiles = m.q_pad / 16;
-            const int n_dq = x < m.H ? q_tiles * KTq : 0;
-            const int n_dkv = m.H % kXcds == x ? (m.kvw_pad / 16) * KTq : 0;
-            const int n_uq = (m.qk_pad / 16) * (m.q_pad / 32), n_uk = (m.kv_pad / 16) * (m.nope_pad / 32);
-            const int heads = x < m.H ? (m.H - x + kXcds - 1) / kXcds : 0;
-            l2_prefetch(n_dq + n_dkv + heads * (n_uq + n_uk), [&](int k) {
-                if (k < n_dq)
-                    return next_dq_dkv + (long long)k * 512;
-                k -= n_dq;
-                if (k < n_dkv)
-                    return next_dq_dkv + ((long long)q_tiles * KTq + k) * 512;
-                k -= n_dkv;
-                const int h = x + kXcds * (k / (n_uq + n_uk));
-                k %= n_uq + n_uk;
-                return k < n_uq ? next_uq + ((long long)h * n_uq + k) * 512
-                                : next_uk + ((long long)h * n_uk + k - n_uq) * 512;
+            if (s.B <= kQkvMaxRows) {
+                // qkv_kernel runs head h with residue h % 8 and the append workgroup (h = H) with
+                // H % 8: head workgroups read the w_dq tiles, the append one the w_dkv tiles, and
+                // head h its w_q blocks (contiguous per head)
+                const int x = block_xcd(), KTq = m.d_pad / 32, q_tiles = m.q_pad / 16;
+                const int n_dq = x < m.H ? q_tiles * KTq : 0;
+                const int n_dkv = m.H % kXcds == x ? (m.kvw_pad / 16) * KTq : 0;
+                const int n_q = (m.hq_pad / 16) * (m.q_pad / 32);
+                const int heads = x < m.H ? (m.H - x + kXcds - 1) / kXcds : 0;
+                l2_prefetch(n_dq + n_dkv + heads * n_q, [&](int k) {
+                    if (k < n_dq)
+                        return next_dq_dkv + (long long)k * 512;
+                    k -= n_dq;
+                    if (k < n_dkv)
+                        return next_dq_dkv + ((long long)q_tiles * KTq + k) * 512;
+                    k -= n_dkv;
+                    const int h = x + kXcds * (k / n_q);
+                    return next_q + ((long long)h * n_q + k % n_q) * 512;
+                }, pf_scratch, 1);
+                return;
+            }
+            // g1_kernel runs column tile t with residue t % 8 (its KT blocks are contiguous)
+            const int x = block_xcd(), KT1 = m.d_pad / 32, tiles = (m.q_pad + m.kvw_pad) / 16;
+            l2_prefetch(x < tiles ? (tiles - x + kXcds - 1) / kXcds * KT1 : 0, [&](int k) {
+                return next_dq_dkv + ((long long)(x + kXcds * (k / KT1)) * KT1 + k % KT1) * 512;
             }, pf_scratch, 1);
         });
 }
@@ -766,18 +850,19 @@ __global__ __launch_bounds__(64 * kWaves) void g5_kernel(StepArgs s, LayerWeight
     const int row0 = blockIdx.y * 16, p = blockIdx.x;
     if (p >= m.ff_pad / 16)
         return;  // the grid's columns are padded to a multiple of 8 (one XCD per pair)
-    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, g = lane >> 4, n = lane & 15;
+    const int wave = wave_index(), lane = threadIdx.x & 63, g = lane >> 4, n = lane & 15;
     const int KT = m.d_pad / 32;
     RmsPrefetch<16> rms;
     rms.issue(s.ss_res, m.d_pad / 16, row0, 16);
     BPre<2, KW> bw;
-    bw.load(L.w_gate_up, 2 * p, 2, KT, wave, kWaves, lane);
+    bw.load(L.w_gate_up, s.zeros, 2 * p, 2, KT, wave, kWaves, lane);
     APre16<KW, 1> a;
-    a.load(s.resw + (long long)row0 * m.d_pad, m.d_pad, KT, wave, kWaves, lane);
+    a.load(s.resw + (long long)row0 * m.d_pad, m.d_pad, s.B - row0, KT, wave, kWaves, lane);
+    operands_issued();
     floatx4 acc[1][2];
     zero(acc);
     mma_steps(acc, bw, [&](int kk, int mt) { return a.x[kk][mt]; });
-    rms.finish(m.d_model, m.eps, inv_s, 16);
+    rms.finish(m.d_pad / 16, m.d_model, m.eps, inv_s, 16);
     int mt;
     floatx4 v[2];
     if (!splitk_reduce<1, 2, kWaves>(acc, part, mt, v))
@@ -837,19 +922,20 @@ __global__ __launch_bounds__(64 * kWaves) void g7_kernel(StepArgs s) {
     __shared__ float inv_s[64];
     const ModelDims& m = s.dims;
     const int row0 = blockIdx.y * 64;
-    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, g = lane >> 4, n = lane & 15;
+    const int wave = wave_index(), lane = threadIdx.x & 63, g = lane >> 4, n = lane & 15;
     const int KT = m.d_pad / 32, kg = wave % kG7KG, ng = wave / kG7KG;
     const int n_tiles = m.vocab_pad / 16, nt0 = blockIdx.x * kG7Tiles;
     RmsPrefetch<8> rms;
     rms.issue(s.ss_x, m.d_pad / 16, row0, 64);
     BPre<NTW, KW> bw;
-    bw.load(s.embed, nt0 + ng * NTW, min(NTW, n_tiles - nt0 - ng * NTW), KT, kg, kG7KG, lane);
+    bw.load(s.embed, s.zeros, nt0 + ng * NTW, min(NTW, n_tiles - nt0 - ng * NTW), KT, kg, kG7KG, lane);
     APre16<KW, 4> a;
-    a.load(s.xw + (long long)row0 * m.d_pad, m.d_pad, KT, kg, kG7KG, lane);
+    a.load(s.xw + (long long)row0 * m.d_pad, m.d_pad, s.B - row0, KT, kg, kG7KG, lane);
+    operands_issued();
     floatx4 acc[4][NTW];
     zero(acc);
     mma_steps(acc, bw, [&](int kk, int mt) { return a.x[kk][mt]; });
-    rms.finish(m.d_model, m.eps, inv_s, 64);
+    rms.finish(m.d_pad / 16, m.d_model, m.eps, inv_s, 64);
     int mt;
     floatx4 v[kG7Tiles];
     if (!splitk_reduce<4, NTW, kG7KG>(acc, part, mt, v))
@@ -998,6 +1084,8 @@ int g7_parts(const ModelDims& m) { return ceil_div(m.vocab_pad / 16, kG7Tiles); 
     default: hipLaunchKernelGGL(KERNEL<4>, __VA_ARGS__); break;                                  \
     }
 
+int layer_pre_launches(int rows) { return rows <= kQkvMaxRows ? 1 : 2; }
+
 size_t qkv_lds_bytes(const ModelDims& m) { return (size_t)qkv_lds(m).total; }
 
 // Kernels whose dynamic LDS can exceed 64 KB: allow what this model's shape needs.
@@ -1023,27 +1111,37 @@ hipError_t launch_embed(const StepArgs& s, const float* first_norm, hipStream_t 
 }
 
 hipError_t launch_layer_pre(const StepArgs& s, const LayerWeights& w, uint16_t* pool,
-                            const PagePrefetch& pf, hipStream_t st) {
+                            hipStream_t st) {
     const ModelDims& m = s.dims;
-    const size_t lds = qkv_lds_bytes(m);
-    // heads padded to 8 columns (see l2_prefetch), then 8 read-ahead columns (page_prefetch,
-    // 1 KB of the LDS per wave)
-    const bool ahead = pf.max_work > 0 && pf.pages > 0 && lds >= kQkvWaves * 1024;
-    const dim3 grid(round_up_to(m.H + 1, kXcds) + (ahead ? kXcds : 0), ceil_div(s.B, kQkvRows));
-    const int nt = max(m.q_pad, m.kvw_pad) / 16;  // <= 16 (mla_model_create checks)
-    const int tiles = nt <= 4 ? 4 : nt <= 8 ? 8 : nt <= 12 ? 12 : 16;
-    // d_pad <= 512: one chunk of two k-steps per wave; <= 1024: two
-    const int kc = m.d_pad / 32 <= 2 * kQkvWaves ? 1 : 2;
+    if (layer_pre_launches(s.B) == 1) {
+        const size_t lds = qkv_lds_bytes(m);
+        const dim3 grid(round_up_to(m.H + 1, kXcds), ceil_div(s.B, kQkvRows));  // padded: see l2_prefetch
+        const int nt = max(m.q_pad, m.kvw_pad) / 16;  // <= 16 (mla_model_create checks)
+        const int tiles = nt <= 4 ? 4 : nt <= 8 ? 8 : nt <= 12 ? 12 : 16;
+        // d_pad <= 512: one chunk of two k-steps per wave; <= 1024: two
+        const int kc = m.d_pad / 32 <= 2 * kWaves ? 1 : 2;
 #define MLA_QKV(KC, NT)                                                                         \
-    hipLaunchKernelGGL((qkv_kernel<KC, NT>), grid, dim3(64 * kQkvWaves), lds, st, s, w, pool, pf)
-    if (kc == 1) {
-        if (tiles == 4) MLA_QKV(1, 4); else if (tiles == 8) MLA_QKV(1, 8);
-        else if (tiles == 12) MLA_QKV(1, 12); else MLA_QKV(1, 16);
-    } else {
-        if (tiles == 4) MLA_QKV(2, 4); else if (tiles == 8) MLA_QKV(2, 8);
-        else if (tiles == 12) MLA_QKV(2, 12); else MLA_QKV(2, 16);
-    }
+    hipLaunchKernelGGL((qkv_kernel<KC, NT>), grid, dim3(64 * kWaves), lds, st, s, w, pool)
+        if (kc == 1) {
+            if (tiles == 4) MLA_QKV(1, 4); else if (tiles == 8) MLA_QKV(1, 8);
+            else if (tiles == 12) MLA_QKV(1, 12); else MLA_QKV(1, 16);
+        } else {
+            if (tiles == 4) MLA_QKV(2, 4); else if (tiles == 8) MLA_QKV(2, 8);
+            else if (tiles == 12) MLA_QKV(2, 12); else MLA_QKV(2, 16);
+        }
 #undef MLA_QKV
+        return hipGetLastError();
+    }
+    const int chunks = ceil_div(s.B, 16);
+    const int tiles = (m.q_pad + m.kvw_pad) / 16;
+    MLA_KW4_DISPATCH(kw_variant(ceil_div(m.d_pad / 32, kWaves)), g1_kernel,
+                     dim3(round_up_to(tiles, kXcds), chunks), dim3(64 * kWaves), 0, st, s, w);
+    hipError_t e = hipGetLastError();
+    if (e != hipSuccess)
+        return e;
+    const int wgs = ceil_div(m.H * (m.hq_pad / 16), kG2Waves);
+    MLA_KW_DISPATCH(kw_variant(m.q_pad / 32), g2_kernel, dim3(round_up_to(wgs + 1, kXcds), chunks),
+                    dim3(64 * kG2Waves), 0, st, s, w, pool);
     return hipGetLastError();
 }
 
@@ -1064,8 +1162,7 @@ hipError_t launch_layer_post(const StepArgs& s, const LayerWeights& w, const flo
         return e;
     MLA_KW_DISPATCH(kw_variant(ceil_div(m.ff_pad / 32, kWaves)), g6_kernel,
                     dim3(d_tiles, chunks), dim3(64 * kWaves), 0, st, s, w, next_norm,
-                    next ? next->w_dq_dkv : nullptr, next ? next->w_uq : nullptr,
-                    next ? next->w_uk : nullptr);
+                    next ? next->w_dq_dkv : nullptr, next ? next->w_q : nullptr);
     return hipGetLastError();
 }
 

@@ -18,11 +18,6 @@ namespace {
 
 int round_up(int x, int m) { return (x + m - 1) / m * m; }
 
-// Leading pages of each decode work item that qkv_kernel reads ahead into L2 (page_prefetch).
-// Config 3 (570 items of 4 pages): 1 page took the step from 0.3854 to 0.3816 ms; 2 and 3
-// pages (20 and 30 MB) outlast qkv_kernel (14.8 and 20 us) and slowed the step.
-constexpr int kReadAheadPages = 1;
-
 // ModelConfig::validate (src/model/config.cpp:20-48) and parameter_count (:7-19).
 size_t parameter_count(const mla_model_config& c) {
     const size_t d = c.d_model, h = c.n_heads, q = c.q_lora_rank, kv = c.kv_lora_rank;
@@ -82,6 +77,23 @@ std::vector<uint16_t> pack(int K, int N, int Kpad, int Npad, F at) {
     return out;
 }
 
+// row[j] += x[t] * b[t * ld + j], t = 0 .. terms - 1 in order, four terms per pass over the row.
+void add_products(float* row, int n, const float* x, const float* b, size_t ld, int terms) {
+    int t = 0;
+    for (; t + 4 <= terms; t += 4, b += 4 * ld)
+        for (int j = 0; j < n; ++j) {
+            float v = row[j];
+            v += x[t] * b[j];
+            v += x[t + 1] * b[ld + j];
+            v += x[t + 2] * b[2 * ld + j];
+            v += x[t + 3] * b[3 * ld + j];
+            row[j] = v;
+        }
+    for (; t < terms; ++t, b += ld)
+        for (int j = 0; j < n; ++j)
+            row[j] += x[t] * b[j];
+}
+
 // Offsets of the reference parameter registry (include/mini_mla/model.hpp:15-30,
 // src/model/model.cpp:40-63): token_embedding, final_norm, then per layer attn_norm,
 // w_dq, q_norm, w_uq, w_dkv, kv_norm, w_uk, w_uv, w_o, ffn_norm, w_gate, w_up, w_down.
@@ -126,9 +138,10 @@ struct Model {
     const float* final_norm = nullptr;
     const float* rope_tab = nullptr;
     float *x, *res, *ctx, *logits, *arg_v;
-    float *ss_x, *ss_res;
+    float *ss_x, *ss_res, *ss_cq, *ss_kv, *ckv;
     float2* rope_rows;
-    uint16_t *xw, *resw, *u, *q_latent, *q_rope;
+    uint16_t *xw, *resw, *u, *q_latent, *q_rope, *cqw;
+    uint16_t* zeros = nullptr;  // 512 zero words
     int32_t* arg_c;
     uint32_t* ban_bits = nullptr;  // [ceil(vocab/32)] banned token ids, allocated on first use
     bool banning = false;          // some id is banned: the greedy token skips them
@@ -196,9 +209,8 @@ ModelDims make_dims(const mla_model_config& c, int page_size) {
     m.d_pad = round_up(c.d_model, 32);
     m.q_pad = round_up(c.q_lora_rank, 32);
     m.kvw_pad = round_up(c.kv_lora_rank + c.head_dim_rope, 16);
-    m.qk_pad = round_up(m.qk, 16);
-    m.nope_pad = round_up(c.head_dim_nope, 32);
     m.kv_pad = round_up(c.kv_lora_rank, 16);
+    m.hq_pad = m.kv_pad + round_up(c.head_dim_rope, 16);
     m.ctx_pad = round_up(c.n_heads * c.kv_lora_rank, 32);
     m.ff_pad = round_up(c.d_ff, 32);
     m.vocab_pad = round_up(c.vocab_size, 16);
@@ -231,7 +243,7 @@ hipError_t upload_weights(Model* M, const float* params) {
             }
         e = M->upload(M->rope_tab, tab);
     }
-    std::vector<float> proj((size_t)H * kv * d);
+    std::vector<float> proj((size_t)H * kv * d), absorbed, uk((size_t)nope * kv);
     std::vector<LayerWeights> layers;
     for (int l = 0; l < c.n_layers && e == hipSuccess; ++l) {
         const float* const* P = R.layer.data() + (size_t)l * P_COUNT;
@@ -252,32 +264,34 @@ hipError_t upload_weights(Model* M, const float* params) {
                                   return 0.0f;
                               return P[P_W_DKV][(size_t)k * kvw + (col - m.q_pad)];
                           }));
-        if (e == hipSuccess)  // w_uq: head h at columns h*qk_pad ..
-            e = M->upload(w.w_uq, pack(q, H * m.qk_pad, m.q_pad, H * m.qk_pad, [&](int k, int col) {
-                              const int h = col / m.qk_pad, cc = col % m.qk_pad;
-                              return cc < qk ? P[P_W_UQ][(size_t)k * H * qk + h * qk + cc] : 0.0f;
-                          }));
-        if (e == hipSuccess) {  // W_uk_h^T per head: (k = nope index, col = latent index)
-            std::vector<uint16_t> all;
+        if (e == hipSuccess) {
+            // w_q, head h at columns h*hq_pad ..: the absorption W_uk_h^T folded into the nope
+            // columns of W_uq (fp32 sums, rounded once, like W_uv.W_o below), then the rope
+            // columns of W_uq
+            absorbed.assign((size_t)q * H * kv, 0.0f);
             for (int h = 0; h < H; ++h) {
-                auto blk = pack(nope, kv, m.nope_pad, m.kv_pad, [&](int k, int col) {
-                    return P[P_W_UK][(size_t)col * H * nope + h * nope + k];
-                });
-                all.insert(all.end(), blk.begin(), blk.end());
+                for (int t = 0; t < nope; ++t)
+                    for (int r = 0; r < kv; ++r)
+                        uk[(size_t)t * kv + r] = P[P_W_UK][(size_t)r * H * nope + h * nope + t];
+                for (int k = 0; k < q; ++k)
+                    add_products(absorbed.data() + ((size_t)k * H + h) * kv, kv,
+                                 P[P_W_UQ] + (size_t)k * H * qk + h * qk, uk.data(), kv, nope);
             }
-            e = M->upload(w.w_uk, all);
+            e = M->upload(w.w_q, pack(q, H * m.hq_pad, m.q_pad, H * m.hq_pad, [&](int k, int col) {
+                              const int h = col / m.hq_pad, cc = col % m.hq_pad;
+                              if (cc < m.kv_pad)
+                                  return cc < kv ? absorbed[((size_t)k * H + h) * kv + cc] : 0.0f;
+                              const int t = nope + cc - m.kv_pad;
+                              return t < qk ? P[P_W_UQ][(size_t)k * H * qk + h * qk + t] : 0.0f;
+                          }));
         }
         if (e == hipSuccess) {  // combined W_uv.W_o (CpuDecoder::prepare_projections, inference.cpp:28-46)
             for (int h = 0; h < H; ++h)
                 for (int r = 0; r < kv; ++r) {
                     float* row = proj.data() + ((size_t)h * kv + r) * d;
                     std::memset(row, 0, (size_t)d * sizeof(float));
-                    for (int t = 0; t < dv; ++t) {
-                        const float a = P[P_W_UV][(size_t)r * H * dv + h * dv + t];
-                        const float* b = P[P_W_O] + (size_t)(h * dv + t) * d;
-                        for (int j = 0; j < d; ++j)
-                            row[j] += a * b[j];
-                    }
+                    add_products(row, d, P[P_W_UV] + (size_t)r * H * dv + h * dv,
+                                 P[P_W_O] + (size_t)h * dv * d, d, dv);
                 }
             e = M->upload(w.w_out, pack(H * kv, d, m.ctx_pad, m.d_pad, [&](int k, int col) {
                               return proj[(size_t)k * d + col];
@@ -339,6 +353,7 @@ int model_forward(Model* M, hipStream_t st, int rows, const int32_t* tokens,
     s.num_pool_pages = md.num_pool_pages;
     s.embed = M->embed;
     s.final_norm = M->final_norm;
+    s.zeros = M->zeros;
     s.rope_tab = reinterpret_cast<const float2*>(M->rope_tab);
     s.x = M->x;
     s.res = M->res;
@@ -354,6 +369,10 @@ int model_forward(Model* M, hipStream_t st, int rows, const int32_t* tokens,
     s.arg_c = M->arg_c;
     s.ban = M->banning ? M->ban_bits : nullptr;
     s.next_tokens = next_tokens;
+    s.cqw = M->cqw;
+    s.ckv = M->ckv;
+    s.ss_cq = M->ss_cq;
+    s.ss_kv = M->ss_kv;
     s.ss_x = M->ss_x;
     s.ss_res = M->ss_res;
     DecodeArgs a{};
@@ -401,23 +420,12 @@ int model_forward(Model* M, hipStream_t st, int rows, const int32_t* tokens,
         return bad;
     // decode (+ the split merge unless the decode launch merges itself)
     const int attn_launches = md.max_work > 0 && B > 0 ? 2 - a.fused_merge : 0;
-    // The MFMA page kernel's leading pages are read ahead into L2 during qkv_kernel.
-    PagePrefetch pf{};
-    if (attn_launches > 0 && !generic && !(md.flags & MLA_STEP_NO_READ_AHEAD) &&
-        decode_mfma_supported(a.H, a.kv_rank, a.rope_dim, a.page_size)) {
-        pf.work_desc = md.work_desc;
-        pf.work_pages = md.work_pages;
-        pf.max_work = md.max_work;
-        pf.pages = kReadAheadPages;
-        pf.page_size = m.page_size;
-        pf.record = m.page_size * (m.kv_rank + m.rope);
-    }
     hipError_t e = launch_embed(s, M->layers[0].attn_norm, st);
     uint64_t launched = 1;
     for (int l = 0; l < m.n_layers && e == hipSuccess; ++l) {
         const float* next_norm = l + 1 < m.n_layers ? M->layers[l + 1].attn_norm : M->final_norm;
         uint16_t* pool = static_cast<uint16_t*>(pages[l]);
-        e = launch_layer_pre(s, M->layers[l], pool, pf, st);
+        e = launch_layer_pre(s, M->layers[l], pool, st);
         if (e != hipSuccess)
             break;
         a.pages = pool;
@@ -432,7 +440,7 @@ int model_forward(Model* M, hipStream_t st, int rows, const int32_t* tokens,
         if (e == hipSuccess)
             e = launch_layer_post(s, M->layers[l], next_norm,
                                   l + 1 < m.n_layers ? &M->layers[l + 1] : nullptr, st);
-        launched += 1 + attn_launches + (max_q_len > 1) + 3;
+        launched += layer_pre_launches(rows) + attn_launches + (max_q_len > 1) + 3;
     }
     if (e == hipSuccess && rows != B && !all_rows) {  // logits of each session's last row only
         StepArgs t = s;
@@ -475,12 +483,12 @@ int mla_model_create(const mla_model_config* config, const float* params, int ma
         return fail(MLA_ERR_INVALID_ARGUMENT, "mla_model_create: invalid argument");
     const mla_model_config& c = *config;
     const ModelDims m = make_dims(c, page_size);
-    // Shapes the step kernels cover: a head's q within one workgroup (<= 4 tiles) and its
-    // absorption within 4 waves x 2 tiles, at most 8 k-steps per split-K wave (d_model,
-    // q_lora_rank: 4 with their on-the-fly norms), fp32 rows read 8 columns at a time.
-    if (m.qk_pad / 16 > 4 || m.kv_pad / 16 > 8 || (c.n_heads * c.kv_lora_rank) % 8 ||
+    // Shapes the step kernels cover: a head's latent and rope columns within 8 waves x 2
+    // tiles, at most 8 k-steps per split-K wave (d_model, q_lora_rank: 4 with their
+    // on-the-fly norms), fp32 rows read 8 columns at a time.
+    if (m.qk > 64 || m.kv_pad / 16 > 8 || (c.n_heads * c.kv_lora_rank) % 8 ||
         c.d_model % 8 || c.q_lora_rank % 8 || m.d_pad > 1024 || m.q_pad > 256 ||
-        m.nope_pad > 128 || m.ctx_pad / 32 > 64 || m.ff_pad / 32 > 64)
+        m.ctx_pad / 32 > 64 || m.ff_pad / 32 > 64)
         return fail(MLA_ERR_UNSUPPORTED,
                     "mla_model_create: shape outside the step kernels (head_dim_nope + "
                     "head_dim_rope <= 64, kv_lora_rank <= 128, head_dim_nope <= 128, "
@@ -508,6 +516,7 @@ int mla_model_create(const mla_model_config* config, const float* params, int ma
     e = upload_weights(M, params);
     const size_t rows = M->m_pad_max;
     const int H = c.n_heads, kv = c.kv_lora_rank;
+    if (e == hipSuccess) e = M->alloc(M->zeros, 512);
     if (e == hipSuccess) e = M->alloc(M->x, rows * m.d_pad);
     if (e == hipSuccess) e = M->alloc(M->res, rows * m.d_pad);
     if (e == hipSuccess) e = M->alloc(M->xw, rows * m.d_pad);
@@ -520,6 +529,10 @@ int mla_model_create(const mla_model_config* config, const float* params, int ma
     if (e == hipSuccess) e = M->alloc(M->logits, (size_t)max_batch * c.vocab_size);
     if (e == hipSuccess) e = M->alloc(M->arg_v, (size_t)max_batch * M->parts);
     if (e == hipSuccess) e = M->alloc(M->arg_c, (size_t)max_batch * M->parts);
+    if (e == hipSuccess) e = M->alloc(M->cqw, rows * m.q_pad);
+    if (e == hipSuccess) e = M->alloc(M->ckv, rows * m.kvw_pad);
+    if (e == hipSuccess) e = M->alloc(M->ss_cq, rows * (m.q_pad / 16));
+    if (e == hipSuccess) e = M->alloc(M->ss_kv, rows * (m.kvw_pad / 16));
     if (e == hipSuccess) e = M->alloc(M->ss_x, rows * (m.d_pad / 16));
     if (e == hipSuccess) e = M->alloc(M->ss_res, rows * (m.d_pad / 16));
     if (e == hipSuccess) e = hipDeviceSynchronize();

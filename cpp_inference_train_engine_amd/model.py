@@ -127,8 +127,8 @@ class HipModel:
              stream=None, read_ahead=True):
         """One decode step.  ``batch`` is the RaggedBatch of mla_build_metadata (q_len = 1,
         ctx_len = positions); ``pages`` is the list of per-layer page pools; tokens and
-        positions are device int32 [B].  read_ahead=False turns off the L2 read-ahead of
-        the attention's pages (MLA_STEP_NO_READ_AHEAD: same results, other timing).
+        positions are device int32 [B].  read_ahead=False passes
+        MLA_STEP_NO_READ_AHEAD, which changes nothing.
         Returns (logits [B x vocab] fp32, next_tokens [B])."""
         import torch
         B = int(tokens.numel())

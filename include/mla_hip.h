@@ -64,9 +64,8 @@ extern "C" {
 /* Decode-attention flags. */
 #define MLA_DECODE_FORCE_GENERIC 1 /* use the portable VALU kernel even when the MFMA one fits */
 #define MLA_DECODE_FUSED_MERGE 2   /* metadata built with placement = 1: merge inside the launch */
-/* mla_model_step / mla_model_forward: no read-ahead of the decode attention's pages into L2
- * during each layer's projection kernel (the results are the same bit for bit; the
- * read-ahead only changes timing). */
+/* mla_model_step / mla_model_forward: accepted and without effect (it turned off a read-ahead of
+ * the decode attention's pages that the step no longer makes). */
 #define MLA_STEP_NO_READ_AHEAD 4
 
 /* Message of the last failed call on this thread ("" if none). */
@@ -375,8 +374,8 @@ int mla_model_update_weights(void* model, const float* params, uint64_t* revisio
  * when the metadata was built XCD-placed (the decode attention of each layer is then
  * one launch, see mla_decode_attention: check mla_decode_status on `workspace` after
  * the step, and rerun it without the flag if a bit is set -- the step's appends are
- * idempotent), else 0; optionally with MLA_STEP_NO_READ_AHEAD (no L2 read-ahead of the
- * attention's pages, same results). */
+ * idempotent), else 0; MLA_STEP_NO_READ_AHEAD is accepted and
+ * changes nothing. */
 int mla_model_step(void* model, void* stream, int B, const int32_t* tokens,
                    const int32_t* positions, const int32_t* cu_seqlens_q,
                    const int32_t* page_table, int max_pages, int num_pool_pages,
