@@ -157,8 +157,7 @@ __device__ __forceinline__ void fused_merge_tail(const DecodeArgs& a, int s, int
             }
         }
         const float inv = L > 0.0f ? 1.0f / L : 0.0f;
-        __builtin_nontemporal_store(
-            O * inv, reinterpret_cast<floatx4*>(a.out + ((long long)row * a.H + h) * KV + c));
+        store_row<true>(a.out, a.out16, ((long long)row * a.H + h) * KV + c, O * inv);
         if (a.lse && c == 0)
             a.lse[(long long)row * a.H + h] = (M + __log2f(L)) * kLn2;
     }
@@ -177,7 +176,7 @@ __device__ __forceinline__ void unplaced_tail(const DecodeArgs& a, int row, bool
         return;
     const float nan = __builtin_nanf("");
     for (int e = tid; e < a.H * KV; e += THREADS)
-        a.out[(long long)row * a.H * KV + e] = nan;
+        store_row(a.out, a.out16, (long long)row * a.H * KV + e, nan);
     if (a.lse)
         for (int h = tid; h < a.H; h += THREADS)
             a.lse[(long long)row * a.H + h] = nan;
@@ -247,6 +246,7 @@ void decode_page_kernel(DecodeArgs a) {
     const float scale_log2 = a.scale_log2;
     // The XCD count the metadata was placed for (the fused merge's premise, checked at the end).
     const int placed_n = FUSED ? a.info[kInfoPlacement] : 0;
+
     asm volatile("" ::"s"(pid[0]), "s"(H), "s"(npool), "s"(pool), "s"(scale_log2), "s"(placed_n));
     const int s = d[0];
     if (s < 0 || d[7] != 1)
@@ -457,8 +457,7 @@ void decode_page_kernel(DecodeArgs a) {
         // 0.3 us less per config-3 launch than plain ones).
         if (ns == 1) {
             const float inv = lh > 0.0f ? 1.0f / lh : 0.0f;
-            __builtin_nontemporal_store(
-                o * inv, reinterpret_cast<floatx4*>(a.out + ((long long)row * a.H + h) * KV + c));
+            store_row<true>(a.out, a.out16, ((long long)row * a.H + h) * KV + c, o * inv);
             if (a.lse && c == 0)
                 a.lse[(long long)row * a.H + h] = (mh + __log2f(lh)) * kLn2;
         } else if constexpr (FUSED) {  // plain stores: the partials stay in this XCD's L2
@@ -591,7 +590,7 @@ __global__ __launch_bounds__(kGenThreads) void decode_generic_kernel(DecodeArgs 
             for (int k = 0; k < kGenMaxAcc; ++k) {
                 const int r = tid + k * kGenThreads;
                 if (r < KV)
-                    a.out[((long long)row * a.H + h) * KV + r] = acc[k] * inv;
+                    store_row(a.out, a.out16, ((long long)row * a.H + h) * KV + r, acc[k] * inv);
             }
             if (a.lse && tid == 0)
                 a.lse[(long long)row * a.H + h] = (m_run + __log2f(l_run)) * kLn2;
@@ -698,7 +697,11 @@ __global__ __launch_bounds__(kMergeElems* G) void merge_kernel(DecodeArgs a) {
     for (int q = 1; q < G; ++q)
         fold1(sm_m[q][t], sm_l[q][t], sm_o[q][t]);
     const float inv = L > 0.0f ? 1.0f / L : 0.0f;
-    *reinterpret_cast<vecV*>(a.out + ((long long)row * H + h) * KV + c) = O * inv;
+    const long long at = ((long long)row * H + h) * KV + c;
+    if constexpr (V == 4)
+        store_row<false>(a.out, a.out16, at, O * inv);
+    else
+        store_row(a.out, a.out16, at, O[0] * inv);
     if (a.lse && c == 0)
         a.lse[(long long)row * H + h] = (M + __log2f(L)) * kLn2;
 }

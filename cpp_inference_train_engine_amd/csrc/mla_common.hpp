@@ -175,6 +175,28 @@ __device__ __forceinline__ void copy_4blocks_to_lds_at(const void* base, uint32_
 }
 #pragma clang diagnostic pop
 
+// Four consecutive values (or one) of a final attention row at element i: fp32 to out, or, for
+// a caller whose next kernel rounds the row to fp16 anyway (the model's output projection),
+// rounded here to out16: the same bits in half the bytes.
+template <bool NT>
+__device__ __forceinline__ void store_row(float* out, uint16_t* out16, long long i, floatx4 v) {
+    typedef _Float16 half4 __attribute__((ext_vector_type(4)));
+    if (out16) {
+        const half4 h = {(_Float16)v[0], (_Float16)v[1], (_Float16)v[2], (_Float16)v[3]};
+        *reinterpret_cast<half4*>(out16 + i) = h;
+    } else if constexpr (NT) {
+        __builtin_nontemporal_store(v, reinterpret_cast<floatx4*>(out + i));
+    } else {
+        *reinterpret_cast<floatx4*>(out + i) = v;
+    }
+}
+__device__ __forceinline__ void store_row(float* out, uint16_t* out16, long long i, float v) {
+    if (out16)
+        out16[i] = F16::from_float(v);
+    else
+        out[i] = v;
+}
+
 // Orders this wave's LDS accesses: nothing before it moves after it, or after it before.
 __device__ __forceinline__ void wave_lds_fence() {
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");

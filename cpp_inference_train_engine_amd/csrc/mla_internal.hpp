@@ -57,6 +57,9 @@ struct DecodeArgs {
     const int32_t *cu_q, *page_table, *num_splits, *cu_splits, *work_desc, *work_pages, *info;
     const uint16_t *pages, *q_latent, *q_rope;
     float *out, *lse, *part_o, *part_ml;
+    // When not null, final rows go here as fp16 instead of to `out` (the model step; every
+    // kernel but decode_wide_kernel, whose shape no model has).
+    uint16_t* out16;
     // Fused merge (decode_page_kernel only): the metadata was built XCD-placed, and the
     // last item of a split session to finish combines the session's partials itself.
     // merge_count[B] (in the workspace, zero between launches) counts finished items.
@@ -80,6 +83,7 @@ struct PrefillArgs {
     const int32_t *cu_q, *cu_k, *page_table, *info;
     const uint16_t *pages, *q_latent, *q_rope;
     float *out, *lse;
+    uint16_t* out16;  // as DecodeArgs::out16
 };
 
 hipError_t launch_build_metadata(const MetadataArgs& a, hipStream_t stream);

@@ -58,7 +58,8 @@ struct StepArgs {
     const float2* rope_tab;    // [max_seq x rope/2] (cos, sin) of pos * theta^(-j/rope)
     float2* rope_rows;         // [m_pad x rope/2] the table rows of this step's positions
     // activations (rows padded to m_pad)
-    float *x, *res, *ctx;       // [m_pad x d_pad], [m_pad x d_pad], [m_pad x H*kv_rank]
+    float *x, *res;             // [m_pad x d_pad]
+    const uint16_t* ctx;        // [m_pad x H*kv_rank] fp16 attention rows
     uint16_t *cqw;              // [m_pad x q_pad] fp16 cq o q_norm
     float* ckv;                 // [m_pad x kvw_pad] latent o kv_norm, then the key before RoPE
     uint16_t *xw, *resw;        // fp16 x o (next norm weight), res o ffn_norm [m_pad x d_pad]

@@ -47,11 +47,6 @@ __device__ __forceinline__ floatx4 mma(V8 a, V8 b, floatx4 c) {
     return __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, c, 0, 0, 0);
 }
 
-__device__ __forceinline__ V8 to_half8(floatx4 a, floatx4 b) {
-    return V8{(_Float16)a[0], (_Float16)a[1], (_Float16)a[2], (_Float16)a[3],
-              (_Float16)b[0], (_Float16)b[1], (_Float16)b[2], (_Float16)b[3]};
-}
-
 // ---- L2 prefetch for the next kernel on the stream -------------------------------------
 // Workgroups b of a launch (x-fastest linear id) with one residue b % 8 run on one XCD:
 // the dispatcher deals workgroups to the 8 XCDs in turn, starting on an XCD that depends
@@ -162,9 +157,9 @@ struct BPre {
 // columns 32kt + 8g .. +7 of each of its k-steps.  Rows past `rows` (>= 1) repeat the last one:
 // their products are dropped, and the lanes that share its address add no traffic.
 template <int KW, int MT>
-struct APre16 {  // fp16 rows, zero-padded to KT*32 columns
+struct APre16 {  // fp16 rows of K % 8 == 0 columns (the weights of columns past K are 0)
     V8 x[KW][MT];
-    __device__ __forceinline__ void load(const uint16_t* X, int ld, int rows, int KT, int kt0,
+    __device__ __forceinline__ void load(const uint16_t* X, int ld, int rows, int K, int kt0,
                                          int ks, int lane) {
         const int g = lane >> 4, n = lane & 15;
 #pragma unroll
@@ -172,25 +167,7 @@ struct APre16 {  // fp16 rows, zero-padded to KT*32 columns
 #pragma unroll
             for (int mt = 0; mt < MT; ++mt)
                 x[kk][mt] = *reinterpret_cast<const V8*>(X + (long long)min(16 * mt + n, rows - 1) * ld +
-                                                         32 * min(kt0 + kk * ks, KT - 1) + 8 * g);
-    }
-};
-template <int KW, int MT>
-struct AHalf32 {  // fp32 rows (K % 8 == 0; the weights of columns past K are 0), rounded to fp16
-    floatx4 x[KW][MT][2];
-    __device__ __forceinline__ void load(const float* X, int ld, int rows, int K, int kt0, int ks,
-                                         int lane) {
-        const int g = lane >> 4, n = lane & 15;
-#pragma unroll
-        for (int kk = 0; kk < KW; ++kk)
-#pragma unroll
-            for (int mt = 0; mt < MT; ++mt) {
-                const floatx4* p = reinterpret_cast<const floatx4*>(
-                    X + (long long)min(16 * mt + n, rows - 1) * ld +
-                    min(32 * (kt0 + kk * ks) + 8 * g, K - 8));
-                x[kk][mt][0] = p[0];
-                x[kk][mt][1] = p[1];
-            }
+                                                         min(32 * (kt0 + kk * ks) + 8 * g, K - 8));
     }
 };
 
@@ -347,7 +324,7 @@ __global__ __launch_bounds__(64 * kWaves) void g1_kernel(StepArgs s, LayerWeight
     BPre<1, KW> bw;
     bw.load(L.w_dq_dkv, s.zeros, nt, 1, KT, wave, kWaves, lane);
     APre16<KW, 1> a;
-    a.load(s.xw + (long long)row0 * m.d_pad, m.d_pad, s.B - row0, KT, wave, kWaves, lane);
+    a.load(s.xw + (long long)row0 * m.d_pad, m.d_pad, s.B - row0, m.d_pad, wave, kWaves, lane);
     // column c of cq (c < q_rank counts in its norm) or of [latent | key] (c < kv_rank)
     const bool kv = nt >= q_tiles;
     const int c = 16 * (kv ? nt - q_tiles : nt) + n, norm_cols = kv ? m.kv_rank : m.q_rank;
@@ -501,7 +478,7 @@ __global__ __launch_bounds__(64 * kG2Waves) void g2_kernel(StepArgs s, LayerWeig
     BPre<1, KW> bw;
     bw.load(L.w_q, s.zeros, T, 1, KTQ, 0, 1, lane);
     APre16<KW, 1> a;
-    a.load(s.cqw + (long long)row0 * m.q_pad, m.q_pad, s.B - row0, KTQ, 0, 1, lane);
+    a.load(s.cqw + (long long)row0 * m.q_pad, m.q_pad, s.B - row0, m.q_pad, 0, 1, lane);
     float2 cs[4];
     const int rhalf = m.rope / 2, j2 = min((16 * max(t - m.kv_pad / 16, 0) + n) / 2, rhalf - 1);
 #pragma unroll
@@ -761,11 +738,10 @@ __global__ __launch_bounds__(64 * kWaves) void g4_kernel(StepArgs s, LayerWeight
     const int KT = m.ctx_pad / 32;
     splitk_residual<KW>(
         [&](floatx4(&acc)[1][1], const BPre<1, KW>& bw, int kt0, int lane) {
-            AHalf32<KW, 1> a;
+            APre16<KW, 1> a;
             a.load(s.ctx + (long long)row0 * ctx_w, ctx_w, s.B - row0, ctx_w, kt0, kWaves, lane);
             operands_issued();
-            mma_steps(acc, bw,
-                      [&](int kk, int mt) { return to_half8(a.x[kk][mt][0], a.x[kk][mt][1]); });
+            mma_steps(acc, bw, [&](int kk, int mt) { return a.x[kk][mt]; });
         },
         L.w_out, s.zeros, KT, m.d_model, s.x, L.ffn_norm, s.res, s.resw, s.ss_res, m.d_pad / 16, m.d_pad,
         row0, s.B, [&]() {
@@ -794,7 +770,7 @@ __global__ __launch_bounds__(64 * kWaves) void g6_kernel(StepArgs s, LayerWeight
     splitk_residual<KW>(
         [&](floatx4(&acc)[1][1], const BPre<1, KW>& bw, int kt0, int lane) {
             APre16<KW, 1> a;
-            a.load(s.u + (long long)row0 * m.ff_pad, m.ff_pad, s.B - row0, KT, kt0, kWaves, lane);
+            a.load(s.u + (long long)row0 * m.ff_pad, m.ff_pad, s.B - row0, m.ff_pad, kt0, kWaves, lane);
             operands_issued();
             mma_steps(acc, bw, [&](int kk, int mt) { return a.x[kk][mt]; });
         },
@@ -857,7 +833,7 @@ __global__ __launch_bounds__(64 * kWaves) void g5_kernel(StepArgs s, LayerWeight
     BPre<2, KW> bw;
     bw.load(L.w_gate_up, s.zeros, 2 * p, 2, KT, wave, kWaves, lane);
     APre16<KW, 1> a;
-    a.load(s.resw + (long long)row0 * m.d_pad, m.d_pad, s.B - row0, KT, wave, kWaves, lane);
+    a.load(s.resw + (long long)row0 * m.d_pad, m.d_pad, s.B - row0, m.d_pad, wave, kWaves, lane);
     operands_issued();
     floatx4 acc[1][2];
     zero(acc);
@@ -930,7 +906,7 @@ __global__ __launch_bounds__(64 * kWaves) void g7_kernel(StepArgs s) {
     BPre<NTW, KW> bw;
     bw.load(s.embed, s.zeros, nt0 + ng * NTW, min(NTW, n_tiles - nt0 - ng * NTW), KT, kg, kG7KG, lane);
     APre16<KW, 4> a;
-    a.load(s.xw + (long long)row0 * m.d_pad, m.d_pad, s.B - row0, KT, kg, kG7KG, lane);
+    a.load(s.xw + (long long)row0 * m.d_pad, m.d_pad, s.B - row0, m.d_pad, kg, kG7KG, lane);
     operands_issued();
     floatx4 acc[4][NTW];
     zero(acc);

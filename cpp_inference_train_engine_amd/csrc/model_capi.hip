@@ -137,10 +137,10 @@ struct Model {
     const uint16_t* embed = nullptr;
     const float* final_norm = nullptr;
     const float* rope_tab = nullptr;
-    float *x, *res, *ctx, *logits, *arg_v;
+    float *x, *res, *logits, *arg_v;
     float *ss_x, *ss_res, *ss_cq, *ss_kv, *ckv;
     float2* rope_rows;
-    uint16_t *xw, *resw, *u, *q_latent, *q_rope, *cqw;
+    uint16_t *xw, *resw, *u, *q_latent, *q_rope, *cqw, *ctx;
     uint16_t* zeros = nullptr;  // 512 zero words
     int32_t* arg_c;
     uint32_t* ban_bits = nullptr;  // [ceil(vocab/32)] banned token ids, allocated on first use
@@ -394,7 +394,7 @@ int model_forward(Model* M, hipStream_t st, int rows, const int32_t* tokens,
     a.info = md.info;
     a.q_latent = M->q_latent;
     a.q_rope = M->q_rope;
-    a.out = M->ctx;
+    a.out16 = M->ctx;
     a.lse = nullptr;
     decode_workspace_layout(workspace, md.max_work, m.H, m.kv_rank, a);
     PrefillArgs pa{};
@@ -412,7 +412,7 @@ int model_forward(Model* M, hipStream_t st, int rows, const int32_t* tokens,
     pa.info = md.info;
     pa.q_latent = M->q_latent;
     pa.q_rope = M->q_rope;
-    pa.out = M->ctx;
+    pa.out16 = M->ctx;
     pa.lse = nullptr;
     const bool generic = (reinterpret_cast<uintptr_t>(workspace) & 15) != 0;
     a.fused_merge = (md.flags & MLA_DECODE_FUSED_MERGE) && decode_fuses_merge(a, generic);

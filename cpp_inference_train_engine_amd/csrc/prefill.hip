@@ -390,7 +390,7 @@ void prefill_page_kernel(PrefillArgs a) {
     const float inv = L > 0.0f ? 1.0f / L : 0.0f;
 #pragma unroll
     for (int gg = 0; gg < 4; ++gg)
-        *reinterpret_cast<floatx4*>(a.out + fr * KV + 16 * rt + 4 * gg) = o[gg] * inv;
+        store_row<false>(a.out, a.out16, fr * KV + 16 * rt + 4 * gg, o[gg] * inv);
     if (a.lse && rt == 0)
         a.lse[fr] = (M + __log2f(L)) * kLn2;
 }
@@ -493,7 +493,7 @@ __global__ __launch_bounds__(kPgThreads) void prefill_generic_kernel(PrefillArgs
     for (int k = 0; k < kPgMaxAcc; ++k) {
         const int r = tid + k * kPgThreads;
         if (r < KV)
-            a.out[fr * KV + r] = acc[k] * inv;
+            store_row(a.out, a.out16, fr * KV + r, acc[k] * inv);
     }
     if (a.lse && tid == 0)
         a.lse[fr] = (m_run + __log2f(l_run)) * kLn2;
