@@ -349,7 +349,7 @@ __global__ __launch_bounds__(64 * kTileWaves) __attribute__((amdgpu_waves_per_eu
             }
             if (ns == 1) {
                 const float inv = L > 0.0f ? 1.0f / L : 0.0f;
-                store_row<false>(a.out, a.out16, (f0 + row) * KV + c, o * inv);
+                store_row<false, kRowAny>(a, (f0 + row) / H, (int)((f0 + row) % H), c, o * inv);
                 if (a.lse && c == 0)
                     a.lse[f0 + row] = (M + __log2f(L)) * kLn2;
             } else if constexpr (!PREFILL) {

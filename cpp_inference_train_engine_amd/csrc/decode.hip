@@ -111,7 +111,7 @@ __device__ __forceinline__ void raise_status(const DecodeArgs& a, int bit) {
     __hip_atomic_fetch_or(a.status, bit, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
-template <int KV, int THREADS>
+template <int KV, int THREADS, int OUT>
 __device__ __forceinline__ void fused_merge_tail(const DecodeArgs& a, int s, int row, int ns,
                                                  long long first) {
     __shared__ int s_last;
@@ -157,7 +157,7 @@ __device__ __forceinline__ void fused_merge_tail(const DecodeArgs& a, int s, int
             }
         }
         const float inv = L > 0.0f ? 1.0f / L : 0.0f;
-        store_row<true>(a.out, a.out16, ((long long)row * a.H + h) * KV + c, O * inv);
+        store_row<true, OUT>(a, row, h, c, O * inv);
         if (a.lse && c == 0)
             a.lse[(long long)row * a.H + h] = (M + __log2f(L)) * kLn2;
     }
@@ -167,7 +167,7 @@ __device__ __forceinline__ void fused_merge_tail(const DecodeArgs& a, int s, int
 // session's items ran on several XCDs, so they do not merge.  Each leaves its partial (as
 // the two-launch path does: mla_decode_merge completes the rows), the first item sets the
 // session's rows to NaN so that no stale row passes for a result, and the call is flagged.
-template <int KV, int THREADS>
+template <int KV, int THREADS, int OUT>
 __device__ __forceinline__ void unplaced_tail(const DecodeArgs& a, int row, bool first_item) {
     const int tid = threadIdx.x;
     if (tid == 0)
@@ -176,7 +176,7 @@ __device__ __forceinline__ void unplaced_tail(const DecodeArgs& a, int row, bool
         return;
     const float nan = __builtin_nanf("");
     for (int e = tid; e < a.H * KV; e += THREADS)
-        store_row(a.out, a.out16, (long long)row * a.H * KV + e, nan);
+        store_row<false, OUT>(a, row, e / KV, e % KV, nan);
     if (a.lse)
         for (int h = tid; h < a.H; h += THREADS)
             a.lse[(long long)row * a.H + h] = nan;
@@ -210,7 +210,7 @@ __device__ __forceinline__ int item_split_index(int kl, int p_begin, int p_end, 
 // device-scope partial stores and loads because the items run on different XCDs,
 // whose L2s do not see each other's writes; measured on config 3 that tail costs
 // 4-8 us against 2-3 us for the separate merge launch.)
-template <typename T, int KV, int RP, int PS, int WAVES, int PPW, bool FUSED>
+template <typename T, int KV, int RP, int PS, int WAVES, int PPW, bool FUSED, int OUT>
 __global__ __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(PPW == 1 ? 3 : PPW == 2 ? 2 : 1, 8)))
 void decode_page_kernel(DecodeArgs a) {
     static_assert(KV % 32 == 0 && RP % 8 == 0 && RP <= 32 && PS % 32 == 0, "tile shape");
@@ -246,7 +246,6 @@ void decode_page_kernel(DecodeArgs a) {
     const float scale_log2 = a.scale_log2;
     // The XCD count the metadata was placed for (the fused merge's premise, checked at the end).
     const int placed_n = FUSED ? a.info[kInfoPlacement] : 0;
-
     asm volatile("" ::"s"(pid[0]), "s"(H), "s"(npool), "s"(pool), "s"(scale_log2), "s"(placed_n));
     const int s = d[0];
     if (s < 0 || d[7] != 1)
@@ -457,7 +456,7 @@ void decode_page_kernel(DecodeArgs a) {
         // 0.3 us less per config-3 launch than plain ones).
         if (ns == 1) {
             const float inv = lh > 0.0f ? 1.0f / lh : 0.0f;
-            store_row<true>(a.out, a.out16, ((long long)row * a.H + h) * KV + c, o * inv);
+            store_row<true, OUT>(a, row, h, c, o * inv);
             if (a.lse && c == 0)
                 a.lse[(long long)row * a.H + h] = (mh + __log2f(lh)) * kLn2;
         } else if constexpr (FUSED) {  // plain stores: the partials stay in this XCD's L2
@@ -479,9 +478,9 @@ void decode_page_kernel(DecodeArgs a) {
         if (ns > 1) {  // the session's first partial slot: this item's, less its split index
             const int sp = item_split_index(kl, p_begin, p_end, ns, PS);
             if (placed_n == a.xcd_n)
-                fused_merge_tail<KV, THREADS>(a, s, row, ns, slot - sp);
+                fused_merge_tail<KV, THREADS, OUT>(a, s, row, ns, slot - sp);
             else
-                unplaced_tail<KV, THREADS>(a, row, sp == 0);
+                unplaced_tail<KV, THREADS, OUT>(a, row, sp == 0);
         }
 }
 
@@ -590,7 +589,7 @@ __global__ __launch_bounds__(kGenThreads) void decode_generic_kernel(DecodeArgs 
             for (int k = 0; k < kGenMaxAcc; ++k) {
                 const int r = tid + k * kGenThreads;
                 if (r < KV)
-                    store_row(a.out, a.out16, ((long long)row * a.H + h) * KV + r, acc[k] * inv);
+                    store_row<false, kRowAny>(a, row, h, r, acc[k] * inv);
             }
             if (a.lse && tid == 0)
                 a.lse[(long long)row * a.H + h] = (m_run + __log2f(l_run)) * kLn2;
@@ -697,11 +696,10 @@ __global__ __launch_bounds__(kMergeElems* G) void merge_kernel(DecodeArgs a) {
     for (int q = 1; q < G; ++q)
         fold1(sm_m[q][t], sm_l[q][t], sm_o[q][t]);
     const float inv = L > 0.0f ? 1.0f / L : 0.0f;
-    const long long at = ((long long)row * H + h) * KV + c;
     if constexpr (V == 4)
-        store_row<false>(a.out, a.out16, at, O * inv);
+        store_row<false, kRowAny>(a, row, h, c, O * inv);
     else
-        store_row(a.out, a.out16, at, O[0] * inv);
+        store_row<false, kRowAny>(a, row, h, c, O[0] * inv);
     if (a.lse && c == 0)
         a.lse[(long long)row * H + h] = (M + __log2f(L)) * kLn2;
 }
@@ -717,17 +715,22 @@ __global__ __launch_bounds__(kMergeElems* G) void merge_kernel(DecodeArgs a) {
 constexpr int kPageWaves = MLA_DECODE_WAVES;
 constexpr int kPagesPerWave = MLA_DECODE_PPW;
 
+template <typename T, bool FUSED, int OUT>
+hipError_t launch_page_as(const DecodeArgs& a, int grid, hipStream_t stream) {
+    hipLaunchKernelGGL((decode_page_kernel<T, 128, 16, 64, kPageWaves, kPagesPerWave, FUSED, OUT>),
+                       dim3(grid), dim3(64 * kPageWaves), 0, stream, a);
+    return hipGetLastError();
+}
+
 template <typename T>
 hipError_t launch_page(const DecodeArgs& a, int grid, hipStream_t stream) {
-    if (a.kv_rank == 128 && a.rope_dim == 16 && a.page_size == 64 && a.fused_merge)
-        hipLaunchKernelGGL((decode_page_kernel<T, 128, 16, 64, kPageWaves, kPagesPerWave, true>),
-                           dim3(grid), dim3(64 * kPageWaves), 0, stream, a);
-    else if (a.kv_rank == 128 && a.rope_dim == 16 && a.page_size == 64)
-        hipLaunchKernelGGL((decode_page_kernel<T, 128, 16, 64, kPageWaves, kPagesPerWave, false>),
-                           dim3(grid), dim3(64 * kPageWaves), 0, stream, a);
-    else
+    if (a.kv_rank != 128 || a.rope_dim != 16 || a.page_size != 64)
         return hipErrorInvalidValue;
-    return hipGetLastError();
+    if (a.out16)
+        return a.fused_merge ? launch_page_as<T, true, kRowF16>(a, grid, stream)
+                             : launch_page_as<T, false, kRowF16>(a, grid, stream);
+    return a.fused_merge ? launch_page_as<T, true, kRowF32>(a, grid, stream)
+                         : launch_page_as<T, false, kRowF32>(a, grid, stream);
 }
 
 }  // namespace

@@ -175,28 +175,6 @@ __device__ __forceinline__ void copy_4blocks_to_lds_at(const void* base, uint32_
 }
 #pragma clang diagnostic pop
 
-// Four consecutive values (or one) of a final attention row at element i: fp32 to out, or, for
-// a caller whose next kernel rounds the row to fp16 anyway (the model's output projection),
-// rounded here to out16: the same bits in half the bytes.
-template <bool NT>
-__device__ __forceinline__ void store_row(float* out, uint16_t* out16, long long i, floatx4 v) {
-    typedef _Float16 half4 __attribute__((ext_vector_type(4)));
-    if (out16) {
-        const half4 h = {(_Float16)v[0], (_Float16)v[1], (_Float16)v[2], (_Float16)v[3]};
-        *reinterpret_cast<half4*>(out16 + i) = h;
-    } else if constexpr (NT) {
-        __builtin_nontemporal_store(v, reinterpret_cast<floatx4*>(out + i));
-    } else {
-        *reinterpret_cast<floatx4*>(out + i) = v;
-    }
-}
-__device__ __forceinline__ void store_row(float* out, uint16_t* out16, long long i, float v) {
-    if (out16)
-        out16[i] = F16::from_float(v);
-    else
-        out[i] = v;
-}
-
 // Orders this wave's LDS accesses: nothing before it moves after it, or after it before.
 __device__ __forceinline__ void wave_lds_fence() {
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
@@ -238,6 +216,44 @@ __host__ __device__ inline long long rope_word(bool tiled, int slot, int c, int 
         return base + (long long)slot * rope_dim + c;
     const int t = slot >> 4, n = slot & 15, ch = c >> 3, e = c & 7;
     return base + (long long)(t * (rope_dim >> 3) + ch) * 128 + n * 8 + e;
+}
+
+// ---- fp16 activations of the model step ------------------------------------------
+// Stored in MFMA-operand order, like the weights: the 16 rows x 32 columns of (row / 16,
+// col / 32) are 512 contiguous words, so that a wave's A-operand load reads 1 KB contiguously
+// (row-major it touched half of a cache line in each of 16 rows, 1 KB apart).  kt: 32-column
+// blocks of a row.  Rows row .. row + 3 (row % 4 == 0) of a column are 8 words apart.
+__host__ __device__ inline long long act_word(long long row, int col, int kt) {
+    return ((row >> 4) * kt + (col >> 5)) * 512 + (((col & 31) >> 3) * 16 + (int)(row & 15)) * 8 +
+           (col & 7);
+}
+
+// Columns c .. c + 3 (or c alone) of head h of a final attention row: fp32 to a.out, or, for the
+// model step, whose output projection rounds the row to fp16 anyway, rounded here to a.out16 (an
+// activation of H * kv_rank columns): the same bits in half the bytes.  OUT: kRowF32, kRowF16, or
+// kRowAny to choose by a.out16 (which costs the page kernels 0.2 us a call at their end).
+enum { kRowF32, kRowF16, kRowAny };
+template <bool NT, int OUT, typename Args>
+__device__ __forceinline__ void store_row(const Args& a, long long row, int h, int c, floatx4 v) {
+    typedef _Float16 half4 __attribute__((ext_vector_type(4)));
+    if (OUT == kRowF16 || (OUT == kRowAny && a.out16)) {
+        const half4 x = {(_Float16)v[0], (_Float16)v[1], (_Float16)v[2], (_Float16)v[3]};
+        *reinterpret_cast<half4*>(
+            a.out16 + act_word(row, h * a.kv_rank + c, (a.H * a.kv_rank + 31) >> 5)) = x;
+        return;
+    }
+    floatx4* p = reinterpret_cast<floatx4*>(a.out + (row * a.H + h) * a.kv_rank + c);
+    if constexpr (NT)
+        __builtin_nontemporal_store(v, p);
+    else
+        *p = v;
+}
+template <bool NT, int OUT, typename Args>
+__device__ __forceinline__ void store_row(const Args& a, long long row, int h, int c, float v) {
+    if (OUT == kRowF16 || (OUT == kRowAny && a.out16))
+        a.out16[act_word(row, h * a.kv_rank + c, (a.H * a.kv_rank + 31) >> 5)] = F16::from_float(v);
+    else
+        a.out[(row * a.H + h) * a.kv_rank + c] = v;
 }
 
 }  // namespace mla

@@ -57,8 +57,8 @@ struct DecodeArgs {
     const int32_t *cu_q, *page_table, *num_splits, *cu_splits, *work_desc, *work_pages, *info;
     const uint16_t *pages, *q_latent, *q_rope;
     float *out, *lse, *part_o, *part_ml;
-    // When not null, final rows go here as fp16 instead of to `out` (the model step; every
-    // kernel but decode_wide_kernel, whose shape no model has).
+    // When not null, final rows go here as an fp16 activation (act_word, mla_common.hpp) instead
+    // of to `out` (the model step; every kernel but decode_wide_kernel, whose shape no model has).
     uint16_t* out16;
     // Fused merge (decode_page_kernel only): the metadata was built XCD-placed, and the
     // last item of a split session to finish combines the session's partials itself.

@@ -59,11 +59,12 @@ struct StepArgs {
     float2* rope_rows;         // [m_pad x rope/2] the table rows of this step's positions
     // activations (rows padded to m_pad)
     float *x, *res;             // [m_pad x d_pad]
-    const uint16_t* ctx;        // [m_pad x H*kv_rank] fp16 attention rows
-    uint16_t *cqw;              // [m_pad x q_pad] fp16 cq o q_norm
+    // fp16 activations, tiled (act_word): ctx, cqw, xw, resw, u
+    const uint16_t* ctx;        // [m_pad x ctx_pad] attention rows
+    uint16_t *cqw;              // [m_pad x q_pad] cq o q_norm
     float* ckv;                 // [m_pad x kvw_pad] latent o kv_norm, then the key before RoPE
-    uint16_t *xw, *resw;        // fp16 x o (next norm weight), res o ffn_norm [m_pad x d_pad]
-    uint16_t *u;                // [m_pad x ff_pad] fp16
+    uint16_t *xw, *resw;        // x o (next norm weight), res o ffn_norm [m_pad x d_pad]
+    uint16_t *u;                // [m_pad x ff_pad]
     uint16_t *q_latent, *q_rope;  // [B x H x kv_rank], [B x H x rope] in the cache dtype
     float* logits;              // [B x vocab]
     float* arg_v;               // [B x parts] greedy partials

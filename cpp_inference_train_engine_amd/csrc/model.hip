@@ -154,20 +154,23 @@ struct BPre {
 };
 
 // Activation (A operand) registers: lane (g, n) needs rows 16mt + n (mt < MT) and
-// columns 32kt + 8g .. +7 of each of its k-steps.  Rows past `rows` (>= 1) repeat the last one:
-// their products are dropped, and the lanes that share its address add no traffic.
+// columns 32kt + 8g .. +7 of each of its k-steps of the activation rows from X on (a whole
+// 16-row tile's first word; KT 32-column blocks a row).  Rows past `rows` (>= 1) repeat the last
+// one: their products are dropped, and the lanes that share its address add no traffic.
 template <int KW, int MT>
-struct APre16 {  // fp16 rows of K % 8 == 0 columns (the weights of columns past K are 0)
+struct APre16 {
     V8 x[KW][MT];
-    __device__ __forceinline__ void load(const uint16_t* X, int ld, int rows, int K, int kt0,
-                                         int ks, int lane) {
+    __device__ __forceinline__ void load(const uint16_t* X, int rows, int KT, int kt0, int ks,
+                                         int lane) {
         const int g = lane >> 4, n = lane & 15;
 #pragma unroll
-        for (int kk = 0; kk < KW; ++kk)
+        for (int mt = 0; mt < MT; ++mt) {
+            const int r = min(16 * mt + n, rows - 1);
+            const uint16_t* p = X + act_word(r, 8 * g, KT);
 #pragma unroll
-            for (int mt = 0; mt < MT; ++mt)
-                x[kk][mt] = *reinterpret_cast<const V8*>(X + (long long)min(16 * mt + n, rows - 1) * ld +
-                                                         min(32 * (kt0 + kk * ks) + 8 * g, K - 8));
+            for (int kk = 0; kk < KW; ++kk)
+                x[kk][mt] = *reinterpret_cast<const V8*>(p + min(kt0 + kk * ks, KT - 1) * 512);
+        }
     }
 };
 
@@ -290,7 +293,7 @@ __global__ __launch_bounds__(256) void embed_kernel(StepArgs s, const float* nor
         }
         if (c < m.d_pad) {
             s.x[(long long)b * m.d_pad + c] = v;
-            s.xw[(long long)b * m.d_pad + c] = F16::from_float(v * w);
+            s.xw[act_word(b, c, KT)] = F16::from_float(v * w);
         }
         const float q = sum16(v * v);
         if ((threadIdx.x & 15) == 0 && c < m.d_pad)
@@ -324,7 +327,7 @@ __global__ __launch_bounds__(64 * kWaves) void g1_kernel(StepArgs s, LayerWeight
     BPre<1, KW> bw;
     bw.load(L.w_dq_dkv, s.zeros, nt, 1, KT, wave, kWaves, lane);
     APre16<KW, 1> a;
-    a.load(s.xw + (long long)row0 * m.d_pad, m.d_pad, s.B - row0, m.d_pad, wave, kWaves, lane);
+    a.load(s.xw + (long long)row0 * m.d_pad, s.B - row0, KT, wave, kWaves, lane);
     // column c of cq (c < q_rank counts in its norm) or of [latent | key] (c < kv_rank)
     const bool kv = nt >= q_tiles;
     const int c = 16 * (kv ? nt - q_tiles : nt) + n, norm_cols = kv ? m.kv_rank : m.q_rank;
@@ -355,7 +358,8 @@ __global__ __launch_bounds__(64 * kWaves) void g1_kernel(StepArgs s, LayerWeight
             if (kv)
                 s.ckv[(long long)row * m.kvw_pad + c] = y[i] * (c < m.kv_rank ? wn : 1.0f);
             else
-                s.cqw[(long long)row * m.q_pad + c] = F16::from_float(c < m.q_rank ? y[i] * wn : 0.0f);
+                s.cqw[act_word(row, c, m.q_pad / 32)] =
+                    F16::from_float(c < m.q_rank ? y[i] * wn : 0.0f);
         }
     }
     if (kv)
@@ -478,7 +482,7 @@ __global__ __launch_bounds__(64 * kG2Waves) void g2_kernel(StepArgs s, LayerWeig
     BPre<1, KW> bw;
     bw.load(L.w_q, s.zeros, T, 1, KTQ, 0, 1, lane);
     APre16<KW, 1> a;
-    a.load(s.cqw + (long long)row0 * m.q_pad, m.q_pad, s.B - row0, m.q_pad, 0, 1, lane);
+    a.load(s.cqw + (long long)row0 * m.q_pad, s.B - row0, KTQ, 0, 1, lane);
     float2 cs[4];
     const int rhalf = m.rope / 2, j2 = min((16 * max(t - m.kv_pad / 16, 0) + n) / 2, rhalf - 1);
 #pragma unroll
@@ -574,7 +578,7 @@ __global__ __launch_bounds__(64 * kWaves) void qkv_kernel(StepArgs s, LayerWeigh
 #pragma unroll
     for (int j = 0; j < NT; ++j)
         acc[j] = floatx4{0, 0, 0, 0};
-    const uint16_t* xw = s.xw + (long long)min(row0 + n, s.B - 1) * m.d_pad;
+    const uint16_t* xw = s.xw + act_word(min(row0 + n, s.B - 1), 8 * g, KT);
     // Head workgroups also prefetch their w_q tiles (used after the reduction; wave w owns
     // tiles w and w + 8 of the head's kv_tiles latent and then rope tiles) and the RoPE
     // rotations of the rows and columns they hold of a rope tile.
@@ -587,7 +591,7 @@ __global__ __launch_bounds__(64 * kWaves) void qkv_kernel(StepArgs s, LayerWeigh
 #pragma unroll
         for (int kk = 0; kk < 2; ++kk) {
             const int kt = wave + kWaves * (2 * c + kk);
-            a[kk] = *reinterpret_cast<const V8*>(xw + 32 * min(kt, KT - 1) + 8 * g);
+            a[kk] = *reinterpret_cast<const V8*>(xw + min(kt, KT - 1) * 512);
 #pragma unroll
             for (int j = 0; j < NT; ++j)
                 b[kk][j] = load_w(L.w_dq_dkv, s.zeros, nt0 + min(j, ntv - 1), kt, KT, lane);
@@ -724,7 +728,7 @@ __device__ __forceinline__ void splitk_residual(ALoad&& aload, const uint16_t* w
         y[i] = col < N ? v[0][i] + res[i] : 0.0f;
         if (row < B && col < N) {
             out[row * ld + col] = y[i];
-            outw[row * ld + col] = F16::from_float(y[i] * wn);
+            outw[act_word(row, col, ld >> 5)] = F16::from_float(y[i] * wn);
         }
     }
     write_ss(y, col < N, ss, n_tiles, nt, row0, B);
@@ -734,12 +738,12 @@ template <int KW>
 __global__ __launch_bounds__(64 * kWaves) void g4_kernel(StepArgs s, LayerWeights L) {
     __shared__ __attribute__((aligned(16))) uint16_t pf_scratch[512];
     const ModelDims& m = s.dims;
-    const int row0 = blockIdx.y * 16, ctx_w = m.H * m.kv_rank;  // attention rows: H*kv_rank
+    const int row0 = blockIdx.y * 16;
     const int KT = m.ctx_pad / 32;
     splitk_residual<KW>(
         [&](floatx4(&acc)[1][1], const BPre<1, KW>& bw, int kt0, int lane) {
             APre16<KW, 1> a;
-            a.load(s.ctx + (long long)row0 * ctx_w, ctx_w, s.B - row0, ctx_w, kt0, kWaves, lane);
+            a.load(s.ctx + (long long)row0 * m.ctx_pad, s.B - row0, KT, kt0, kWaves, lane);
             operands_issued();
             mma_steps(acc, bw, [&](int kk, int mt) { return a.x[kk][mt]; });
         },
@@ -770,7 +774,7 @@ __global__ __launch_bounds__(64 * kWaves) void g6_kernel(StepArgs s, LayerWeight
     splitk_residual<KW>(
         [&](floatx4(&acc)[1][1], const BPre<1, KW>& bw, int kt0, int lane) {
             APre16<KW, 1> a;
-            a.load(s.u + (long long)row0 * m.ff_pad, m.ff_pad, s.B - row0, m.ff_pad, kt0, kWaves, lane);
+            a.load(s.u + (long long)row0 * m.ff_pad, s.B - row0, KT, kt0, kWaves, lane);
             operands_issued();
             mma_steps(acc, bw, [&](int kk, int mt) { return a.x[kk][mt]; });
         },
@@ -833,7 +837,7 @@ __global__ __launch_bounds__(64 * kWaves) void g5_kernel(StepArgs s, LayerWeight
     BPre<2, KW> bw;
     bw.load(L.w_gate_up, s.zeros, 2 * p, 2, KT, wave, kWaves, lane);
     APre16<KW, 1> a;
-    a.load(s.resw + (long long)row0 * m.d_pad, m.d_pad, s.B - row0, m.d_pad, wave, kWaves, lane);
+    a.load(s.resw + (long long)row0 * m.d_pad, s.B - row0, KT, wave, kWaves, lane);
     operands_issued();
     floatx4 acc[1][2];
     zero(acc);
@@ -850,7 +854,7 @@ __global__ __launch_bounds__(64 * kWaves) void g5_kernel(StepArgs s, LayerWeight
             const int row = row0 + 4 * g + i;
             const float inv = inv_s[4 * g + i];
             if (row < s.B)
-                s.u[(long long)row * m.ff_pad + col] =
+                s.u[act_word(row, col, m.ff_pad / 32)] =
                     F16::from_float(silu_stable(v[0][i] * inv) * (v[1][i] * inv));
         }
 }
@@ -906,7 +910,7 @@ __global__ __launch_bounds__(64 * kWaves) void g7_kernel(StepArgs s) {
     BPre<NTW, KW> bw;
     bw.load(s.embed, s.zeros, nt0 + ng * NTW, min(NTW, n_tiles - nt0 - ng * NTW), KT, kg, kG7KG, lane);
     APre16<KW, 4> a;
-    a.load(s.xw + (long long)row0 * m.d_pad, m.d_pad, s.B - row0, m.d_pad, kg, kG7KG, lane);
+    a.load(s.xw + (long long)row0 * m.d_pad, s.B - row0, KT, kg, kG7KG, lane);
     operands_issued();
     floatx4 acc[4][NTW];
     zero(acc);
@@ -961,7 +965,8 @@ __global__ __launch_bounds__(256) void gather_last_kernel(StepArgs s, int B, con
     const int b = blockIdx.x, d_tiles = m.d_pad / 16;
     const int src = b < B ? cu_q[b + 1] - 1 : -1;
     for (int c = threadIdx.x; c < m.d_pad; c += 256)
-        xw_out[(long long)b * m.d_pad + c] = src >= 0 ? s.xw[(long long)src * m.d_pad + c] : 0;
+        xw_out[act_word(b, c, m.d_pad / 32)] =
+            src >= 0 ? s.xw[act_word(src, c, m.d_pad / 32)] : 0;
     for (int c = threadIdx.x; c < d_tiles; c += 256)
         ss_out[(long long)b * d_tiles + c] = src >= 0 ? s.ss_x[(long long)src * d_tiles + c] : 0.0f;
 }

@@ -522,7 +522,7 @@ int mla_model_create(const mla_model_config* config, const float* params, int ma
     if (e == hipSuccess) e = M->alloc(M->xw, rows * m.d_pad);
     if (e == hipSuccess) e = M->alloc(M->resw, rows * m.d_pad);
     if (e == hipSuccess) e = M->alloc(M->rope_rows, rows * (size_t)(c.head_dim_rope / 2));
-    if (e == hipSuccess) e = M->alloc(M->ctx, rows * (size_t)H * kv);
+    if (e == hipSuccess) e = M->alloc(M->ctx, rows * (size_t)m.ctx_pad);
     if (e == hipSuccess) e = M->alloc(M->u, rows * m.ff_pad);
     if (e == hipSuccess) e = M->alloc(M->q_latent, (size_t)max_batch * H * kv);
     if (e == hipSuccess) e = M->alloc(M->q_rope, (size_t)max_batch * H * c.head_dim_rope);

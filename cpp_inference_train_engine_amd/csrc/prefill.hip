@@ -65,7 +65,7 @@ constexpr int kPfMaxIds = 512;        // page ids staged in LDS (later pages: pa
 // measurement: 0 conflict cycles with 12, 168.6 M per config-5 dispatch as stored).
 constexpr int kPfRot = 12;
 
-template <typename T, int KV, int RP, int PS>
+template <typename T, int KV, int RP, int PS, int OUT>
 __global__ __launch_bounds__(64 * kPfWaves) __attribute__((amdgpu_waves_per_eu(2, 8)))
 void prefill_page_kernel(PrefillArgs a) {
     static_assert(KV % 32 == 0 && RP % 8 == 0 && RP <= 32 && PS % kPfUnit == 0, "tile shape");
@@ -390,7 +390,10 @@ void prefill_page_kernel(PrefillArgs a) {
     const float inv = L > 0.0f ? 1.0f / L : 0.0f;
 #pragma unroll
     for (int gg = 0; gg < 4; ++gg)
-        store_row<false>(a.out, a.out16, fr * KV + 16 * rt + 4 * gg, o[gg] * inv);
+        if constexpr (OUT == kRowF32)
+            *reinterpret_cast<floatx4*>(a.out + fr * KV + 16 * rt + 4 * gg) = o[gg] * inv;
+        else
+            store_row<false, OUT>(a, q0 + row / H, row % H, 16 * rt + 4 * gg, o[gg] * inv);
     if (a.lse && rt == 0)
         a.lse[fr] = (M + __log2f(L)) * kLn2;
 }
@@ -493,7 +496,7 @@ __global__ __launch_bounds__(kPgThreads) void prefill_generic_kernel(PrefillArgs
     for (int k = 0; k < kPgMaxAcc; ++k) {
         const int r = tid + k * kPgThreads;
         if (r < KV)
-            store_row(a.out, a.out16, fr * KV + r, acc[k] * inv);
+            store_row<false, kRowAny>(a, q0 + i, h, r, acc[k] * inv);
     }
     if (a.lse && tid == 0)
         a.lse[fr] = (m_run + __log2f(l_run)) * kLn2;
@@ -503,8 +506,13 @@ template <typename T>
 hipError_t launch_prefill_page(const PrefillArgs& a, int max_q_len, hipStream_t stream) {
     constexpr int rows = kPfQT * 16;
     const long long gx = ((long long)max_q_len * a.H + rows - 1) / rows;
-    hipLaunchKernelGGL((prefill_page_kernel<T, 128, 16, 64>), dim3((unsigned)gx, a.B),
-                       dim3(64 * kPfWaves), 0, stream, a);
+    const dim3 grid((unsigned)gx, a.B);
+    if (a.out16)
+        hipLaunchKernelGGL((prefill_page_kernel<T, 128, 16, 64, kRowF16>), grid,
+                           dim3(64 * kPfWaves), 0, stream, a);
+    else
+        hipLaunchKernelGGL((prefill_page_kernel<T, 128, 16, 64, kRowF32>), grid,
+                           dim3(64 * kPfWaves), 0, stream, a);
     return hipGetLastError();
 }
 

@@ -45,7 +45,7 @@ def _steps(gpu, cfg, counts, page=16):
 @pytest.mark.gpu
 @pytest.mark.parametrize("cfg", [dict(MLA36M, n_layers=2), TINY, ODD, WIDE],
                          ids=["mla36m", "tiny", "odd", "wide"])
-@pytest.mark.parametrize("counts", [(3, 16, 17, 70)])
+@pytest.mark.parametrize("counts", [(3, 16, 17, 70), (13, 191, 192, 260)])
 def test_row_count_does_not_change_a_bit(gpu, cfg, counts):
     _say(f"row routes d={cfg['d_model']} {counts}")
     got = _steps(gpu, cfg, counts)
