@@ -329,7 +329,7 @@ int step(Engine* E, int n, const int* ids, const int* counts, const uint16_t* to
                                  hipMemcpyDeviceToHost, E->stream);
         if (err == hipSuccess)
             err = hipStreamSynchronize(E->stream);
-        E->meta_launches += 1;
+        E->meta_launches += metadata_launches(n, E->max_pages);
         E->copies += 2 + placed + !all_rows + (logits != nullptr);
         E->host_waits += 1;
         return gpu_status(err, fn);

@@ -1,9 +1,10 @@
 // (a) Ragged-batch metadata and (b) paged latent append, gfx950.
 //
-// The metadata build runs as ONE workgroup of 1024 threads: batches are at
-// most a few thousand sessions, so a single-block scan beats a multi-kernel
-// device-wide scan (no inter-block traffic, one launch).  All arithmetic is
-// int32/int64 and bit-exact with the CPU builder in the oracle.
+// Batches whose page table is small are built by ONE workgroup of 1024 threads in one launch
+// (build_metadata_lds_kernel).  Larger ones take two: plan_metadata_kernel, one workgroup that
+// validates and scans, and fill_metadata_kernel, one workgroup per session that writes its part
+// of the table, the work list and the slots.  All arithmetic is int32/int64 and bit-exact with
+// the CPU builder in the oracle.
 #include "mla_common.hpp"
 #include "mla_internal.hpp"
 
@@ -18,34 +19,48 @@ namespace {
 constexpr int kMetaThreads = 1024;
 constexpr int kMetaWaves = kMetaThreads / 64;
 
-// Inclusive block scan of three int64 values; returns the chunk totals in tot[].
-__device__ void block_scan3(long long v[3], long long tot[3], long long* lds) {
+// One DPP move of a 64-bit value (both halves with the same control); lanes the
+// control gives no source, and rows outside row_mask, receive 0.
+template <int CTRL, int ROW_MASK>
+__device__ __forceinline__ long long dpp64(long long v) {
+    const int lo = __builtin_amdgcn_update_dpp(0, (int)(uint32_t)v, CTRL, ROW_MASK, 0xf, true);
+    const int hi = __builtin_amdgcn_update_dpp(0, (int)(uint32_t)(v >> 32), CTRL, ROW_MASK, 0xf,
+                                               true);
+    return (long long)(((uint64_t)(uint32_t)hi << 32) | (uint32_t)lo);
+}
+
+// Inclusive scan over the 64 lanes of a wave on DPP moves (no LDS round trips): shifts
+// of 1, 2, 4, 8 lanes within each row of 16, then lane 15 of each row broadcast into
+// the next row (rows 1, 3) and lane 31 into the upper half (rows 2, 3).
+__device__ __forceinline__ long long wave_scan_incl(long long v) {
+    v += dpp64<0x111, 0xf>(v);  // row_shr:1
+    v += dpp64<0x112, 0xf>(v);  // row_shr:2
+    v += dpp64<0x114, 0xf>(v);  // row_shr:4
+    v += dpp64<0x118, 0xf>(v);  // row_shr:8
+    v += dpp64<0x142, 0xa>(v);  // row_bcast:15
+    v += dpp64<0x143, 0xc>(v);  // row_bcast:31
+    return v;
+}
+
+// Inclusive block scan of N int64 values; returns the chunk totals in tot[].
+template <int N>
+__device__ void block_scan(long long (&v)[N], long long (&tot)[N], long long* lds) {
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
 #pragma unroll
-    for (int k = 0; k < 3; ++k)
-        for (int off = 1; off < 64; off <<= 1) {
-            const long long up = __shfl_up(v[k], off, 64);
-            if (lane >= off)
-                v[k] += up;
-        }
-    if (lane == 63)
-        for (int k = 0; k < 3; ++k)
+    for (int k = 0; k < N; ++k) {
+        v[k] = wave_scan_incl(v[k]);
+        if (lane == 63)
             lds[k * kMetaWaves + wave] = v[k];
-    __syncthreads();
-    if (wave == 0) {
-        for (int k = 0; k < 3; ++k) {
-            long long x = lane < kMetaWaves ? lds[k * kMetaWaves + lane] : 0;
-            for (int off = 1; off < kMetaWaves; off <<= 1) {
-                const long long up = __shfl_up(x, off, 64);
-                if (lane >= off)
-                    x += up;
-            }
-            if (lane < kMetaWaves)
-                lds[k * kMetaWaves + lane] = x;
-        }
     }
     __syncthreads();
-    for (int k = 0; k < 3; ++k) {
+    if (wave < N) {
+        const long long x = wave_scan_incl(lane < kMetaWaves ? lds[wave * kMetaWaves + lane] : 0);
+        if (lane < kMetaWaves)
+            lds[wave * kMetaWaves + lane] = x;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < N; ++k) {
         if (wave > 0)
             v[k] += lds[k * kMetaWaves + wave - 1];
         tot[k] = lds[k * kMetaWaves + kMetaWaves - 1];
@@ -66,19 +81,16 @@ __device__ int upper_index(const int32_t* a, int n, long long x) {
     return lo;
 }
 
-// For batches up to kMetaLdsCap sessions the per-session inputs and prefix arrays live
-// in LDS, and so does the padded page table when it has at most kMetaPtCap entries, so
-// the build waits on global memory twice (the session inputs, then the page ids) and
-// every later lookup and binary search reads LDS.
-constexpr int kMetaLdsCap = 4096;
-constexpr int kMetaPtCap = 16384;
-constexpr int kMetaUnroll = 16;  // page-table entries whose loads a thread issues together
+constexpr int kMetaLdsCap = 4096;  // sessions of build_metadata_lds_kernel
 
+__device__ void write_error_info(const MetadataArgs& a, int session) {
+    if (threadIdx.x < kInfoInts)
+        a.info[threadIdx.x] = threadIdx.x == 0 ? -1 : threadIdx.x == 1 ? session : 0;
+}
 __device__ void write_error(const MetadataArgs& a, int session) {
     for (int w = threadIdx.x; w < a.max_work; w += kMetaThreads)
         a.work_desc[(long long)w * kWorkDescInts] = -1;
-    if (threadIdx.x < kInfoInts)
-        a.info[threadIdx.x] = threadIdx.x == 0 ? -1 : threadIdx.x == 1 ? session : 0;
+    write_error_info(a, session);
 }
 
 // ceil(x / d) for x >= 0 and d >= 1, in 32-bit arithmetic when both are below 2^31.
@@ -99,15 +111,14 @@ __device__ __forceinline__ long long ceil_div_nn(long long x, long long d) {
 // XCD x lands in slot x + n * (k + sp), k the items of that XCD's sessions of rounds < q.
 // There are ceil(B / n) rounds (up to 256 when n = 1); wave x takes them 64 at a time,
 // one lane per round, carrying the running item count from pass to pass.
-__device__ long long wave_scan_incl(long long v);  // inclusive sum over the wave's lanes
 
 struct Placement {
     int32_t weight[kPlaceMaxSessions], order[kPlaceMaxSessions], bin[kPlaceMaxSessions],
         k0[kPlaceMaxSessions], cnt[kPlaceMaxXcds];
 };
 
-// All threads call it (B <= kPlaceMaxSessions, 1 <= n <= kPlaceMaxXcds <= kMetaWaves); q(b),
-// ctx(b) and cus(b) read the session inputs and the work-item prefix.  Ends with a barrier.
+// All threads call it (B <= kPlaceMaxSessions, 1 <= n <= kPlaceMaxXcds); q(b), ctx(b) and
+// cus(b) read the session inputs and the work-item prefix.  Ends with a barrier.
 template <typename Q, typename C, typename S>
 __device__ void place_sessions(int B, int n, int page_size, Q q, C ctx, S cus, Placement& p) {
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -135,8 +146,7 @@ __device__ void place_sessions(int B, int n, int page_size, Q q, C ctx, S cus, P
             p.order[r] = b;
     }
     __syncthreads();
-    if (wave < n) {  // wave x: lane l holds XCD x's session of round q0 + l
-        const int x = wave;
+    for (int x = wave; x < n; x += kMetaWaves) {  // lane l holds XCD x's session of round q0 + l
         long long carry = 0;  // items of XCD x's sessions of earlier passes
         for (int q0 = 0; q0 * n < B; q0 += 64) {
             const int qr = q0 + lane;
@@ -165,220 +175,206 @@ __device__ __forceinline__ long long placed_slots(const Placement& p, int n) {
     return (long long)m * n;
 }
 
-// L: the batch fits the LDS mirrors (B <= kMetaLdsCap); the compiler then reads them
-// with LDS instructions rather than flat loads.
-template <bool L>
-__global__ __launch_bounds__(kMetaThreads) void build_metadata_kernel(MetadataArgs a) {
-    constexpr int CAP = L ? kMetaLdsCap : 1, PT = L ? kMetaPtCap : 1;
+// ------------------------------------------------------------- larger batches ----
+// Work items of a session of kl keys with q new rows.
+__device__ __forceinline__ long long item_count(long long kl, long long q, long long page_size,
+                                                long long split) {
+    return q > 0 ? ceil_div_nn(ceil_div_nn(kl, page_size), split) : 0;
+}
+
+// One workgroup: page-id and length checks, cu_seqlens_q / k, num_splits, cu_splits and info.  On
+// an error info says so, and fill_metadata_kernel empties the work list.
+__global__ __launch_bounds__(kMetaThreads) void plan_metadata_kernel(MetadataArgs a) {
     __shared__ long long lds[3 * kMetaWaves];
-    __shared__ long long carry[3];
     __shared__ int err;
-    __shared__ int32_t s_cup[CAP + 1], s_cuq[CAP + 1], s_cus[CAP + 1];
-    __shared__ int32_t s_q[CAP], s_ctx[CAP], s_pt[PT];
-    const int tid = threadIdx.x;
-    constexpr bool in_lds = L;
-    const long long entries = (long long)a.B * a.max_pages;
-    const bool pt_lds = L && entries <= kMetaPtCap;
-    const int32_t* __restrict__ qlen = L ? s_q : a.q_len;
-    const int32_t* __restrict__ ctxl = L ? s_ctx : a.ctx_len;
-    const int32_t* cup = L ? s_cup : a.cu_pages;
-    const int32_t* cuq = L ? s_cuq : a.cu_seqlens_q;
-    const int32_t* cus = L ? s_cus : a.cu_splits;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     if (tid == 0) {
-        carry[0] = carry[1] = carry[2] = 0;
         err = INT_MAX;
-        a.cu_seqlens_q[0] = 0;
-        a.cu_seqlens_k[0] = 0;
-        a.cu_splits[0] = 0;
-        if (L) {
-            s_cuq[0] = 0;
-            s_cus[0] = 0;
-        }
+        a.cu_seqlens_q[0] = a.cu_seqlens_k[0] = a.cu_splits[0] = 0;
     }
-    if (in_lds)
-        for (int b = tid; b <= a.B; b += kMetaThreads) {
-            const int32_t cp = a.cu_pages[b];
-            const int32_t q = b < a.B ? a.q_len[b] : 0, c = b < a.B ? a.ctx_len[b] : 0;
-            s_cup[b] = cp;
-            if (b < a.B) {
-                s_q[b] = q;
-                s_ctx[b] = c;
-            }
-        }
     __syncthreads();
-    // Phase 1: padded page table and page-id validation (a session listing more than
-    // max_pages pages is invalid anyway and only its first max_pages ids are read), then
-    // cu_seqlens_q/k, validation and the total pages of sessions with queries.
-    const bool small = entries <= INT_MAX;  // 32-bit index arithmetic
-    for (long long e0 = tid; e0 < entries; e0 += (long long)kMetaThreads * kMetaUnroll) {
-        int32_t pid[kMetaUnroll];
-        int bs[kMetaUnroll], js[kMetaUnroll];
+    // Page ids: each wave checks the lists of its share of the sessions, 64 sessions at a time,
+    // as one flat run (consecutive lists are adjacent), kIds loads of a lane in flight.  Only when
+    // that finds a bad id, or a list is too long or negative (then only its first max_pages ids
+    // may be read), the group is walked session by session to name the first bad one.
+    constexpr int kIds = 16;
+    const int per_wave = (a.B + kMetaWaves - 1) / kMetaWaves;
+    const int b_end = min(a.B, (wave + 1) * per_wave);
+    for (int base = wave * per_wave; base < b_end; base += 64) {
+        const int mine = min(base + lane, a.B - 1), sessions = min(64, b_end - base);
+        const int my_first = a.cu_pages[mine], my_pages = a.cu_pages[mine + 1] - my_first;
+        bool walk = __ballot(my_pages < 0 || my_pages > a.max_pages) != 0;
+        if (!walk) {
+            const int lo = __builtin_amdgcn_readlane(my_first, 0);
+            const int hi = __builtin_amdgcn_readlane(my_first + my_pages, sessions - 1);
+            bool bad = false;
+            for (int e0 = lo; e0 < hi; e0 += 64 * kIds) {
+                int32_t id[kIds];
 #pragma unroll
-        for (int k = 0; k < kMetaUnroll; ++k) {
-            const long long e = e0 + (long long)k * kMetaThreads;
-            pid[k] = -1;
-            bs[k] = -1;
-            js[k] = 0;
-            if (e < entries) {
-                if (small) {
-                    bs[k] = (int)e / a.max_pages;
-                    js[k] = (int)e - bs[k] * a.max_pages;
-                } else {
-                    bs[k] = (int)(e / a.max_pages);
-                    js[k] = (int)(e % a.max_pages);
-                }
-                if (js[k] < cup[bs[k] + 1] - cup[bs[k]])
-                    pid[k] = a.page_ids[cup[bs[k]] + js[k]];
-                else
-                    bs[k] = -2;  // padding entry
+                for (int k = 0; k < kIds; ++k)
+                    id[k] = a.page_ids[min(e0 + 64 * k + lane, hi - 1)];
+#pragma unroll
+                for (int k = 0; k < kIds; ++k)
+                    bad |= id[k] < 0 || id[k] >= a.num_pool_pages;
             }
+            walk = __ballot(bad) != 0;
         }
-        int bad_b = INT_MAX;
-#pragma unroll
-        for (int k = 0; k < kMetaUnroll; ++k) {
-            const long long e = e0 + (long long)k * kMetaThreads;
-            if (bs[k] == -1)
-                continue;  // past the table
-            if (bs[k] >= 0 && (pid[k] < 0 || pid[k] >= a.num_pool_pages))
-                bad_b = min(bad_b, bs[k]);
-            a.page_table[e] = pid[k];
-            if (pt_lds)
-                s_pt[e] = pid[k];
-        }
-        if (bad_b != INT_MAX)
-            atomicMin(&err, bad_b);
+        if (walk)
+            for (int u = 0; u < sessions; ++u) {
+                const int first = __builtin_amdgcn_readlane(my_first, u);
+                const int count = min(__builtin_amdgcn_readlane(my_pages, u), a.max_pages);
+                for (int j = lane; j < count; j += 64) {
+                    const int32_t id = a.page_ids[first + j];
+                    if (id < 0 || id >= a.num_pool_pages)
+                        atomicMin(&err, base + u);
+                }
+            }
     }
+    // Cumulative rows and keys, and the pages that sessions with new rows read.
+    long long total[3] = {0, 0, 0};
     for (int base = 0; base < a.B; base += kMetaThreads) {
         const int b = base + tid;
         long long v[3] = {0, 0, 0}, tot[3];
-        int bad = 0;
+        bool bad = false;
         if (b < a.B) {
-            const long long q = qlen[b], ctx = ctxl[b];
-            const long long npages = (long long)cup[b + 1] - cup[b];
-            const long long kl = ctx + q;
+            const long long q = a.q_len[b], ctx = a.ctx_len[b], kl = ctx + q;
+            const long long npages = (long long)a.cu_pages[b + 1] - a.cu_pages[b];
             const long long need = kl < 0 ? 0 : ceil_div_nn(kl, a.page_size);
             bad = q < 0 || ctx < 0 || npages < 0 || npages > a.max_pages || need > npages;
             v[0] = q;
             v[1] = kl;
             v[2] = q > 0 ? need : 0;
         }
-        block_scan3(v, tot, lds);
+        block_scan<3>(v, tot, lds);
         if (b < a.B) {
-            const long long iq = v[0] + carry[0], ik = v[1] + carry[1];
+            const long long iq = v[0] + total[0], ik = v[1] + total[1];
             if (bad || iq > INT_MAX || ik > INT_MAX || iq > a.max_rows)
                 atomicMin(&err, b);
             a.cu_seqlens_q[b + 1] = (int32_t)iq;
             a.cu_seqlens_k[b + 1] = (int32_t)ik;
-            if (in_lds)
-                s_cuq[b + 1] = (int32_t)iq;
         }
-        __syncthreads();
-        if (tid == 0)
-            for (int k = 0; k < 3; ++k)
-                carry[k] += tot[k];
-        __syncthreads();
+#pragma unroll
+        for (int k = 0; k < 3; ++k)
+            total[k] += tot[k];
     }
+    __syncthreads();
     if (err != INT_MAX) {
-        write_error(a, err);
+        write_error_info(a, err);
         return;
     }
-    const long long total_q = carry[0], total_k = carry[1], total_pages = carry[2];
     long long split = a.split_pages;
     if (split == 0) {
-        split = (total_pages + a.target_blocks - 1) / a.target_blocks;
+        split = (total[2] + a.target_blocks - 1) / a.target_blocks;
         if (split < 1)
             split = 1;
     }
-    __syncthreads();
+    // Split-K work items per session.
+    __shared__ int32_t s_cus[kPlaceMaxSessions + 1];  // cu_splits of a batch to be placed
     if (tid == 0)
-        carry[0] = 0;
-    __syncthreads();
-    // Phase 2: split-K work items per session.
+        s_cus[0] = 0;
+    long long W = 0;
     for (int base = 0; base < a.B; base += kMetaThreads) {
         const int b = base + tid;
-        long long v[3] = {0, 0, 0}, tot[3];
-        if (b < a.B && qlen[b] > 0) {
-            const long long kl = (long long)ctxl[b] + qlen[b];
-            v[0] = ceil_div_nn(ceil_div_nn(kl, a.page_size), split);
-        }
+        long long v[1] = {0}, tot[1];
+        if (b < a.B)
+            v[0] = item_count((long long)a.ctx_len[b] + a.q_len[b], a.q_len[b], a.page_size, split);
         const long long ns = v[0];
-        block_scan3(v, tot, lds);
+        block_scan<1>(v, tot, lds);
         if (b < a.B) {
-            const long long w = v[0] + carry[0];
-            if (w > a.max_work)
+            if (v[0] + W > a.max_work)
                 atomicMin(&err, b);
             a.num_splits[b] = (int32_t)ns;
-            a.cu_splits[b + 1] = (int32_t)w;
-            if (in_lds)
-                s_cus[b + 1] = (int32_t)w;
+            a.cu_splits[b + 1] = (int32_t)(v[0] + W);
+            if (b < kPlaceMaxSessions)
+                s_cus[b + 1] = (int32_t)(v[0] + W);
         }
-        __syncthreads();
-        if (tid == 0)
-            carry[0] += tot[0];
-        __syncthreads();
+        W += tot[0];
     }
+    __syncthreads();
     if (err != INT_MAX) {
-        write_error(a, err);
+        write_error_info(a, err);
         return;
     }
-    const long long W = carry[0];
-    // Phase 3: block-to-session map, work descriptors, slot mapping.
-    __shared__ Placement place[1];
-    const int n = L ? a.placement : 0;
-    if (n > 0) {
-        place_sessions(a.B, n, a.page_size, [&](int b) { return qlen[b]; },
-                       [&](int b) { return ctxl[b]; }, [&](int b) { return cus[b]; }, place[0]);
-        if (placed_slots(place[0], n) > a.max_work) {
-            write_error(a, a.B);  // max_work cannot hold the placed work list
+    __shared__ Placement place;
+    if (a.placement > 0) {
+        place_sessions(a.B, a.placement, a.page_size, [&](int b) { return a.q_len[b]; },
+                                     [&](int b) { return a.ctx_len[b]; },
+                                     [&](int b) { return s_cus[b]; }, place);
+        if (placed_slots(place, a.placement) > a.max_work) {
+            write_error_info(a, a.B);  // max_work cannot hold the placed work list
             return;
         }
+        // For fill_metadata_kernel: the first slot of session b, in the first entry of its page
+        // table row, which workgroup b reads before it writes the row.  The empty slots are
+        // marked here, where the XCDs' counts are.
+        const int n = a.placement;
+        for (int b = tid; b < a.B; b += kMetaThreads)
+            a.page_table[(long long)b * a.max_pages] = place.bin[b] + n * place.k0[b];
+        for (int w = tid; w < a.max_work; w += kMetaThreads)
+            if (w / n >= place.cnt[w % n])
+                a.work_desc[(long long)w * kWorkDescInts] = -1;
     }
-    for (long long w = tid; w < a.max_work; w += kMetaThreads) {
-        const bool empty = n > 0 ? w / n >= place[0].cnt[w % n] : w >= W;
-        if (empty)
-            a.work_desc[w * kWorkDescInts] = -1;
+    if (tid < kInfoInts)
+        a.info[tid] = tid == 0   ? (int32_t)W
+                      : tid == 1 ? (int32_t)split
+                      : tid == 2 ? (int32_t)total[0]
+                      : tid == 3 ? (int32_t)total[1]
+                      : tid == kInfoPlacement ? a.placement
+                                              : 0;
+}
+
+// Workgroup b < B writes session b's row of the page table, its work items and its slots; the
+// workgroups past B mark the empty slots of a work list in session order, kFillSlots each (all
+// slots after a failed plan).
+constexpr int kFillThreads = 256;
+constexpr int kFillSlots = 4096;
+
+__global__ __launch_bounds__(kFillThreads) void fill_metadata_kernel(MetadataArgs a) {
+    const int tid = threadIdx.x, b = blockIdx.x, n = a.placement;
+    const int W = a.info[0];
+    if (b >= a.B) {
+        const long long w0 = (long long)(b - a.B) * kFillSlots;
+        for (long long w = w0 + tid; w < min(w0 + kFillSlots, (long long)a.max_work); w += kFillThreads)
+            if (W < 0 || (n == 0 && w >= W))
+                a.work_desc[w * kWorkDescInts] = -1;
+        return;
     }
-    for (long long u = tid; u < W; u += kMetaThreads) {
-        const int b = upper_index(cus, a.B, u);
-        const int sp = (int)(u - cus[b]);
-        const long long w = n > 0 ? place[0].bin[b] + (long long)n * (place[0].k0[b] + sp) : u;
+    const int first = a.cu_pages[b], listed = min(a.cu_pages[b + 1] - first, a.max_pages);
+    int32_t* row = a.page_table + (long long)b * a.max_pages;
+    const int slot0 = n > 0 ? row[0] : 0;  // placed: the session's first slot, from the plan
+    __syncthreads();
+    for (int j = tid; j < a.max_pages; j += kFillThreads)
+        row[j] = j < listed ? a.page_ids[first + j] : -1;
+    if (W < 0)
+        return;
+    const int split = a.info[1], q = a.q_len[b], ctx = a.ctx_len[b], kl = ctx + q;
+    const int q0 = a.cu_seqlens_q[b], u0 = a.cu_splits[b], ns = a.cu_splits[b + 1] - u0;
+    const int need = (kl + a.page_size - 1) / a.page_size;
+    for (int sp = tid; sp < ns; sp += kFillThreads) {
+        const int u = u0 + sp;
+        const long long w = n > 0 ? slot0 + (long long)n * sp : u;
         int32_t* d = a.work_desc + w * kWorkDescInts;
         int32_t* pg = a.work_pages + w * kWorkPages;
-        const int kl = ctxl[b] + qlen[b];
-        const int need = (kl + a.page_size - 1) / a.page_size;
-        const int p0 = (int)(sp * split);
-        const int p1 = (int)(p0 + split < need ? p0 + split : need);
+        const int p0 = sp * split, p1 = min(need - p0, split) + p0;  // p0 < need
         a.work_session[w] = b;
         a.work_split[w] = sp;
         d[0] = b;
-        d[1] = cuq[b];
+        d[1] = q0;
         d[2] = kl;
         d[3] = p0;
         d[4] = p1;
-        d[5] = cus[b + 1] - cus[b];
-        d[6] = (int32_t)u;
-        d[7] = qlen[b];
+        d[5] = ns;
+        d[6] = u;
+        d[7] = q;
 #pragma unroll
         for (int j = 0; j < kWorkPages; ++j)
-            pg[j] = p0 + j < p1 ? (pt_lds ? s_pt[(long long)b * a.max_pages + p0 + j]
-                                          : a.page_ids[cup[b] + p0 + j])
-                                : -1;
+            pg[j] = p0 + j < p1 ? a.page_ids[first + p0 + j] : -1;
     }
-    for (long long i = tid; i < total_q; i += kMetaThreads) {
-        const int b = upper_index(cuq, a.B, i);
-        const long long pos = (long long)ctxl[b] + (i - cuq[b]);
-        const long long j = pos / a.page_size;
-        const int32_t page = pt_lds ? s_pt[(long long)b * a.max_pages + j] : a.page_ids[cup[b] + j];
-        a.slot_mapping[i] = (int32_t)(page * (long long)a.page_size + pos % a.page_size);
-    }
-    if (tid == 0) {
-        a.info[0] = (int32_t)W;
-        a.info[1] = (int32_t)split;
-        a.info[2] = (int32_t)total_q;
-        a.info[3] = (int32_t)total_k;
-        a.info[kInfoPlacement] = n;
-        for (int k = kInfoPlacement + 1; k < kInfoInts; ++k)
-            a.info[k] = 0;
+    for (int i = tid; i < q; i += kFillThreads) {
+        const int pos = ctx + i;
+        a.slot_mapping[q0 + i] = (int32_t)(a.page_ids[first + pos / a.page_size] *
+                                               (long long)a.page_size +
+                                           pos % a.page_size);
     }
 }
 
@@ -390,29 +386,6 @@ __global__ __launch_bounds__(kMetaThreads) void build_metadata_kernel(MetadataAr
 // all waves write every output, with no global store before the last barrier.  Outputs
 // are bit-identical to build_metadata_kernel's.
 constexpr int kMetaSmallPt = 8192;
-
-// One DPP move of a 64-bit value (both halves with the same control); lanes the
-// control gives no source, and rows outside row_mask, receive 0.
-template <int CTRL, int ROW_MASK>
-__device__ __forceinline__ long long dpp64(long long v) {
-    const int lo = __builtin_amdgcn_update_dpp(0, (int)(uint32_t)v, CTRL, ROW_MASK, 0xf, true);
-    const int hi = __builtin_amdgcn_update_dpp(0, (int)(uint32_t)(v >> 32), CTRL, ROW_MASK, 0xf,
-                                               true);
-    return (long long)(((uint64_t)(uint32_t)hi << 32) | (uint32_t)lo);
-}
-
-// Inclusive scan over the 64 lanes of a wave on DPP moves (no LDS round trips): shifts
-// of 1, 2, 4, 8 lanes within each row of 16, then lane 15 of each row broadcast into
-// the next row (rows 1, 3) and lane 31 into the upper half (rows 2, 3).
-__device__ __forceinline__ long long wave_scan_incl(long long v) {
-    v += dpp64<0x111, 0xf>(v);  // row_shr:1
-    v += dpp64<0x112, 0xf>(v);  // row_shr:2
-    v += dpp64<0x114, 0xf>(v);  // row_shr:4
-    v += dpp64<0x118, 0xf>(v);  // row_shr:8
-    v += dpp64<0x142, 0xa>(v);  // row_bcast:15
-    v += dpp64<0x143, 0xc>(v);  // row_bcast:31
-    return v;
-}
 
 __global__ __launch_bounds__(kMetaThreads) void build_metadata_lds_kernel(MetadataArgs a) {
     __shared__ int32_t s_cup[kMetaLdsCap + 1], s_q[kMetaLdsCap], s_ctx[kMetaLdsCap];
@@ -620,14 +593,21 @@ __global__ __launch_bounds__(256) void append_kernel(AppendArgs a) {
 
 }  // namespace
 
+int metadata_launches(int B, int max_pages) {
+    return B <= kMetaLdsCap && (long long)B * max_pages <= kMetaSmallPt ? 1 : 2;
+}
+
 hipError_t launch_build_metadata(const MetadataArgs& a, hipStream_t stream) {
-    if (a.B <= kMetaLdsCap && (long long)a.B * a.max_pages <= kMetaSmallPt)
+    if (metadata_launches(a.B, a.max_pages) == 1)
         hipLaunchKernelGGL(build_metadata_lds_kernel, dim3(1), dim3(kMetaThreads), 0, stream, a);
-    else if (a.B <= kMetaLdsCap)
-        hipLaunchKernelGGL(build_metadata_kernel<true>, dim3(1), dim3(kMetaThreads), 0, stream, a);
-    else
-        hipLaunchKernelGGL(build_metadata_kernel<false>, dim3(1), dim3(kMetaThreads), 0, stream,
-                           a);
+    else {
+        hipLaunchKernelGGL(plan_metadata_kernel, dim3(1), dim3(kMetaThreads), 0, stream, a);
+        const hipError_t e = hipGetLastError();
+        if (e != hipSuccess)
+            return e;
+        const int marks = (a.max_work + kFillSlots - 1) / kFillSlots;
+        hipLaunchKernelGGL(fill_metadata_kernel, dim3(a.B + marks), dim3(kFillThreads), 0, stream, a);
+    }
     return hipGetLastError();
 }
 

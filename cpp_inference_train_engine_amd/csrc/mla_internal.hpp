@@ -86,6 +86,8 @@ struct PrefillArgs {
     uint16_t* out16;  // as DecodeArgs::out16
 };
 
+// Launches of launch_build_metadata: 1, or 2 for a large page table or session count.
+int metadata_launches(int B, int max_pages);
 hipError_t launch_build_metadata(const MetadataArgs& a, hipStream_t stream);
 // Workspace of decode attention: a head block of fixed size first -- the fused merge's
 // per-session counters (fused calls have placed metadata, B <= kPlaceMaxSessions), then

@@ -77,7 +77,8 @@ const char* mla_last_error(void);
 int mla_abi_version(void);
 
 /* ------------------------------------------------------------------ (a)
- * Ragged-batch metadata, built on the GPU in one launch.  No reference
+ * Ragged-batch metadata, built on the GPU in one launch (two when B > 4096 or
+ * B * max_pages > 8192).  No reference
  * function: the reference keeps one contiguous cache per session
  * (src/infer/inference.cpp:15-18).  Nearest precedent: the Gemma engine's
  * per-row lengths/cursors/write slots (src/infer/gemma.cpp:383-427).
