@@ -18,10 +18,12 @@
 #include "mla_model.hpp"
 
 #include <algorithm>
+#include <atomic>
 #include <cmath>
 #include <cstring>
 #include <mutex>
 #include <string>
+#include <thread>
 #include <vector>
 
 namespace mla {
@@ -67,6 +69,8 @@ struct Engine {
     float* d_logits = nullptr;
     float* d_logits_all = nullptr;  // [max_rows x vocab] for mla_engine_forward (first use)
     int32_t* d_next_all = nullptr;  // [max_rows]
+    int32_t* h_next_all = nullptr;  // [max_rows] pinned, with d_logits_all
+    std::vector<hipEvent_t> copied;  // one per piece of rows_to_host, created on first use
     void* workspace = nullptr;
     size_t ws_bytes = 0;
     // pinned host
@@ -82,6 +86,8 @@ struct Engine {
             (void)hipStreamSynchronize(stream);
         if (model)
             mla_model_destroy(model);
+        for (hipEvent_t ev : copied)
+            (void)hipEventDestroy(ev);
         for (void* p : dev_allocs)
             (void)hipFree(p);
         for (void* p : host_allocs)
@@ -142,10 +148,83 @@ hipError_t copy_page(Engine* E, int32_t dst, int32_t src) {
     return hipSuccess;
 }
 
+// A run of the device logits that goes to one place in the caller's buffer.
+struct RowRun {
+    size_t src;  // first float in d_logits_all (and h_logits_all)
+    float* dst;
+    size_t n;
+};
+
+// Device logits to the caller's (pageable) rows, in pieces: each is copied to the pinned staging
+// buffer on the engine's stream, and threads move the pieces that have landed on while later ones
+// are on their way.  One thread after the last copy took 5 times the copy itself: a fresh buffer of
+// 65 MB costs its page faults, and one core moves about 10 GB/s.
+constexpr size_t kRowPiece = 512 * 1024;  // floats
+constexpr unsigned kRowThreads = 8;
+
+hipError_t rows_to_host(Engine* E, const std::vector<RowRun>& runs) {
+    std::vector<RowRun> pieces;
+    for (const RowRun& r : runs)
+        for (size_t o = 0; o < r.n; o += kRowPiece)
+            pieces.push_back({r.src + o, r.dst + o, std::min(kRowPiece, r.n - o)});
+    hipError_t e = hipSuccess;
+    while (E->copied.size() < pieces.size() && e == hipSuccess) {
+        hipEvent_t ev = nullptr;
+        e = hipEventCreateWithFlags(&ev, hipEventDisableTiming);
+        if (e == hipSuccess)
+            E->copied.push_back(ev);
+    }
+    size_t issued = 0;
+    for (; issued < pieces.size() && e == hipSuccess; ++issued) {
+        const RowRun& r = pieces[issued];
+        e = hipMemcpyAsync(E->h_logits_all + r.src, E->d_logits_all + r.src, r.n * sizeof(float),
+                           hipMemcpyDeviceToHost, E->stream);
+        if (e == hipSuccess)
+            e = hipEventRecord(E->copied[issued], E->stream);
+        ++E->copies;
+    }
+    int device = 0;
+    if (e == hipSuccess)
+        e = hipGetDevice(&device);
+    if (e != hipSuccess) {
+        (void)hipStreamSynchronize(E->stream);
+        return e;
+    }
+    std::atomic<size_t> next{0};
+    std::atomic<int> failed{(int)hipSuccess};
+    auto move = [&]() {
+        hipError_t w = hipSetDevice(device);
+        for (size_t k; (k = next.fetch_add(1)) < pieces.size();) {
+            if (w == hipSuccess)
+                w = hipEventSynchronize(E->copied[k]);
+            if (w != hipSuccess) {
+                failed.store((int)w);
+                continue;
+            }
+            std::memcpy(pieces[k].dst, E->h_logits_all + pieces[k].src, pieces[k].n * sizeof(float));
+        }
+    };
+    const unsigned threads = (unsigned)std::min<size_t>(
+        {kRowThreads, pieces.size(), std::max(1u, std::thread::hardware_concurrency())});
+    std::vector<std::thread> pool;
+    try {
+        for (unsigned t = 1; t < threads; ++t)
+            pool.emplace_back(move);
+    } catch (const std::exception&) {
+        // fewer threads: those that started and this one share the pieces
+    }
+    move();
+    for (std::thread& t : pool)
+        t.join();
+    ++E->host_waits;
+    return static_cast<hipError_t>(failed.load());
+}
+
 // One batched step: session ids[i] appends counts[i] tokens (tokens concatenated in
 // order).  Logits of each session's last new row go to `logits` [n x vocab] (host,
 // may be null), greedy tokens to `next` [n] (host, may be null).  Lengths advance only
-// on success.
+// on success.  all_rows: every row's logits stay in d_logits_all (the caller fetches them, also
+// after MLA_ERR_NUMERICAL), `logits` and `next` are not used.
 // Whether this step's work list is built XCD-placed (each layer's decode attention then one
 // launch): the device supports it, the batch has at most MLA_PLACE_MAX_SESSIONS sessions,
 // and the placed list fits the work capacity.  The slot count repeats mla_build_metadata's
@@ -272,7 +351,7 @@ int step(Engine* E, int n, const int* ids, const int* counts, const uint16_t* to
     }
     float* const d_logits = all_rows ? E->d_logits_all : E->d_logits;
     int32_t* const d_next = all_rows ? E->d_next_all : E->d_next;
-    float* const h_logits = all_rows ? E->h_logits_all : E->h_logits;
+    int32_t* const h_next = all_rows ? E->h_next_all : E->h_out + kHostNext;
     const long long out_rows = all_rows ? rows : n;
     int32_t* h = E->h_in;
     int32_t *h_ctx = h, *h_q = h + n, *h_cup = h + 2 * n, *h_tok = h + 3 * n + 1;
@@ -320,17 +399,16 @@ int step(Engine* E, int n, const int* ids, const int* counts, const uint16_t* to
         if (err == hipSuccess && placed)
             err = hipMemcpyAsync(E->h_out + kHostHead, E->workspace, kHeadInts * sizeof(int32_t),
                                  hipMemcpyDeviceToHost, E->stream);
-        if (err == hipSuccess && !all_rows)
-            err = hipMemcpyAsync(E->h_out + kHostNext, d_next, n * sizeof(int32_t),
+        if (err == hipSuccess)
+            err = hipMemcpyAsync(h_next, d_next, out_rows * sizeof(int32_t),
                                  hipMemcpyDeviceToHost, E->stream);
         if (err == hipSuccess && logits)
-            err = hipMemcpyAsync(h_logits, d_logits,
-                                 (size_t)out_rows * c.vocab_size * sizeof(float),
+            err = hipMemcpyAsync(E->h_logits, d_logits, (size_t)n * c.vocab_size * sizeof(float),
                                  hipMemcpyDeviceToHost, E->stream);
         if (err == hipSuccess)
             err = hipStreamSynchronize(E->stream);
         E->meta_launches += metadata_launches(n, E->max_pages);
-        E->copies += 2 + placed + !all_rows + (logits != nullptr);
+        E->copies += 3 + placed + (logits != nullptr);
         E->host_waits += 1;
         return gpu_status(err, fn);
     };
@@ -364,18 +442,15 @@ int step(Engine* E, int n, const int* ids, const int* counts, const uint16_t* to
         Session& S = E->sessions[ids[i]];
         S.length += counts[i];
         S.revision = E->revision;
-        if (all_rows)
-            continue;
-        finite = finite && E->h_out[kHostNext + i] != -1;
-        open = open && E->h_out[kHostNext + i] != -2;
+        if (!all_rows)
+            open = open && h_next[i] != -2;
         if (next)
-            next[i] = E->h_out[kHostNext + i];
+            next[i] = h_next[i];
     }
-    if (logits && logits != h_logits)
-        std::memcpy(logits, h_logits, (size_t)out_rows * c.vocab_size * sizeof(float));
-    if (all_rows && logits)
-        for (size_t k = 0; k < (size_t)out_rows * c.vocab_size && finite; ++k)
-            finite = std::isfinite(logits[k]);
+    for (long long k = 0; k < out_rows; ++k)  // -1: some logit of the row is not finite
+        finite = finite && h_next[k] != -1;
+    if (logits)
+        std::memcpy(logits, E->h_logits, (size_t)n * c.vocab_size * sizeof(float));
     if (!finite)  // inference.cpp:170-172
         return fail(MLA_ERR_NUMERICAL, "Nonfinite decode output");
     if (!open)  // inference.cpp:375-377
@@ -671,6 +746,8 @@ int mla_engine_forward(void* engine, int batch, int sequence, const uint16_t* id
             e = E->dalloc(E->d_next_all, (size_t)E->max_rows);
         if (e == hipSuccess)
             e = E->halloc(E->h_logits_all, (size_t)E->max_rows * c.vocab_size);
+        if (e == hipSuccess)
+            e = E->halloc(E->h_next_all, (size_t)E->max_rows);
         if (e != hipSuccess) {
             E->d_logits_all = nullptr;
             return gpu_status(e, "mla_engine_forward");
@@ -708,16 +785,19 @@ int mla_engine_forward(void* engine, int batch, int sequence, const uint16_t* id
             for (int i = 0; i < nb; ++i)
                 std::memcpy(toks.data() + (size_t)i * cnt,
                             ids + (size_t)(b0 + i) * sequence + off, (size_t)cnt * 2);
-            const int st = step(E, nb, temp.data(), counts.data(), toks.data(), E->h_logits_all,
-                                nullptr, "mla_engine_forward", true);
+            int st = step(E, nb, temp.data(), counts.data(), toks.data(), nullptr, nullptr,
+                          "mla_engine_forward", true);
             if (st && st != MLA_ERR_NUMERICAL) {
                 release_all();
                 return st;
             }
+            std::vector<RowRun> runs;
+            const size_t run = (size_t)cnt * c.vocab_size;
             for (int i = 0; i < nb; ++i)
-                std::memcpy(logits + ((size_t)(b0 + i) * sequence + off) * c.vocab_size,
-                            E->h_logits_all + (size_t)i * cnt * c.vocab_size,
-                            (size_t)cnt * c.vocab_size * sizeof(float));
+                runs.push_back({i * run, logits + ((size_t)(b0 + i) * sequence + off) * c.vocab_size,
+                                run});
+            if (const int copy = gpu_status(rows_to_host(E, runs), "mla_engine_forward"))
+                st = copy;
             if (st) {  // a non-finite logit: the rows are out, the error stands
                 release_all();
                 return st;

@@ -176,6 +176,11 @@ __device__ __forceinline__ long long placed_slots(const Placement& p, int n) {
 }
 
 // ------------------------------------------------------------- larger batches ----
+// One workgroup did all of this before: filling a table of 64 K entries with a division per
+// entry, and a binary search per work item and row, took 69 us at 500 sessions of up to 8,192
+// tokens (16 of them with 256 new rows) and 29 us at 200 placed decode sessions.  Now the plan
+// takes 6.3 and 10.6 us (two scans and, placed, the deal; latency of one workgroup) and the fill
+// 4.3 and 4.1 us.  Up to kMetaSmallPt entries the single launch stays (7-11 us).
 // Work items of a session of kl keys with q new rows.
 __device__ __forceinline__ long long item_count(long long kl, long long q, long long page_size,
                                                 long long split) {

@@ -83,7 +83,8 @@ def build_metadata(ctx_len, q_len, cu_pages, page_ids, page_size: int, max_pages
                    placement: bool = False, placement_xcds: int | None = None,
                    stream=None) -> RaggedBatch:
     """(a) Build cu_seqlens, padded page tables, slot mapping and the block-to-session
-    map on the GPU (one launch).  Inputs are device int32 tensors.  ``placement``: lay
+    map on the GPU (one launch, two for a large
+    page table).  Inputs are device int32 tensors.  ``placement``: lay
     the work list out so that each session's items run on one XCD (B <= 256; max_work
     must hold ``placed_work_slots``); decode attention over it then merges the split
     partials inside its launch.  ``placement_xcds``: the placed layout for that many XCDs
