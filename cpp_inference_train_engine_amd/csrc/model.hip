@@ -14,8 +14,8 @@
 //               is the combined W_uv.W_o of prepare_projections, inference.cpp:28-46)
 //   g5_kernel   RMSNorm(ffn_norm) -> [w_gate | w_up] -> SwiGLU  (inference.cpp:157-161)
 //   g6_kernel   . w_down + residual  (inference.cpp:162-165)
-// Per step: embed_kernel (token rows, RoPE rows), g7_kernel (final RMSNorm, tied logits
-// h.E^T, inference.cpp:166-168, with a per-workgroup greedy partial) and argmax_kernel
+// Per step: embed_kernel (token rows, RoPE rows), g7_kernel or g7_rows_kernel (final RMSNorm,
+// tied logits h.E^T, inference.cpp:166-168, with a greedy partial per 64 columns) and argmax_kernel
 // (sample_token's greedy rule, inference.cpp:345-380).
 //
 // Every projection is a skinny GEMM on v_mfma_f32_16x16x32_f16 (fp16 operands, fp32
@@ -895,6 +895,47 @@ __device__ __forceinline__ uint64_t row_max16(uint64_t v) {
     return t > v ? t : v;
 }
 
+// A wave's 16 rows x 64 columns of logits: the values, and per row the greedy winner of the
+// group's columns.  v[j]: lane (g, n) holds rows row0 + 4g + i of column 16j + n.
+__device__ __forceinline__ void logits_out(const StepArgs& s, const floatx4 (&v)[kG7Tiles], int row0,
+                                           const float* inv, int part, int parts) {
+    const ModelDims& m = s.dims;
+    const int lane = threadIdx.x & 63, g = lane >> 4, n = lane & 15;
+    uint64_t best[4] = {0, 0, 0, 0};
+    uint64_t nonfinite[4] = {0, 0, 0, 0};  // 1 when some logit of the row is not finite
+#pragma unroll
+    for (int j = 0; j < kG7Tiles; ++j) {
+        const int col = (part * kG7Tiles + j) * 16 + n;
+        const bool valid = col < m.vocab;
+        const bool open = valid && !(s.ban && ((s.ban[col >> 5] >> (col & 31)) & 1u));
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const int row = row0 + 4 * g + i;
+            const float y = v[j][i] * inv[4 * g + i];
+            if (valid && row < s.B)
+                s.logits[(long long)row * m.vocab + col] = y;
+            if (valid && !isfinite(y))
+                nonfinite[i] = 1;
+            const uint64_t k = open ? greedy_key(y, col) : 0;
+            best[i] = k > best[i] ? k : best[i];
+        }
+    }
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        // the 16 lanes of a row hold 16 columns each; lane 15 gathers the row's winner
+        const uint64_t k = row_max16(best[i]);
+        const uint64_t bad = row_max16(nonfinite[i]);
+        const int row = row0 + 4 * g + i;
+        if (n == 15 && row < s.B) {
+            const long long idx = (long long)row * parts + part;
+            const uint32_t ord = (uint32_t)(k >> 32);
+            const uint32_t b = ord & 0x80000000u ? ord ^ 0x80000000u : ~ord;
+            s.arg_v[idx] = k ? __uint_as_float(b) : -INFINITY;
+            s.arg_c[idx] = bad ? -1 : k ? (int)~(uint32_t)k : 0x7fffffff;
+        }
+    }
+}
+
 template <int KW>
 __global__ __launch_bounds__(64 * kWaves) void g7_kernel(StepArgs s) {
     constexpr int NTW = kG7Tiles / (kWaves / kG7KG);
@@ -920,39 +961,100 @@ __global__ __launch_bounds__(64 * kWaves) void g7_kernel(StepArgs s) {
     floatx4 v[kG7Tiles];
     if (!splitk_reduce<4, NTW, kG7KG>(acc, part, mt, v))
         return;
-    uint64_t best[4] = {0, 0, 0, 0};
-    uint64_t nonfinite[4] = {0, 0, 0, 0};  // 1 when some logit of the row is not finite
+    logits_out(s, v, row0 + 16 * mt, inv_s + 16 * mt, blockIdx.x, gridDim.x);
+}
+
+// The same product for many 64 x 64 blocks: each of a workgroup's four waves computes one by
+// itself, K group after K group in g7_kernel's order (the same bits).  g7_kernel's exchange of
+// partial sums takes 131 KB of LDS, so a CU runs one workgroup at a time, about 7 us a round,
+// with nothing to hide its loads and stores behind; here nothing is exchanged, two workgroups
+// share a CU (256 VGPRs), the waves read the same activations, and a column group's workgroups
+// all run on one XCD (grid padded to its count), whose L2 keeps its share of the embedding.
+// d_model 512, vocabulary 16000: 200 rows 28.0 -> 16.7 us, 1000 rows 100 -> 43 us, about 24 us of
+// it products, 11 the 64 MB of logits, 8 the greedy keys.
+constexpr int kG7RowsWaves = 4;
+
+template <int KW>
+__global__ __launch_bounds__(64 * kG7RowsWaves, 2) void g7_rows_kernel(StepArgs s, int parts) {
+    __shared__ float inv_s[64];
+    const ModelDims& m = s.dims;
+    const int row0 = blockIdx.y * 64, part0 = blockIdx.x * kG7RowsWaves;
+    if (part0 >= parts)
+        return;  // the grid is padded to a multiple of the XCDs
+    const int wave = wave_index(), lane = threadIdx.x & 63, g = lane >> 4, n = lane & 15;
+    const int KT = m.d_pad / 32, n_tiles = m.vocab_pad / 16;
+    const int part = min(part0 + wave, parts - 1), nt0 = part * kG7Tiles;
+    RmsPrefetch<8> rms[2];  // 32 rows each
+    rms[0].issue(s.ss_x, m.d_pad / 16, row0, 32);
+    rms[1].issue(s.ss_x, m.d_pad / 16, row0 + 32, 32);
+    const uint16_t *x[4], *w[kG7Tiles];
 #pragma unroll
-    for (int j = 0; j < kG7Tiles; ++j) {
-        const int col = (nt0 + j) * 16 + n;
-        const bool valid = nt0 + j < n_tiles && col < m.vocab;
-        const bool open = valid && !(s.ban && ((s.ban[col >> 5] >> (col & 31)) & 1u));
+    for (int j = 0; j < kG7Tiles; ++j)
+        w[j] = s.embed + (long long)min(nt0 + j, n_tiles - 1) * KT * 512 + lane * 8;
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const int row = row0 + 16 * mt + 4 * g + i;
-            const float y = v[j][i] * inv_s[16 * mt + 4 * g + i];
-            if (valid && row < s.B)
-                s.logits[(long long)row * m.vocab + col] = y;
-            if (valid && !isfinite(y))
-                nonfinite[i] = 1;
-            const uint64_t k = open ? greedy_key(y, col) : 0;
-            best[i] = k > best[i] ? k : best[i];
+    for (int mt = 0; mt < 4; ++mt)
+        x[mt] = s.xw + act_word(min(row0 + 16 * mt + n, s.B - 1), 8 * g, KT);
+    // Step kk of a K group uses buffer kk % kBufs and refills it for the step kBufs later.  The
+    // loop over the groups stays rolled: unrolled, the compiler gathers the loads of all
+    // groups at its top and spills.
+    constexpr int kBufs = KW < 2 ? KW : 2;  // divides KW
+    static_assert(KW % kBufs == 0, "buffers");
+    V8 a[kBufs][4], b[kBufs][kG7Tiles];
+    auto load = [&](int kg, int kk) {
+        const int kt = min(kg + kk * kG7KG, KT - 1) * 512;
+#pragma unroll
+        for (int j = 0; j < kG7Tiles; ++j)
+            b[kk % kBufs][j] = *reinterpret_cast<const V8*>(w[j] + kt);
+#pragma unroll
+        for (int mt = 0; mt < 4; ++mt)
+            a[kk % kBufs][mt] = *reinterpret_cast<const V8*>(x[mt] + kt);
+    };
+#pragma unroll
+    for (int kk = 0; kk < kBufs; ++kk)
+        load(0, kk);
+    floatx4 sum[4][kG7Tiles];
+    zero(sum);
+    auto group = [&](int kg, bool more) {
+        floatx4 acc[4][kG7Tiles];
+        zero(acc);
+#pragma unroll
+        for (int kk = 0; kk < KW; ++kk) {
+            operands_issued();
+            // The activations of a step past KT count as zeros (no branch: it would hold the
+            // accumulators in two places).
+            const uint32_t in = kg + kk * kG7KG < KT ? 0xffffffffu : 0u;
+#pragma unroll
+            for (int mt = 0; mt < 4; ++mt) {
+                const V8 x0 = __builtin_bit_cast(
+                    V8, __builtin_bit_cast(u32x4, a[kk % kBufs][mt]) & in);
+#pragma unroll
+                for (int j = 0; j < kG7Tiles; ++j)
+                    acc[mt][j] = mma(x0, b[kk % kBufs][j], acc[mt][j]);
+            }
+            if (kk + kBufs < KW)
+                load(kg, kk + kBufs);
+            else if (more)
+                load(kg + 1, kk + kBufs - KW);
         }
-    }
+        operands_issued();
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        // the 16 lanes of a row hold 16 columns each; lane 15 gathers the row's winner
-        const uint64_t k = row_max16(best[i]);
-        const uint64_t bad = row_max16(nonfinite[i]);
-        const int row = row0 + 16 * mt + 4 * g + i;
-        if (n == 15 && row < s.B) {
-            const long long idx = (long long)row * gridDim.x + blockIdx.x;
-            const uint32_t ord = (uint32_t)(k >> 32);
-            const uint32_t b = ord & 0x80000000u ? ord ^ 0x80000000u : ~ord;
-            s.arg_v[idx] = k ? __uint_as_float(b) : -INFINITY;
-            s.arg_c[idx] = bad ? -1 : k ? (int)~(uint32_t)k : 0x7fffffff;
-        }
-    }
+        for (int mt = 0; mt < 4; ++mt)
+#pragma unroll
+            for (int j = 0; j < kG7Tiles; ++j)
+                sum[mt][j] += acc[mt][j];
+    };
+#pragma unroll 1
+    for (int kg = 0; kg < kG7KG - 1; ++kg)
+        group(kg, true);
+    group(kG7KG - 1, false);
+    rms[0].finish(m.d_pad / 16, m.d_model, m.eps, inv_s, 32);
+    rms[1].finish(m.d_pad / 16, m.d_model, m.eps, inv_s + 32, 32);
+    __syncthreads();
+    if (part0 + wave >= parts)
+        return;
+#pragma unroll
+    for (int mt = 0; mt < 4; ++mt)
+        logits_out(s, sum[mt], row0 + 16 * mt, inv_s + 16 * mt, part, parts);
 }
 
 // Last row of each session (cu_q[b+1] - 1) to row b of the logits operands: the
@@ -1157,8 +1259,20 @@ hipError_t launch_gather_last(const StepArgs& s, int B, const int32_t* cu_q, uin
 hipError_t launch_logits(const StepArgs& s, hipStream_t st) {
     const ModelDims& m = s.dims;
     const int parts = g7_parts(m);
-    MLA_KW_DISPATCH(kw_variant(ceil_div(m.d_pad / 32, kG7KG)), g7_kernel,
-                    dim3(parts, ceil_div(s.B, 64)), dim3(64 * kWaves), 0, st, s);
+    const int kw = kw_variant(ceil_div(m.d_pad / 32, kG7KG)), chunks = ceil_div(s.B, 64);
+    // g7_kernel up to two rounds of one workgroup a CU.  A step, one layer, us (g7_kernel /
+    // g7_rows_kernel): 500 workgroups (128 rows of 16000 tokens, d_model 512) 53.0 / 53.3, 750
+    // (129 rows) 60.5 / 54.9, 782 (1 row of 50000) 58.0 / 55.4; below, 32 (256 rows of 500)
+    // 49.7 / 56.9.
+    const dim3 rows_grid(round_up_to(ceil_div(parts, kG7RowsWaves), kXcds), chunks);
+    if (parts * chunks <= 512)
+        MLA_KW4_DISPATCH(kw, g7_kernel, dim3(parts, chunks), dim3(64 * kWaves), 0, st, s)
+    else if (kw == 1)
+        hipLaunchKernelGGL(g7_rows_kernel<1>, rows_grid, dim3(64 * kG7RowsWaves), 0, st, s, parts);
+    else if (kw == 2)
+        hipLaunchKernelGGL(g7_rows_kernel<2>, rows_grid, dim3(64 * kG7RowsWaves), 0, st, s, parts);
+    else  // three buffers spill: a third step counts as a third and an empty fourth
+        hipLaunchKernelGGL(g7_rows_kernel<4>, rows_grid, dim3(64 * kG7RowsWaves), 0, st, s, parts);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess)
         return e;
