@@ -58,7 +58,8 @@ struct Engine {
     std::vector<Session> sessions;
     uint64_t steps = 0;
     uint64_t revision = 0;  // bumped by mla_engine_update_weights
-    // stats: model forwards submitted, host waits on the stream, kernels and copies issued
+    // stats: model forwards submitted, host waits on the stream (one a forward, its rows' pieces
+    // included), kernels and copies issued
     uint64_t host_waits = 0, meta_launches = 0, copies = 0;
     // device
     int32_t* d_in = nullptr;  // staged inputs, see step()
@@ -216,7 +217,6 @@ hipError_t rows_to_host(Engine* E, const std::vector<RowRun>& runs) {
     move();
     for (std::thread& t : pool)
         t.join();
-    ++E->host_waits;
     return static_cast<hipError_t>(failed.load());
 }
 
