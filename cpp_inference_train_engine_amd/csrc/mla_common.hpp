@@ -9,6 +9,7 @@
 namespace mla {
 
 typedef _Float16 half8 __attribute__((ext_vector_type(8)));
+typedef _Float16 half4 __attribute__((ext_vector_type(4)));
 typedef __bf16 bf8 __attribute__((ext_vector_type(8)));
 typedef float floatx4 __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
@@ -236,7 +237,6 @@ __host__ __device__ inline long long act_word(long long row, int col, int kt) {
 enum { kRowF32, kRowF16, kRowAny };
 template <bool NT, int OUT, typename Args>
 __device__ __forceinline__ void store_row(const Args& a, long long row, int h, int c, floatx4 v) {
-    typedef _Float16 half4 __attribute__((ext_vector_type(4)));
     if (OUT == kRowF16 || (OUT == kRowAny && a.out16)) {
         const half4 x = {(_Float16)v[0], (_Float16)v[1], (_Float16)v[2], (_Float16)v[3]};
         *reinterpret_cast<half4*>(
@@ -252,7 +252,8 @@ __device__ __forceinline__ void store_row(const Args& a, long long row, int h, i
 template <bool NT, int OUT, typename Args>
 __device__ __forceinline__ void store_row(const Args& a, long long row, int h, int c, float v) {
     if (OUT == kRowF16 || (OUT == kRowAny && a.out16))
-        a.out16[act_word(row, h * a.kv_rank + c, (a.H * a.kv_rank + 31) >> 5)] = F16::from_float(v);
+        a.out16[act_word(row, h * a.kv_rank + c, (a.H * a.kv_rank + 31) >> 5)] =
+            F16::from_float(v);
     else
         a.out[(row * a.H + h) * a.kv_rank + c] = v;
 }

@@ -26,10 +26,11 @@ struct ModelDims {
     int max_seq;   // max_sequence_length: RoPE table rows
     // padded sizes (K dimensions to 32, N dimensions to 16; see above)
     int d_pad;      // d_model -> 32
-    int q_pad;      // q_rank -> 32 (N of w_dq, K of w_q)
+    int q_pad;      // q_rank -> 32 (N of w_dq, K of w_uq)
     int kvw_pad;    // kv_rank + rope -> 16 (N of w_dkv)
-    int kv_pad;     // kv_rank -> 16 (a head's latent columns of w_q)
-    int hq_pad;     // kv_pad + (rope -> 16): a head's columns of w_q
+    int qk_pad;     // qk -> 16 (per-head N of w_uq)
+    int nope_pad;   // nope -> 32 (K of the absorption)
+    int kv_pad;     // kv_rank -> 16 (N of the absorption)
     int ctx_pad;    // H * kv_rank -> 32 (K of the output projection)
     int ff_pad;     // d_ff -> 32 (N of gate/up, K of down)
     int vocab_pad;  // vocab -> 16 (N of the tied logits)
@@ -38,8 +39,8 @@ struct ModelDims {
 struct LayerWeights {
     const float *attn_norm, *q_norm, *kv_norm, *ffn_norm;
     const uint16_t* w_dq_dkv;   // [d x (q_pad + kvw_pad)] tiled: q columns, then kv columns
-    const uint16_t* w_q;        // [q_rank x H*hq_pad] tiled, head h at columns h*hq_pad..: the
-                                // kv_pad latent columns (W_uq_nope . W_uk_h^T), then rope
+    const uint16_t* w_uq;       // [q_rank x H*qk_pad] tiled, head h at columns h*qk_pad..
+    const uint16_t* w_uk;       // H blocks [nope x kv_rank] tiled (W_uk_h^T)
     const uint16_t* w_out;      // [H*kv_rank x d] tiled: combined W_uv.W_o
     const uint16_t* w_gate_up;  // [d x 2*ff_pad] tiled, gate/up tiles interleaved
     const uint16_t* w_down;     // [d_ff x d] tiled
@@ -82,7 +83,7 @@ int g7_parts(const ModelDims& m);
 size_t qkv_lds_bytes(const ModelDims& m);
 hipError_t model_kernel_attributes(const ModelDims& m);
 // Launches of launch_layer_pre for a batch of `rows` rows: 1 (qkv) or 2 (g1, g2).
-int layer_pre_launches(int rows);
+int layer_pre_launches(const ModelDims& m, int rows);
 // first_norm: attn_norm of layer 0
 hipError_t launch_embed(const StepArgs& s, const float* first_norm, hipStream_t st);
 hipError_t launch_layer_pre(const StepArgs& s, const LayerWeights& w, uint16_t* pool,

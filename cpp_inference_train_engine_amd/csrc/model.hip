@@ -4,11 +4,11 @@
 //
 // Per layer, in launch order (y = x.W for every projection, as in ops.cpp:8-18):
 //   g1_kernel   RMSNorm(x, attn_norm) . [w_dq | w_dkv]  (inference.cpp:85-95)
-//   g2_kernel   per head, q_norm(cq) . [W_uq_nope . W_uk_h^T | W_uq_rope]: q_latent with the
-//               absorption folded into the weight (inference.cpp:85-90,121-124) and, after
-//               RoPE, q_rope, both stored in the cache dtype as the MPS graph does
-//               (mps_backend.mm:561); one more workgroup kv_norms the latent, RoPEs the key,
-//               rounds both and appends them to the paged cache (inference.cpp:91-103)
+//   g2_kernel   per head, q_norm(cq) . w_uq, RoPE of the rope columns (q_rope) and the absorption
+//               q_latent = W_uk_h^T q_nope (inference.cpp:85-90,121-124), both stored in the
+//               cache dtype as the MPS graph does (mps_backend.mm:561); one more workgroup
+//               kv_norms the latent, RoPEs the key, rounds both and appends them to the paged
+//               cache (inference.cpp:91-103)
 //   (decode attention partials + merge: decode.hip)
 //   g4_kernel   latent_ctx [H*kv_rank] . out_proj + x  (inference.cpp:154-156; out_proj
 //               is the combined W_uv.W_o of prepare_projections, inference.cpp:28-46)
@@ -304,13 +304,28 @@ __global__ __launch_bounds__(256) void embed_kernel(StepArgs s, const float* nor
 // --------------------------------------------------------------- g1 and g2 ----
 // Between the residual stream x and the attention (inference.cpp:85-103).  g1: per 16 rows and
 // 16-column tile, y = RMSNorm(x, attn_norm) . [w_dq | w_dkv], 8 waves splitting K.  The norms
-// that follow are RMSNorm(v)_c = v_c * inv * w_c with one inv per row, and what follows them is
-// linear, so g1 leaves v o w (cq: fp16, g2's A operand; latent: fp32) with the rows' sums of
-// squares per tile, and g2 applies inv to its products.  g2: wave w of workgroup b owns column
-// tile 4b + w of the H x hq_pad columns of w_q for 16 rows: no split of K (q_rank <= 256), no
-// exchange between waves.
-// Batches of up to 16 rows run both in one launch (qkv_kernel, below), with the same results
-// bit for bit (the same K groups, summed in the same order).
+// that follow are RMSNorm(v)_c = v_c * inv * w_c with one inv per row, so g1 leaves v o w (cq:
+// fp16, g2's A operand; latent: fp32) with the rows' sums of squares per tile, and g2 applies inv
+// to its products.  g2: workgroup h computes head h's queries for 16 rows (q_head), W_uq and W_uk
+// as two products: their product as one fp16 weight falls into fp16's subnormals for small
+// weights (std 0.001: error of q_latent 3.2e-4 -> 2.5e-3) and past its range for large ones.
+// Smaller batches run both in one launch (qkv_kernel, below), with the same results bit for bit
+// (the same K groups, summed in the same order).
+// Block k < head_blocks of head h's w_uq and w_uk tiles (each contiguous per head).
+__device__ __forceinline__ int uq_blocks(const ModelDims& m) {
+    return (m.qk_pad / 16) * (m.q_pad / 32);
+}
+__device__ __forceinline__ int uk_blocks(const ModelDims& m) {
+    return (m.kv_pad / 16) * (m.nope_pad / 32);
+}
+__device__ __forceinline__ int head_blocks(const ModelDims& m) { return uq_blocks(m) + uk_blocks(m); }
+__device__ __forceinline__ const uint16_t* head_block(const ModelDims& m, const uint16_t* w_uq,
+                                                      const uint16_t* w_uk, int h, int k) {
+    const int nq = uq_blocks(m), nk = uk_blocks(m);
+    return k < nq ? w_uq + ((long long)h * nq + k) * 512
+                  : w_uk + ((long long)h * nk + k - nq) * 512;
+}
+
 template <int KW>
 __global__ __launch_bounds__(64 * kWaves) void g1_kernel(StepArgs s, LayerWeights L) {
     __shared__ __attribute__((aligned(16))) floatx4 part[kWaves * 64];
@@ -340,12 +355,10 @@ __global__ __launch_bounds__(64 * kWaves) void g1_kernel(StepArgs s, LayerWeight
     int mt;
     floatx4 v[1];
     if (!splitk_reduce<1, 1, kWaves>(acc, part, mt, v)) {
-        // g2 (next on the stream) runs workgroup b with residue b % 8: its four tiles are
-        // 4 * KTQ contiguous blocks of w_q
-        const int x = block_xcd(), KTQ = m.q_pad / 32, all = m.H * (m.hq_pad / 16) * KTQ;
-        const int wgs = (m.H * (m.hq_pad / 16) + 3) / 4, per = 4 * KTQ;
-        l2_prefetch(x < wgs ? (wgs - x + kXcds - 1) / kXcds * per : 0, [&](int k) {
-            return L.w_q + (long long)min((x + kXcds * (k / per)) * per + k % per, all - 1) * 512;
+        // g2 (next on the stream) runs head h with residue h % 8
+        const int x = block_xcd(), per = head_blocks(m);
+        l2_prefetch(x < m.H ? (m.H - x + kXcds - 1) / kXcds * per : 0, [&](int k) {
+            return head_block(m, L.w_uq, L.w_uk, x + kXcds * (k / per), k % per);
         }, scratch, 1);
         return;
     }
@@ -396,7 +409,8 @@ __device__ __forceinline__ void append_rows(const StepArgs& s, uint16_t* pool, c
     uint16_t* base = pool + (long long)page * m.page_size * width;
     for (int c = threadIdx.x % per; c < width; c += per) {
         if (c < m.kv_rank) {
-            base[latent_word(tiled, off, c, m.page_size, m.kv_rank)] = F16::from_float(yr[c] * inv);
+            base[latent_word(tiled, off, c, m.page_size, m.kv_rank)] =
+                F16::from_float(yr[c] * inv);
         } else {
             const int j = c - m.kv_rank;
             const float2 cs = cs_s[r * (m.rope / 2) + j / 2];
@@ -408,26 +422,116 @@ __device__ __forceinline__ void append_rows(const StepArgs& s, uint16_t* pool, c
 }
 constexpr int kMaxHalfRope = 32;  // rope <= 64 (mla_model_create checks)
 
-// One 16x16 tile of g2's products (rows row0 + 4g + i, column 16t + n of head h's columns),
-// times the rows' q_norm factors: q_latent, or q_rope after RoPE.
-__device__ __forceinline__ void store_q_tile(const StepArgs& s, floatx4 q, int h, int t, int row0,
-                                             const float2 (&cs)[4]) {
-    const ModelDims& m = s.dims;
-    const int lane = threadIdx.x & 63, g = lane >> 4, n = lane & 15, kv_tiles = m.kv_pad / 16;
-    const bool rope = t >= kv_tiles;
-    const int c = 16 * (rope ? t - kv_tiles : t) + n;
+// The sum of a row's n <= 16 partial sums of squares v[0 .. 15], in tile order (one order for every
+// kernel that forms q_norm or kv_norm).
+__device__ __forceinline__ float sum_tiles(const float (&v)[16], int n) {
+    float ss = 0.0f;
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        const int row = row0 + 4 * g + i;
-        if (!rope) {
-            if (row < s.B && c < m.kv_rank)
-                s.q_latent[((long long)row * m.H + h) * m.kv_rank + c] = F16::from_float(q[i]);
+    for (int j = 0; j < 16; ++j)
+        ss += j < n ? v[j] : 0.0f;
+    return ss;
+}
+
+// Head h's queries for rows row0 .. row0 + 15 from the rows' activation cq o q_norm (xq(k): lane
+// (g, n)'s operand of k-step k: row n, columns 32k + 8g ..), by WAVES waves.  Wave w computes column
+// tiles w, w + WAVES, .. of q = cq . w_uq transposed (lane (g, n): columns 4g + i of row n) into LDS
+// (qf, 16 rows of qk_pad + 4 floats, free before the call); after the barrier RoPE of the rope
+// columns goes to q_rope and the nope columns, rounded to fp16, are the operand of q_latent =
+// W_uk_h^T q_nope, of which wave w computes column tiles w, w + WAVES, ...  inv_s, cs_s: the rows'
+// q_norm factors and rotations in LDS, visible after the barrier.  bq / bu: this wave's weight
+// tiles, loaded with the caller's operands.
+constexpr int kQkTiles = 4, kKvTiles = 8, kNopeSteps = 2;  // limits (mla_model_create checks)
+
+template <int WAVES, int KQ>
+struct HeadWeights {
+    static constexpr int QT = (kQkTiles + WAVES - 1) / WAVES, UT = (kKvTiles + WAVES - 1) / WAVES;
+    V8 bq[QT][KQ], bu[UT][kNopeSteps];
+    __device__ __forceinline__ void load(const ModelDims& m, const LayerWeights& L,
+                                         const uint16_t* zeros, int h, int wave, int lane) {
+        const int qk_tiles = m.qk_pad / 16, kv_tiles = m.kv_pad / 16;
+        const int KTQ = m.q_pad / 32, KTU = m.nope_pad / 32;
+#pragma unroll
+        for (int t = 0; t < QT; ++t)
+            if (wave + WAVES * t < qk_tiles)  // scalar, and nothing else writes the registers
+#pragma unroll
+                for (int k = 0; k < KQ; ++k)
+                    bq[t][k] = load_w(L.w_uq, zeros, h * qk_tiles + wave + WAVES * t, k, KTQ, lane);
+#pragma unroll
+        for (int t = 0; t < UT; ++t)
+            if (wave + WAVES * t < kv_tiles)
+#pragma unroll
+                for (int k = 0; k < kNopeSteps; ++k)
+                    bu[t][k] = load_w(L.w_uk, zeros, h * kv_tiles + wave + WAVES * t, k, KTU, lane);
+    }
+};
+
+template <int WAVES, int KQ, typename XQ>
+__device__ __forceinline__ void q_head(const StepArgs& s, const HeadWeights<WAVES, KQ>& w, int h,
+                                       int row0, XQ&& xq, const float* inv_s, const float2* cs_s,
+                                       float* qf) {
+    constexpr int QT = HeadWeights<WAVES, KQ>::QT, UT = HeadWeights<WAVES, KQ>::UT;
+    const ModelDims& m = s.dims;
+    const int wave = wave_index(), lane = threadIdx.x & 63, g = lane >> 4, n = lane & 15;
+    const int KTQ = m.q_pad / 32, ld = m.qk_pad + 4;
+#pragma unroll
+    for (int t = 0; t < QT; ++t) {
+        const int tile = wave + WAVES * t;
+        if (tile >= m.qk_pad / 16)
+            break;
+        floatx4 q = {0, 0, 0, 0};
+#pragma unroll
+        for (int k = 0; k < KQ; ++k)
+            if (k < KTQ)
+                q = mma(w.bq[t][k], xq(k), q);
+        *reinterpret_cast<floatx4*>(qf + n * ld + 16 * tile + 4 * g) = q;
+    }
+    __syncthreads();
+    // q_latent first: nothing waits for RoPE's stores
+    const float inv = inv_s[n];
+    V8 qn[kNopeSteps];
+#pragma unroll
+    for (int k = 0; k < kNopeSteps; ++k) {
+        const int c0 = min(32 * k + 8 * g, m.qk_pad - 8);  // past nope: dropped below
+        const floatx4 a = *reinterpret_cast<const floatx4*>(qf + n * ld + c0);
+        const floatx4 b = *reinterpret_cast<const floatx4*>(qf + n * ld + c0 + 4);
+#pragma unroll
+        for (int e = 0; e < 8; ++e)
+            qn[k][e] = (_Float16)(32 * k + 8 * g + e < m.nope ? (e < 4 ? a[e] : b[e - 4]) * inv : 0.0f);
+    }
+#pragma unroll
+    for (int t = 0; t < UT; ++t) {
+        const int tile = wave + WAVES * t, c = 16 * tile + 4 * g, row = row0 + n;
+        if (tile >= m.kv_pad / 16)
+            break;
+        floatx4 ql = {0, 0, 0, 0};
+#pragma unroll
+        for (int k = 0; k < kNopeSteps; ++k)
+            if (k < m.nope_pad / 32)
+                ql = mma(w.bu[t][k], qn[k], ql);
+        if (row >= s.B)
             continue;
+        uint16_t* out = s.q_latent + ((long long)row * m.H + h) * m.kv_rank + c;
+        if (m.kv_rank % 4 == 0) {  // a lane's four columns, 8 bytes
+            if (c < m.kv_rank)
+                *reinterpret_cast<u32x2*>(out) = __builtin_bit_cast(
+                    u32x2, half4{(_Float16)ql[0], (_Float16)ql[1], (_Float16)ql[2], (_Float16)ql[3]});
+        } else {
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+                if (c + i < m.kv_rank)
+                    out[i] = F16::from_float(ql[i]);
         }
-        const float o = dpp_mov<0xB1>(q[i]);  // quad_perm [1,0,3,2]: the pair's other column
-        const float y = n & 1 ? rope_odd(o, q[i], cs[i]) : rope_even(q[i], o, cs[i]);
-        if (row < s.B && c < m.rope)
-            s.q_rope[((long long)row * m.H + h) * m.rope + c] = F16::from_float(y);
+    }
+    const int rhalf = m.rope / 2;
+    for (int e = threadIdx.x; e < 16 * rhalf; e += 64 * WAVES) {
+        const int r = e / rhalf, jp = 2 * (e % rhalf), row = row0 + r;
+        if (row >= s.B)
+            continue;
+        const float a0 = qf[r * ld + m.nope + jp] * inv_s[r];
+        const float a1 = qf[r * ld + m.nope + jp + 1] * inv_s[r];
+        uint16_t* qr = s.q_rope + ((long long)row * m.H + h) * m.rope + jp;
+        qr[0] = F16::from_float(rope_even(a0, a1, cs_s[e]));
+        qr[1] = F16::from_float(rope_odd(a0, a1, cs_s[e]));
     }
 }
 
@@ -436,81 +540,83 @@ constexpr int kG2Waves = 4;
 template <int KW>
 __global__ __launch_bounds__(64 * kG2Waves) void g2_kernel(StepArgs s, LayerWeights L,
                                                            uint16_t* pool) {
-    __shared__ __attribute__((aligned(16))) float inv_s[16];
-    __shared__ float y_s[16 * (192 + 4)];  // the append workgroup's (kvw_pad <= 192)
+    __shared__ __attribute__((aligned(16))) float qf[16 * (192 + 4)];  // or the appended rows
+    __shared__ float inv_s[16];
     __shared__ int32_t slot_s[16];
     __shared__ float2 cs_s[16 * kMaxHalfRope];
     const ModelDims& m = s.dims;
-    const int wave = wave_index(), lane = threadIdx.x & 63, g = lane >> 4, n = lane & 15;
-    const int row0 = blockIdx.y * 16, KTQ = m.q_pad / 32, hq_tiles = m.hq_pad / 16;
-    const int all = m.H * hq_tiles, wgs = (all + kG2Waves - 1) / kG2Waves;
-    if ((int)blockIdx.x > wgs)
+    const int tid = threadIdx.x, wave = wave_index(), lane = tid & 63, g = lane >> 4, n = lane & 15;
+    const int row0 = blockIdx.y * 16, h = blockIdx.x, rh = m.rope / 2;
+    if (h > m.H)
         return;  // columns are padded to a multiple of 8 (see l2_prefetch)
-    RmsPrefetch<16> rms;
-    if ((int)blockIdx.x == wgs) {  // the append workgroup
-        // every load in flight at once (a thread: 12 columns of row tid / 16, one slot, two
-        // rotations), then from LDS: element by element from memory this workgroup took 9 us
-        rms.issue(s.ss_kv, m.kvw_pad / 16, row0, 16);
-        const int tid = threadIdx.x, row = row0 + tid / 16, ld = m.kvw_pad + 4, rh = m.rope / 2;
+    // every load in flight at once, the rows' rotations (two a thread) and, in the last wave, the
+    // sums of squares of row n among them
+    const bool kv = h == m.H;
+    const int ss_tiles = (kv ? m.kvw_pad : m.q_pad) / 16;
+    float sv[16];
+    if (wave == kG2Waves - 1) {  // scalar, and nothing else writes the registers
+        const float* ss = (kv ? s.ss_kv : s.ss_cq) + (long long)(row0 + n) * ss_tiles;
+#pragma unroll
+        for (int j = 0; j < 16; ++j)
+            sv[j] = ss[min(j, ss_tiles - 1)];
+    }
+    float2 r2[2];
+#pragma unroll
+    for (int k = 0; k < 2; ++k)
+        r2[k] = s.rope_rows[(long long)row0 * rh + min(tid + 256 * k, 16 * rh - 1)];
+    auto row_inputs = [&]() {  // q_norm / kv_norm factors and rotations of the rows, to LDS
+        if (wave == kG2Waves - 1 && g == 0) {
+            const int cols = kv ? m.kv_rank : m.q_rank;
+            inv_s[n] = 1.0f / sqrtf(sum_tiles(sv, ss_tiles) / (float)cols + m.eps);
+        }
+#pragma unroll
+        for (int k = 0; k < 2; ++k)
+            if (tid + 256 * k < 16 * rh)
+                cs_s[tid + 256 * k] = r2[k];
+    };
+    if (kv) {  // the append workgroup: a thread loads 12 columns of row tid / 16 and its slot
+        const int row = row0 + tid / 16, ld = m.kvw_pad + 4;
         float v[12];
 #pragma unroll
         for (int k = 0; k < 12; ++k)
             v[k] = s.ckv[(long long)row * m.kvw_pad + min(16 * k + tid % 16, m.kvw_pad - 1)];
         const int32_t slot = s.slot_mapping[min(row, s.B - 1)];
-        float2 r2[2];
-#pragma unroll
-        for (int k = 0; k < 2; ++k)
-            r2[k] = s.rope_rows[(long long)row0 * rh + min(tid + 256 * k, 16 * rh - 1)];
         operands_issued();
-        rms.finish(m.kvw_pad / 16, m.kv_rank, m.eps, inv_s, 16);
+        row_inputs();
 #pragma unroll
         for (int k = 0; k < 12; ++k)
             if (16 * k < m.kvw_pad)
-                y_s[tid / 16 * ld + 16 * k + tid % 16] = v[k];
+                qf[tid / 16 * ld + 16 * k + tid % 16] = v[k];
         if (tid % 16 == 0)
             slot_s[tid / 16] = row < s.B ? slot : -1;
-#pragma unroll
-        for (int k = 0; k < 2; ++k)
-            if (tid + 256 * k < 16 * rh)
-                cs_s[tid + 256 * k] = r2[k];
         __syncthreads();
-        append_rows(s, pool, y_s, ld, inv_s, slot_s, cs_s);
+        append_rows(s, pool, qf, ld, inv_s, slot_s, cs_s);
         return;
     }
-    rms.issue(s.ss_cq, m.q_pad / 16, row0, 16);
-    const int T = min(kG2Waves * (int)blockIdx.x + wave, all - 1), h = T / hq_tiles, t = T % hq_tiles;
-    BPre<1, KW> bw;
-    bw.load(L.w_q, s.zeros, T, 1, KTQ, 0, 1, lane);
+    HeadWeights<kG2Waves, KW> w;
+    w.load(m, L, s.zeros, h, wave, lane);
     APre16<KW, 1> a;
-    a.load(s.cqw + (long long)row0 * m.q_pad, s.B - row0, KTQ, 0, 1, lane);
-    float2 cs[4];
-    const int rhalf = m.rope / 2, j2 = min((16 * max(t - m.kv_pad / 16, 0) + n) / 2, rhalf - 1);
-#pragma unroll
-    for (int i = 0; i < 4; ++i)
-        cs[i] = s.rope_rows[(long long)(row0 + 4 * g + i) * rhalf + j2];
+    a.load(s.cqw + (long long)row0 * m.q_pad, s.B - row0, m.q_pad / 32, 0, 1, lane);
     operands_issued();
-    floatx4 acc[1][1];
-    zero(acc);
-    mma_steps(acc, bw, [&](int kk, int mt) { return a.x[kk][mt]; });
-    rms.finish(m.q_pad / 16, m.q_rank, m.eps, inv_s, 16);
-    __syncthreads();
-    if (kG2Waves * (int)blockIdx.x + wave >= all)
-        return;
-    store_q_tile(s, acc[0][0] * *reinterpret_cast<const floatx4*>(inv_s + 4 * g), h, t, row0, cs);
+    row_inputs();
+    q_head(s, w, h, row0, [&](int k) { return a.x[k][0]; }, inv_s, cs_s, qf);
 }
 
-// qkv_kernel -- g1 and g2 in one launch for up to 16 rows: workgroup h < H computes head h's
+// qkv_kernel -- g1 and g2 in one launch for smaller batches: workgroup h < H computes head h's
 // queries, workgroup H the cache append.  Both start with g1's split-K GEMM over their column
 // range, so no other workgroup's output is waited for: each head workgroup recomputes the whole
-// cq row it needs for q_norm.  Each of the 9 workgroups (at 8 heads) then pulls 250 KB of
-// weights through one CU's load path, so from 17 rows on two launches, whose workgroups pull
-// 32 KB each, are faster.  A whole step, one launch against two: 278 / 279 us (1 session), 307 /
-// 310 (8), 317 / 325 (16), 314 / 310 (32), 321 / 315 (48), 328 / 322 (64).  Copying the first
-// page of each attention work item into L2 from idle workgroups of these launches, which paid
-// when one slower kernel did all of this (8.9 us at 64 rows; g1 and g2: 4.2 each), now costs
-// more than it saves (399 us without, 416 with every fourth item, 473 with all).
+// cq row it needs for q_norm.  Each of the 9 workgroups (at 8 heads) of 16 rows then pulls 240 KB
+// of weights through one CU's load path, and one workgroup fills a CU; that costs less than a
+// second launch and its round trip until some XCD has more workgroups than CUs (an XCD runs the
+// columns of one residue, see l2_prefetch).  A step of sessions of 100 to 200 tokens, one launch /
+// two, us: 8 heads (the line lies at 256 rows) 17 rows 263 / 276, 64 273 / 287, 128 295 / 308, 256
+// 358 / 374, 320 471 / 439, 640 657 / 589; 16 heads (160 rows) 160 rows 357 / 370, 176 405 / 378; 4
+// heads (512 rows) 512 rows 474 / 492, 528 556 / 533.
 constexpr int kQkvRows = 16;
-constexpr int kQkvMaxRows = 16;
+constexpr int kXcdCus = 32;
+__host__ __device__ inline bool qkv_one_launch(const ModelDims& m, int rows) {
+    return (rows + kQkvRows - 1) / kQkvRows * ((m.H + kXcds) / kXcds) <= kXcdCus;
+}
 constexpr int kQkvMaxTiles = 16;  // q_pad <= 256, kvw_pad <= 192: at most 16 column tiles
 constexpr int kQkvPad = 8;        // fp16 pad of the LDS A-operand rows
 // fp32 pad of the LDS y rows: with a pitch of 36 mod 64 words, the split-K reduction's
@@ -519,7 +625,7 @@ constexpr int kQkvYPad = 36;
 
 // LDS layout of qkv_kernel (bytes), from the model dims.
 struct QkvLds {
-    int part, y, ya, total;
+    int part, y, ya, qf, total;
 };
 __host__ __device__ inline QkvLds qkv_lds(const ModelDims& m) {
     const int nt = max(m.q_pad, m.kvw_pad) / 16;
@@ -527,6 +633,7 @@ __host__ __device__ inline QkvLds qkv_lds(const ModelDims& m) {
     // A head workgroup writes ya where the append workgroup keeps y (neither needs the other).
     QkvLds l;
     l.part = 0;                      // [8 waves][nt][64] floatx4
+    l.qf = 0;                        // [16][qk_pad + 4] fp32, once the partials are summed
     l.y = kWaves * nt * 64 * 16;     // [16][ncol + kQkvYPad] fp32
     l.ya = l.y;                      // [16][q_pad + pad] fp16
     l.total = l.y + kQkvRows * (ncol + kQkvYPad) * 4;
@@ -539,15 +646,17 @@ template <int KC, int NT>
 __global__ __launch_bounds__(64 * kWaves) void qkv_kernel(StepArgs s, LayerWeights L,
                                                           uint16_t* pool) {
     extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
-    constexpr int KQ = NT / 2;  // k-steps of w_q
+    constexpr int KQ = NT / 2;  // k-steps of w_uq
     const ModelDims& m = s.dims;
     const QkvLds lay = qkv_lds(m);
     floatx4* part = reinterpret_cast<floatx4*>(smem + lay.part);
     float* y = reinterpret_cast<float*>(smem + lay.y);
     _Float16* ya = reinterpret_cast<_Float16*>(smem + lay.ya);
+    float* qf = reinterpret_cast<float*>(smem + lay.qf);
     __shared__ float inv_x[kQkvRows];
-    __shared__ __attribute__((aligned(16))) float inv_n[kQkvRows];  // kv_norm factor per row
-    __shared__ float ss_part[kQkvRows][kQkvMaxTiles];  // row sums of squares per column tile
+    __shared__ float inv_n[kQkvRows];  // q_norm / kv_norm factor per row
+    // row sums of squares per column tile (a pitch of 20: the rows' reads start in different banks)
+    __shared__ __attribute__((aligned(16))) float ss_part[kQkvRows][kQkvMaxTiles + 4];
     __shared__ int32_t slot_s[kQkvRows];
     __shared__ float2 cs_s[kQkvRows * kMaxHalfRope];
 
@@ -579,12 +688,7 @@ __global__ __launch_bounds__(64 * kWaves) void qkv_kernel(StepArgs s, LayerWeigh
     for (int j = 0; j < NT; ++j)
         acc[j] = floatx4{0, 0, 0, 0};
     const uint16_t* xw = s.xw + act_word(min(row0 + n, s.B - 1), 8 * g, KT);
-    // Head workgroups also prefetch their w_q tiles (used after the reduction; wave w owns
-    // tiles w and w + 8 of the head's kv_tiles latent and then rope tiles) and the RoPE
-    // rotations of the rows and columns they hold of a rope tile.
-    const int KTQ = m.q_pad / 32, kv_tiles = m.kv_pad / 16, hq_tiles = m.hq_pad / 16;
-    V8 bq[2][KQ];
-    float2 qcs[2][4];
+    HeadWeights<kWaves, KQ> hw;  // head workgroups: used after the reduction
 #pragma unroll
     for (int c = 0; c < KC; ++c) {
         V8 a[2], b[2][NT];
@@ -596,22 +700,8 @@ __global__ __launch_bounds__(64 * kWaves) void qkv_kernel(StepArgs s, LayerWeigh
             for (int j = 0; j < NT; ++j)
                 b[kk][j] = load_w(L.w_dq_dkv, s.zeros, nt0 + min(j, ntv - 1), kt, KT, lane);
         }
-        if (c == 0 && !kv) {
-#pragma unroll
-            for (int t = 0; t < 2; ++t) {
-                const int tile = wave + kWaves * t;
-                if (tile < hq_tiles) {  // scalar, and nothing else writes the registers
-                    const int j2 = (16 * max(tile - kv_tiles, 0) + n) / 2;
-#pragma unroll
-                    for (int k = 0; k < KQ; ++k)
-                        bq[t][k] = load_w(L.w_q, s.zeros, h * hq_tiles + tile, k, KTQ, lane);
-#pragma unroll
-                    for (int i = 0; i < 4; ++i)
-                        qcs[t][i] =
-                            s.rope_rows[(long long)(row0 + 4 * g + i) * rhalf + min(j2, rhalf - 1)];
-                }
-            }
-        }
+        if (c == 0 && !kv)
+            hw.load(m, L, s.zeros, h, wave, lane);
         operands_issued();
 #pragma unroll
         for (int kk = 0; kk < 2; ++kk)
@@ -658,33 +748,23 @@ __global__ __launch_bounds__(64 * kWaves) void qkv_kernel(StepArgs s, LayerWeigh
         }
     }
     __syncthreads();
-    // the norm factors of this lane group's rows 4g + i (ops.cpp:37-44: 1/sqrt(mean(v^2) + eps))
-    floatx4 inv;
+    // the norm factors of the rows (ops.cpp:37-44: 1/sqrt(mean(v^2) + eps))
+    if (wave == kWaves - 1 && g == 0) {
+        float ssv[kQkvMaxTiles];
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
-        inv[i] = 1.0f / sqrtf(sum16(ss_part[4 * g + i][n]) / (float)ncols + m.eps);
+        for (int j = 0; j < kQkvMaxTiles; ++j)
+            ssv[j] = ss_part[n][j];
+        inv_n[n] = 1.0f / sqrtf(sum_tiles(ssv, kQkvMaxTiles) / (float)ncols + m.eps);
+    }
 
     if (kv) {  // ---- kv_norm, RoPE of the key, rounding and the paged append ----
-        if (wave == 0 && n == 0)
-            *reinterpret_cast<floatx4*>(inv_n + 4 * g) = inv;
         __syncthreads();
         append_rows(s, pool, y, ldy, inv_n, slot_s, cs_s);
         return;
     }
-    // ---- (cq o q_norm weight) . w_q[head h], times the row's inv ----
-#pragma unroll
-    for (int t = 0; t < 2; ++t) {
-        const int tile = wave + kWaves * t;
-        if (tile >= hq_tiles)
-            break;
-        floatx4 q = {0, 0, 0, 0};
-#pragma unroll
-        for (int k = 0; k < KQ; ++k)
-            if (k < KTQ)
-                q = mma(*reinterpret_cast<const V8*>(ya + n * (m.q_pad + kQkvPad) + 32 * k + 8 * g),
-                        bq[t][k], q);
-        store_q_tile(s, q * inv, h, tile, row0, qcs[t]);
-    }
+    q_head(s, hw, h, row0, [&](int k) {
+        return *reinterpret_cast<const V8*>(ya + n * (m.q_pad + kQkvPad) + 32 * k + 8 * g);
+    }, inv_n, cs_s, qf);
 }
 
 // ----------------------------------------------------------- g4 and g6 ----
@@ -767,7 +847,8 @@ template <int KW>
 __global__ __launch_bounds__(64 * kWaves) void g6_kernel(StepArgs s, LayerWeights L,
                                                          const float* next_norm,
                                                          const uint16_t* next_dq_dkv,
-                                                         const uint16_t* next_q) {
+                                                         const uint16_t* next_uq,
+                                                         const uint16_t* next_uk) {
     __shared__ __attribute__((aligned(16))) uint16_t pf_scratch[512];
     const ModelDims& m = s.dims;
     const int row0 = blockIdx.y * 16, KT = m.ff_pad / 32;
@@ -782,24 +863,23 @@ __global__ __launch_bounds__(64 * kWaves) void g6_kernel(StepArgs s, LayerWeight
         row0, s.B, [&]() {
             if (!next_dq_dkv)
                 return;
-            if (s.B <= kQkvMaxRows) {
+            if (qkv_one_launch(m, s.B)) {
                 // qkv_kernel runs head h with residue h % 8 and the append workgroup (h = H) with
                 // H % 8: head workgroups read the w_dq tiles, the append one the w_dkv tiles, and
-                // head h its w_q blocks (contiguous per head)
+                // head h its w_uq and w_uk blocks
                 const int x = block_xcd(), KTq = m.d_pad / 32, q_tiles = m.q_pad / 16;
                 const int n_dq = x < m.H ? q_tiles * KTq : 0;
                 const int n_dkv = m.H % kXcds == x ? (m.kvw_pad / 16) * KTq : 0;
-                const int n_q = (m.hq_pad / 16) * (m.q_pad / 32);
+                const int per = head_blocks(m);
                 const int heads = x < m.H ? (m.H - x + kXcds - 1) / kXcds : 0;
-                l2_prefetch(n_dq + n_dkv + heads * n_q, [&](int k) {
+                l2_prefetch(n_dq + n_dkv + heads * per, [&](int k) {
                     if (k < n_dq)
                         return next_dq_dkv + (long long)k * 512;
                     k -= n_dq;
                     if (k < n_dkv)
                         return next_dq_dkv + ((long long)q_tiles * KTq + k) * 512;
                     k -= n_dkv;
-                    const int h = x + kXcds * (k / n_q);
-                    return next_q + ((long long)h * n_q + k % n_q) * 512;
+                    return head_block(m, next_uq, next_uk, x + kXcds * (k / per), k % per);
                 }, pf_scratch, 1);
                 return;
             }
@@ -1167,7 +1247,7 @@ int g7_parts(const ModelDims& m) { return ceil_div(m.vocab_pad / 16, kG7Tiles); 
     default: hipLaunchKernelGGL(KERNEL<4>, __VA_ARGS__); break;                                  \
     }
 
-int layer_pre_launches(int rows) { return rows <= kQkvMaxRows ? 1 : 2; }
+int layer_pre_launches(const ModelDims& m, int rows) { return qkv_one_launch(m, rows) ? 1 : 2; }
 
 size_t qkv_lds_bytes(const ModelDims& m) { return (size_t)qkv_lds(m).total; }
 
@@ -1196,7 +1276,7 @@ hipError_t launch_embed(const StepArgs& s, const float* first_norm, hipStream_t 
 hipError_t launch_layer_pre(const StepArgs& s, const LayerWeights& w, uint16_t* pool,
                             hipStream_t st) {
     const ModelDims& m = s.dims;
-    if (layer_pre_launches(s.B) == 1) {
+    if (qkv_one_launch(m, s.B)) {
         const size_t lds = qkv_lds_bytes(m);
         const dim3 grid(round_up_to(m.H + 1, kXcds), ceil_div(s.B, kQkvRows));  // padded: see l2_prefetch
         const int nt = max(m.q_pad, m.kvw_pad) / 16;  // <= 16 (mla_model_create checks)
@@ -1222,8 +1302,7 @@ hipError_t launch_layer_pre(const StepArgs& s, const LayerWeights& w, uint16_t* 
     hipError_t e = hipGetLastError();
     if (e != hipSuccess)
         return e;
-    const int wgs = ceil_div(m.H * (m.hq_pad / 16), kG2Waves);
-    MLA_KW_DISPATCH(kw_variant(m.q_pad / 32), g2_kernel, dim3(round_up_to(wgs + 1, kXcds), chunks),
+    MLA_KW_DISPATCH(kw_variant(m.q_pad / 32), g2_kernel, dim3(round_up_to(m.H + 1, kXcds), chunks),
                     dim3(64 * kG2Waves), 0, st, s, w, pool);
     return hipGetLastError();
 }
@@ -1245,7 +1324,8 @@ hipError_t launch_layer_post(const StepArgs& s, const LayerWeights& w, const flo
         return e;
     MLA_KW_DISPATCH(kw_variant(ceil_div(m.ff_pad / 32, kWaves)), g6_kernel,
                     dim3(d_tiles, chunks), dim3(64 * kWaves), 0, st, s, w, next_norm,
-                    next ? next->w_dq_dkv : nullptr, next ? next->w_q : nullptr);
+                    next ? next->w_dq_dkv : nullptr, next ? next->w_uq : nullptr,
+                    next ? next->w_uk : nullptr);
     return hipGetLastError();
 }
 

@@ -209,8 +209,9 @@ ModelDims make_dims(const mla_model_config& c, int page_size) {
     m.d_pad = round_up(c.d_model, 32);
     m.q_pad = round_up(c.q_lora_rank, 32);
     m.kvw_pad = round_up(c.kv_lora_rank + c.head_dim_rope, 16);
+    m.qk_pad = round_up(m.qk, 16);
+    m.nope_pad = round_up(c.head_dim_nope, 32);
     m.kv_pad = round_up(c.kv_lora_rank, 16);
-    m.hq_pad = m.kv_pad + round_up(c.head_dim_rope, 16);
     m.ctx_pad = round_up(c.n_heads * c.kv_lora_rank, 32);
     m.ff_pad = round_up(c.d_ff, 32);
     m.vocab_pad = round_up(c.vocab_size, 16);
@@ -243,7 +244,7 @@ hipError_t upload_weights(Model* M, const float* params) {
             }
         e = M->upload(M->rope_tab, tab);
     }
-    std::vector<float> proj((size_t)H * kv * d), absorbed, uk((size_t)nope * kv);
+    std::vector<float> proj((size_t)H * kv * d);
     std::vector<LayerWeights> layers;
     for (int l = 0; l < c.n_layers && e == hipSuccess; ++l) {
         const float* const* P = R.layer.data() + (size_t)l * P_COUNT;
@@ -264,26 +265,20 @@ hipError_t upload_weights(Model* M, const float* params) {
                                   return 0.0f;
                               return P[P_W_DKV][(size_t)k * kvw + (col - m.q_pad)];
                           }));
-        if (e == hipSuccess) {
-            // w_q, head h at columns h*hq_pad ..: the absorption W_uk_h^T folded into the nope
-            // columns of W_uq (fp32 sums, rounded once, like W_uv.W_o below), then the rope
-            // columns of W_uq
-            absorbed.assign((size_t)q * H * kv, 0.0f);
-            for (int h = 0; h < H; ++h) {
-                for (int t = 0; t < nope; ++t)
-                    for (int r = 0; r < kv; ++r)
-                        uk[(size_t)t * kv + r] = P[P_W_UK][(size_t)r * H * nope + h * nope + t];
-                for (int k = 0; k < q; ++k)
-                    add_products(absorbed.data() + ((size_t)k * H + h) * kv, kv,
-                                 P[P_W_UQ] + (size_t)k * H * qk + h * qk, uk.data(), kv, nope);
-            }
-            e = M->upload(w.w_q, pack(q, H * m.hq_pad, m.q_pad, H * m.hq_pad, [&](int k, int col) {
-                              const int h = col / m.hq_pad, cc = col % m.hq_pad;
-                              if (cc < m.kv_pad)
-                                  return cc < kv ? absorbed[((size_t)k * H + h) * kv + cc] : 0.0f;
-                              const int t = nope + cc - m.kv_pad;
-                              return t < qk ? P[P_W_UQ][(size_t)k * H * qk + h * qk + t] : 0.0f;
+        if (e == hipSuccess)  // w_uq: head h at columns h*qk_pad ..
+            e = M->upload(w.w_uq, pack(q, H * m.qk_pad, m.q_pad, H * m.qk_pad, [&](int k, int col) {
+                              const int h = col / m.qk_pad, cc = col % m.qk_pad;
+                              return cc < qk ? P[P_W_UQ][(size_t)k * H * qk + h * qk + cc] : 0.0f;
                           }));
+        if (e == hipSuccess) {  // W_uk_h^T per head: (k = nope index, col = latent index)
+            std::vector<uint16_t> all;
+            for (int h = 0; h < H; ++h) {
+                auto blk = pack(nope, kv, m.nope_pad, m.kv_pad, [&](int k, int col) {
+                    return P[P_W_UK][(size_t)col * H * nope + h * nope + k];
+                });
+                all.insert(all.end(), blk.begin(), blk.end());
+            }
+            e = M->upload(w.w_uk, all);
         }
         if (e == hipSuccess) {  // combined W_uv.W_o (CpuDecoder::prepare_projections, inference.cpp:28-46)
             for (int h = 0; h < H; ++h)
@@ -445,7 +440,7 @@ int model_forward(Model* M, hipStream_t st, int rows, const int32_t* tokens,
         if (e == hipSuccess)
             e = launch_layer_post(s, M->layers[l], next_norm,
                                   l + 1 < m.n_layers ? &M->layers[l + 1] : nullptr, st);
-        launched += layer_pre_launches(rows) + attn_launches + (max_q_len > 1) + 3;
+        launched += layer_pre_launches(m, rows) + attn_launches + (max_q_len > 1) + 3;
     }
     if (e == hipSuccess && rows != B && !all_rows) {  // logits of each session's last row only
         StepArgs t = s;
@@ -488,10 +483,10 @@ int mla_model_create(const mla_model_config* config, const float* params, int ma
         return fail(MLA_ERR_INVALID_ARGUMENT, "mla_model_create: invalid argument");
     const mla_model_config& c = *config;
     const ModelDims m = make_dims(c, page_size);
-    // Shapes the step kernels cover: a head's latent and rope columns within 8 waves x 2
-    // tiles, at most 8 k-steps per split-K wave (d_model, q_lora_rank: 4 with their
-    // on-the-fly norms), fp32 rows read 8 columns at a time.
-    if (m.qk > 64 || m.kv_pad / 16 > 8 || (c.n_heads * c.kv_lora_rank) % 8 ||
+    // Shapes the step kernels cover: a head's q within 4 column tiles and its latent within 8, at
+    // most 8 k-steps per split-K wave (d_model, q_lora_rank: 4 with their on-the-fly norms),
+    // fp32 rows read 8 columns at a time.
+    if (m.qk_pad / 16 > 4 || m.kv_pad / 16 > 8 || (c.n_heads * c.kv_lora_rank) % 8 ||
         c.d_model % 8 || c.q_lora_rank % 8 || m.d_pad > 1024 || m.q_pad > 256 ||
         m.ctx_pad / 32 > 64 || m.ff_pad / 32 > 64)
         return fail(MLA_ERR_UNSUPPORTED,
