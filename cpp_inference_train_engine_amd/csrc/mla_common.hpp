@@ -219,6 +219,14 @@ __host__ __device__ inline long long rope_word(bool tiled, int slot, int c, int 
     return base + (long long)(t * (rope_dim >> 3) + ch) * 128 + n * 8 + e;
 }
 
+// x as fp32 storage would hold it.  A product that is rounded to 16 bits right away may become one
+// v_fma_mix instruction, which rounds once; a value that another route passes through fp32 memory
+// or LDS is rounded twice, and now and then to the other neighbour.
+__device__ __forceinline__ float as_stored(float x) {
+    asm("" : "+v"(x));
+    return x;
+}
+
 // ---- fp16 activations of the model step ------------------------------------------
 // Stored in MFMA-operand order, like the weights: the 16 rows x 32 columns of (row / 16,
 // col / 32) are 512 contiguous words, so that a wave's A-operand load reads 1 KB contiguously
@@ -238,7 +246,8 @@ enum { kRowF32, kRowF16, kRowAny };
 template <bool NT, int OUT, typename Args>
 __device__ __forceinline__ void store_row(const Args& a, long long row, int h, int c, floatx4 v) {
     if (OUT == kRowF16 || (OUT == kRowAny && a.out16)) {
-        const half4 x = {(_Float16)v[0], (_Float16)v[1], (_Float16)v[2], (_Float16)v[3]};
+        const half4 x = {(_Float16)as_stored(v[0]), (_Float16)as_stored(v[1]),
+                         (_Float16)as_stored(v[2]), (_Float16)as_stored(v[3])};
         *reinterpret_cast<half4*>(
             a.out16 + act_word(row, h * a.kv_rank + c, (a.H * a.kv_rank + 31) >> 5)) = x;
         return;
@@ -253,7 +262,7 @@ template <bool NT, int OUT, typename Args>
 __device__ __forceinline__ void store_row(const Args& a, long long row, int h, int c, float v) {
     if (OUT == kRowF16 || (OUT == kRowAny && a.out16))
         a.out16[act_word(row, h * a.kv_rank + c, (a.H * a.kv_rank + 31) >> 5)] =
-            F16::from_float(v);
+            F16::from_float(as_stored(v));
     else
         a.out[(row * a.H + h) * a.kv_rank + c] = v;
 }

@@ -372,7 +372,7 @@ __global__ __launch_bounds__(64 * kWaves) void g1_kernel(StepArgs s, LayerWeight
                 s.ckv[(long long)row * m.kvw_pad + c] = y[i] * (c < m.kv_rank ? wn : 1.0f);
             else
                 s.cqw[act_word(row, c, m.q_pad / 32)] =
-                    F16::from_float(c < m.q_rank ? y[i] * wn : 0.0f);
+                    F16::from_float(as_stored(c < m.q_rank ? y[i] * wn : 0.0f));
         }
     }
     if (kv)
@@ -410,13 +410,13 @@ __device__ __forceinline__ void append_rows(const StepArgs& s, uint16_t* pool, c
     for (int c = threadIdx.x % per; c < width; c += per) {
         if (c < m.kv_rank) {
             base[latent_word(tiled, off, c, m.page_size, m.kv_rank)] =
-                F16::from_float(yr[c] * inv);
+                F16::from_float(as_stored(yr[c] * inv));
         } else {
             const int j = c - m.kv_rank;
             const float2 cs = cs_s[r * (m.rope / 2) + j / 2];
             const float a = yr[m.kv_rank + (j & ~1)], b = yr[m.kv_rank + (j | 1)];
             base[rope_word(tiled, off, j, m.page_size, m.kv_rank, m.rope)] =
-                F16::from_float(j & 1 ? rope_odd(a, b, cs) : rope_even(a, b, cs));
+                F16::from_float(as_stored(j & 1 ? rope_odd(a, b, cs) : rope_even(a, b, cs)));
         }
     }
 }
@@ -741,7 +741,7 @@ __global__ __launch_bounds__(64 * kWaves) void qkv_kernel(StepArgs s, LayerWeigh
             if (kv)
                 y[r * ldy + col] = yv * wc;
             else
-                ya[r * (m.q_pad + kQkvPad) + col] = (_Float16)(yv * wc);
+                ya[r * (m.q_pad + kQkvPad) + col] = (_Float16)as_stored(yv * wc);
             const float sq = sum16(col < ncols ? yv * yv : 0.0f);
             if (n == 0)
                 ss_part[r][j] = sq;
