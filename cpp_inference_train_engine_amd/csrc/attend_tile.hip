@@ -20,6 +20,10 @@
 //                       sum of 16-bit parts that together hold its 22 (fp16: 2 parts) or 24
 //                       (bf16: 3 parts) bits
 //   The waves' states meet in LDS once at the end.
+// A key beyond a row's position, or of weight zero, adds nothing to the row, whatever its latent
+// holds, as in the portable kernels.  The product adds 0 times the latent, so an infinite or NaN
+// latent is zeroed in the slot first.  Such a latent makes the key's score non-finite in every row:
+// a row that sees the key is NaN through its probability, or weighs it 0 (a score of -inf).
 // One slot per wave and no second buffer: with two to five workgroups on a CU the other waves'
 // copies are in flight while one computes, and the LDS it would take halves that count.
 // What bounds it: the latency of the copies, and for wide kv_rank the LDS reads (each row tile
@@ -172,6 +176,25 @@ __global__ __launch_bounds__(64 * kTileWaves) __attribute__((amdgpu_waves_per_eu
                 *reinterpret_cast<u32x4*>(sp + 32 * KV + tt * 16 * RP + c * 8) = zero;
     };
 
+    // Infinite and NaN latents of the unit become 0 (its scores have been computed).
+    auto drop_nonfinite = [&]() {
+        constexpr uint32_t kExp = T::exp_mask;
+#pragma unroll 1
+        for (int k = 0; k < 2 * ks; ++k) {  // both tiles' 512-word blocks are contiguous
+            u32x4* p = reinterpret_cast<u32x4*>(sp + k * 512 + lane * 8);
+            u32x4 v = *p;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                if ((v[e] & kExp) == kExp)
+                    v[e] &= 0xffff0000u;
+                if (((v[e] >> 16) & kExp) == kExp)
+                    v[e] &= 0x0000ffffu;
+            }
+            *p = v;
+        }
+        wave_lds_fence();
+    };
+
     const int s_lane = g * 128 + (n ^ ((g & 1) * kTileRot)) * 8;
     const int tr_par = (n & 3) >> 1;
     const int tr_lane = tr_par * 128 + ((4 * g + (n >> 2)) ^ (tr_par * kTileRot)) * 8 + 4 * (n & 1);
@@ -247,6 +270,11 @@ __global__ __launch_bounds__(64 * kTileWaves) __attribute__((amdgpu_waves_per_eu
                         sc[tt][q] = T::mma32(ka, qv[q][KSM + j], sc[tt][q]);
                 }
 
+        // Not 0 when a score of the first row tile is not finite; tested once the probabilities,
+        // which do not wait for it, are done.
+        floatx4 odd = sc[0][0] * 0.0f + sc[1][0] * 0.0f;
+        odd[0] += odd[1] + (odd[2] + odd[3]);
+
         V8 pb[NP][QT];
 #pragma unroll
         for (int q = 0; q < QT; ++q) {
@@ -293,6 +321,8 @@ __global__ __launch_bounds__(64 * kTileWaves) __attribute__((amdgpu_waves_per_eu
                 }
             l_run[q] += psum;
         }
+        if (__builtin_amdgcn_ballot_w64(odd[0] != 0.0f))
+            drop_nonfinite();
 #pragma unroll
         for (int rt = 0; rt < RTM; ++rt)
             if (rt < 2 * ks) {

@@ -24,6 +24,7 @@ struct F16 {
     using scalar = _Float16;
     using vec8 = half8;
     static constexpr int code = 0;
+    static constexpr uint32_t exp_mask = 0x7c00;  // all ones: infinite or NaN
     // Softmax probabilities enter the P.C MFMA as one fp16 operand (2^-11 relative).
     static constexpr bool split_p = false;
     __device__ static float to_float(uint16_t bits) {
@@ -42,6 +43,7 @@ struct BF16 {
     using scalar = __bf16;
     using vec8 = bf8;
     static constexpr int code = 1;
+    static constexpr uint32_t exp_mask = 0x7f80;
     // bf16 keeps 8 mantissa bits: probabilities enter the P.C MFMA as hi + lo bf16
     // parts (two MFMAs, about 16 bits), so the output stays within the fp32 tolerance.
     static constexpr bool split_p = true;

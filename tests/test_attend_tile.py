@@ -46,3 +46,38 @@ def test_tile_kernel_edges(gpu, orc, H, kv, rope, page, dtype):
         got, lse = _run(gpu, batch, flags=flags, scale=scale)
         np.testing.assert_allclose(got, want, rtol=1e-5, atol=1e-5, err_msg=f"flags={flags}")
         np.testing.assert_allclose(lse, want_lse, rtol=1e-5, atol=1e-5)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("H,kv,rope,page,dtype", [
+    (4, 32, 8, 16, 0), (17, 128, 16, 64, 1), (32, 256, 32, 32, 1), (16, 512, 64, 64, 0)])
+def test_nonfinite_latents_reach_only_the_rows_that_weigh_them(gpu, H, kv, rope, page, dtype):
+    """Infinite and NaN latents of a chunk's token leave the queries before it alone, and make
+    those from it on NaN; a decode row whose score of such a key is -inf does not see it.  As in the
+    portable kernel, and equal to it up to the bound of test_tile_kernel_edges."""
+    from cpp_inference_train_engine_amd.ops import latent_word
+    _say(f"tile kernel, non-finite latents H={H} kv={kv} page={page} dtype={dtype}")
+    batch, scale = _batch(H, kv, rope, page, dtype, seed=7), 1.0 / np.sqrt(kv + rope)
+    one, inf, nan = (0x3C00, 0x7C00, 0x7FC0) if dtype == 0 else (0x3F80, 0x7F80, 0x7FC0)
+    q0 = np.concatenate([[0], np.cumsum(batch.q_len)])
+
+    def put(b, t, c, bits):
+        p = batch.page_ids[batch.cu_pages[b] + t // page]
+        batch.pages[0, p, latent_word(t % page, c, page, kv, rope)] = bits
+
+    batch.q_latent[q0[9]:, :, 3] = one    # a score of inf, and NaN its softmax
+    batch.q_latent[q0[5], :, 5] = one     # decode: a score of -inf
+    clean, _ = _run(gpu, batch, scale=scale)
+    put(9, 267 + 23, 3, inf)              # seen by queries 23.. of 33
+    put(9, 267 + 30, kv - 1, nan)
+    put(8, 9, 0, nan)                     # the session's own tokens only: queries 9.. of 17
+    put(5, 300, 5, 0x8000 | inf)
+    got, lse = _run(gpu, batch, scale=scale)
+    want, want_lse = _run(gpu, batch, flags=1, scale=scale)
+    for first, n, seen in ((q0[9], 33, 23), (q0[8], 17, 9)):
+        assert np.isnan(got[first + seen:first + n]).all()
+        np.testing.assert_allclose(got[first:first + seen], clean[first:first + seen],
+                                   rtol=1e-5, atol=1e-5)
+    assert np.isfinite(got[q0[5]]).all()
+    np.testing.assert_allclose(got, want, rtol=1e-5, atol=1e-5)
+    np.testing.assert_allclose(lse, want_lse, rtol=1e-5, atol=1e-5)
