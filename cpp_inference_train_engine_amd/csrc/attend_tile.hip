@@ -90,9 +90,10 @@ __global__ __launch_bounds__(64 * kTileWaves) __attribute__((amdgpu_waves_per_eu
         const int q0 = a.cu_q[s], q_len = a.cu_q[s + 1] - q0;
         k_len = a.cu_k[s + 1] - a.cu_k[s];
         rb = (gridDim.x - 1 - blockIdx.x) * (16 * QT);  // later queries see more keys: first
-        if (q_len < 2 || rb >= q_len * H)
+        const int rows = min(q_len, a.max_q_len) * H;
+        if (q_len < 2 || rb >= rows)
             return;
-        n_rows = min(16 * QT, q_len * H - rb);
+        n_rows = min(16 * QT, rows - rb);
         ctx = k_len - q_len;
         tile_begin = 0;
         key_end = ctx + (rb + n_rows - 1) / H + 1;

@@ -79,6 +79,7 @@ constexpr int kStatusUnplaced = 2;  // fused flag over metadata not placed for t
 // Chunked-prefill attention (sessions with q_len > 1, causal within the chunk).
 struct PrefillArgs {
     int B, H, kv_rank, rope_dim, page_size, max_pages, num_pool_pages;
+    int max_q_len;     // rows of a longer session past it are not written (set by launch_prefill)
     float scale_log2;  // softmax scale * log2(e)
     const int32_t *cu_q, *cu_k, *page_table, *info;
     const uint16_t *pages, *q_latent, *q_rope;

@@ -91,7 +91,7 @@ void prefill_page_kernel(PrefillArgs a) {
     const int q0 = a.cu_q[b], q_len = a.cu_q[b + 1] - q0;
     const int k_len = a.cu_k[b + 1] - a.cu_k[b];
     const int H = a.H;
-    const int n_rows = q_len * H;
+    const int n_rows = min(q_len, a.max_q_len) * H;
     // Heavier workgroups (later queries see more keys) first.
     const int rb = (gridDim.x - 1 - blockIdx.x) * WG_ROWS;
     if (q_len < 2 || rb >= n_rows)
@@ -523,10 +523,12 @@ bool prefill_mfma_supported(int H, int kv_rank, int rope_dim, int page_size) {
 }
 
 
-hipError_t launch_prefill(const PrefillArgs& a, int max_q_len, int dtype, bool force_generic,
+hipError_t launch_prefill(const PrefillArgs& args, int max_q_len, int dtype, bool force_generic,
                           hipStream_t stream) {
-    if (a.B <= 0 || max_q_len < 2)
+    if (args.B <= 0 || max_q_len < 2)
         return hipSuccess;
+    PrefillArgs a = args;
+    a.max_q_len = max_q_len;
     if (!force_generic && prefill_mfma_supported(a.H, a.kv_rank, a.rope_dim, a.page_size))
         return dtype == 0 ? launch_prefill_page<F16>(a, max_q_len, stream)
                           : launch_prefill_page<BF16>(a, max_q_len, stream);

@@ -34,7 +34,7 @@ def _batch(H, kv, rope, page, dtype, seed):
 @pytest.mark.parametrize("H,kv,rope,page,dtype", [
     (4, 32, 8, 16, 0), (1, 64, 16, 64, 1), (16, 96, 24, 48, 0), (17, 128, 16, 64, 1),
     (20, 128, 64, 32, 0), (33, 64, 40, 16, 1), (8, 128, 32, 64, 0), (32, 256, 32, 32, 1),
-    (12, 224, 8, 64, 0), (16, 288, 64, 16, 1), (16, 512, 64, 64, 0), (40, 512, 56, 64, 1)])
+    (12, 224, 8, 64, 0), (16, 288, 64, 16, 1), (8, 64, 0, 32, 0), (16, 512, 64, 64, 0), (40, 512, 56, 64, 1)])
 def test_tile_kernel_edges(gpu, orc, H, kv, rope, page, dtype):
     """Probabilities keep fp32 precision, so the bound is fp32's: scores of magnitude <= 16 in
     log2 units carry 16 * 2^-24 = 1e-6 into each weight, the sums about as much again."""

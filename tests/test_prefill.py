@@ -197,3 +197,39 @@ def test_prefill_wide_page_table(gpu, orc, max_pages):
     want, want_lse = _oracle(orc, batch)
     _check(got, want, f"max_pages={max_pages}")
     np.testing.assert_allclose(lse, want_lse, rtol=1e-4, atol=1e-3)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("H, kv, rope, page", [(8, 128, 16, 64), (5, 128, 16, 64), (4, 32, 8, 16),
+                                               (7, 64, 16, 64), (3, 24, 4, 16)],
+                         ids=["page8", "page5", "tile4", "tile7", "portable"])
+@pytest.mark.parametrize("max_q", [2, 3, 7])
+def test_prefill_rows_past_max_q_len_are_not_written(gpu, H, kv, rope, page, max_q):
+    """A session with more new rows than max_q_len gets its first max_q_len rows, and no other
+    (the kernels' row blocks do not end there)."""
+    import torch
+    rng = np.random.default_rng(max_q)
+    q = np.array([5, 33, 1, 2], np.int32)
+    ctx = np.array([70, 0, 9, 30], np.int32)
+    need = (ctx + q + page - 1) // page
+    P, rows = int(need.sum()), int(q.sum())
+    draw = lambda *s: torch.from_numpy(rng.standard_normal(s, dtype=np.float32)).cuda().half()
+    pages, ql, qr = draw(P, page * (kv + rope)), draw(rows, H, kv), draw(rows, H, rope)
+    cu = np.concatenate([[0], np.cumsum(need)]).astype(np.int32)
+    rb = gpu.build_metadata(_dev(ctx), _dev(q), _dev(cu), _dev(np.arange(P, dtype=np.int32)), page,
+                            int(need.max()), P, split_pages=4, max_rows=rows)
+    out = {}
+    for m in (max_q, 33):
+        o = torch.full((rows, H, kv), 7.0, device="cuda")
+        l = torch.full((rows, H), 7.0, device="cuda")
+        gpu.prefill_attention(rb, pages, ql, qr, 0.125, kv_rank=kv, rope_dim=rope, max_q_len=m,
+                              dtype=0, out=o, lse=l)
+        out[m] = (o.cpu().numpy(), l.cpu().numpy())
+    rb.read_info()
+    first = np.concatenate([[0], np.cumsum(q)])
+    for b, n in enumerate(q):
+        done = 0 if n < 2 else min(n, max_q)
+        for part, full in zip(out[max_q], out[33]):
+            np.testing.assert_allclose(part[first[b]:first[b] + done], full[first[b]:first[b] + done],
+                                       rtol=RTOL, atol=ATOL)  # the blocks' key ranges differ
+            assert (part[first[b] + done:first[b + 1]] == 7.0).all(), f"session {b}"
