@@ -409,7 +409,12 @@ int model_forward(Model* M, hipStream_t st, int rows, const int32_t* tokens,
     pa.q_rope = M->q_rope;
     pa.out16 = M->ctx;
     pa.lse = nullptr;
-    const bool generic = (reinterpret_cast<uintptr_t>(workspace) & 15) != 0;
+    // The MFMA attention kernels read pages, and write partials, 16 bytes at a time.
+    uintptr_t pool_bits = 0;
+    for (int l = 0; l < m.n_layers; ++l)
+        pool_bits |= reinterpret_cast<uintptr_t>(pages[l]);
+    const bool odd_pools = (pool_bits & 15) != 0;
+    const bool generic = odd_pools || (reinterpret_cast<uintptr_t>(workspace) & 15) != 0;
     a.fused_merge = (md.flags & MLA_DECODE_FUSED_MERGE) && decode_fuses_merge(a, generic);
     if (int bad = fused_checks(a, md.flags, "model forward"))
         return bad;
@@ -436,7 +441,7 @@ int model_forward(Model* M, hipStream_t st, int rows, const int32_t* tokens,
         if (e == hipSuccess && decode_rows && !a.fused_merge)
             e = launch_merge(a, st);
         if (e == hipSuccess && max_q_len > 1)
-            e = launch_prefill(pa, max_q_len, MLA_DTYPE_F16, false, st);
+            e = launch_prefill(pa, max_q_len, MLA_DTYPE_F16, odd_pools, st);
         if (e == hipSuccess)
             e = launch_layer_post(s, M->layers[l], next_norm,
                                   l + 1 < m.n_layers ? &M->layers[l + 1] : nullptr, st);
