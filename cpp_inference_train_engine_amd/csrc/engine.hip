@@ -58,8 +58,7 @@ struct Engine {
     std::vector<Session> sessions;
     uint64_t steps = 0;
     uint64_t revision = 0;  // bumped by mla_engine_update_weights
-    // stats: model forwards submitted, host waits on the stream (one a forward, its rows' pieces
-    // included), kernels and copies issued
+    // stats: model forwards submitted, host waits on the stream, kernels and copies issued
     uint64_t host_waits = 0, meta_launches = 0, copies = 0;
     // device
     int32_t* d_in = nullptr;  // staged inputs, see step()
@@ -157,13 +156,16 @@ struct RowRun {
 };
 
 // Device logits to the caller's (pageable) rows, in pieces: each is copied to the pinned staging
-// buffer on the engine's stream, and threads move the pieces that have landed on while later ones
-// are on their way.  One thread after the last copy took 5 times the copy itself: a fresh buffer of
-// 65 MB costs its page faults, and one core moves about 10 GB/s.
+// buffer on the engine's stream, right behind the forward, and threads move the pieces that have
+// landed on while later ones are on their way.  This is the host's one wait for the forward:
+// landed() is asked once, when the first piece (and so all that was issued before it) is there, and
+// no row is moved on when it says no.  One thread after the last copy took 5 times the copy itself:
+// a fresh buffer of 65 MB costs its page faults, and one core moves about 10 GB/s.
 constexpr size_t kRowPiece = 512 * 1024;  // floats
 constexpr unsigned kRowThreads = 8;
 
-hipError_t rows_to_host(Engine* E, const std::vector<RowRun>& runs) {
+template <typename F>
+hipError_t rows_to_host(Engine* E, const std::vector<RowRun>& runs, F&& landed) {
     std::vector<RowRun> pieces;
     for (const RowRun& r : runs)
         for (size_t o = 0; o < r.n; o += kRowPiece)
@@ -187,10 +189,10 @@ hipError_t rows_to_host(Engine* E, const std::vector<RowRun>& runs) {
     int device = 0;
     if (e == hipSuccess)
         e = hipGetDevice(&device);
-    if (e != hipSuccess) {
-        (void)hipStreamSynchronize(E->stream);
+    if (e == hipSuccess)
+        e = hipEventSynchronize(E->copied[0]);
+    if (e != hipSuccess || !landed())
         return e;
-    }
     std::atomic<size_t> next{0};
     std::atomic<int> failed{(int)hipSuccess};
     auto move = [&]() {
@@ -220,11 +222,6 @@ hipError_t rows_to_host(Engine* E, const std::vector<RowRun>& runs) {
     return static_cast<hipError_t>(failed.load());
 }
 
-// One batched step: session ids[i] appends counts[i] tokens (tokens concatenated in
-// order).  Logits of each session's last new row go to `logits` [n x vocab] (host,
-// may be null), greedy tokens to `next` [n] (host, may be null).  Lengths advance only
-// on success.  all_rows: every row's logits stay in d_logits_all (the caller fetches them, also
-// after MLA_ERR_NUMERICAL), `logits` and `next` are not used.
 // Whether this step's work list is built XCD-placed (each layer's decode attention then one
 // launch): the device supports it, the batch has at most MLA_PLACE_MAX_SESSIONS sessions,
 // and the placed list fits the work capacity.  The slot count repeats mla_build_metadata's
@@ -247,8 +244,14 @@ bool placed_fits(const Engine* E, int n, const int32_t* ctx, const int32_t* q) {
     return (long long)E->n_xcd * *std::max_element(items.begin(), items.end()) <= E->work_cap;
 }
 
+// One batched step: session ids[i] appends counts[i] tokens (tokens concatenated in
+// order).  Logits of each session's last new row go to `logits` [n x vocab] (host,
+// may be null), greedy tokens to `next` [n] (host, may be null).  Lengths advance only
+// on success.  all_rows: every row's logits go where these runs say (also when the step returns
+// MLA_ERR_NUMERICAL), `logits` and `next` are not used.
 int step(Engine* E, int n, const int* ids, const int* counts, const uint16_t* tokens,
-         float* logits, int32_t* next, const char* fn, bool all_rows = false) {
+         float* logits, int32_t* next, const char* fn,
+         const std::vector<RowRun>* all_rows = nullptr) {
     const mla_model_config& c = E->cfg;
     if (n < 1 || n > E->max_sessions || !ids || !counts || !tokens)
         return fail(MLA_ERR_INVALID_ARGUMENT, std::string(fn) + ": invalid batch");
@@ -375,7 +378,8 @@ int step(Engine* E, int n, const int* ids, const int* counts, const uint16_t* to
     int32_t *d_pos = d_tok + rows, *d_ids = d_pos + rows;
     int st = gpu_status(e, fn);
     // Metadata build, forward and read-back of one attempt; placed: the work list XCD-placed
-    // and each layer's decode attention one launch.
+    // and each layer's decode attention one launch.  merged: its fused merges (if any) held.
+    bool merged = true;
     auto attempt = [&](bool placed) {
         int rc = mla_build_metadata(E->stream, n, d_ctx, d_q, d_cup, d_ids, E->page_size,
                                     E->max_pages, E->num_pages, kSplitPages, 1024, E->work_cap,
@@ -389,7 +393,7 @@ int step(Engine* E, int n, const int* ids, const int* counts, const uint16_t* to
                               placed ? MLA_DECODE_FUSED_MERGE : 0};
             rc = model_forward(static_cast<Model*>(E->model), E->stream, (int)rows, d_tok, d_pos,
                                n, max_q, md, E->layer_pools.data(), E->workspace, E->ws_bytes,
-                               d_logits, d_next, all_rows);
+                               d_logits, d_next, all_rows != nullptr);
         }
         if (rc)
             return rc;
@@ -405,8 +409,17 @@ int step(Engine* E, int n, const int* ids, const int* counts, const uint16_t* to
         if (err == hipSuccess && logits)
             err = hipMemcpyAsync(E->h_logits, d_logits, (size_t)n * c.vocab_size * sizeof(float),
                                  hipMemcpyDeviceToHost, E->stream);
-        if (err == hipSuccess)
+        auto landed = [&]() {
+            merged = !placed || decode_head_status(E->h_out + kHostHead) == 0;
+            return merged && E->h_out[kHostInfo] >= 0;
+        };
+        if (err == hipSuccess && all_rows) {
+            err = rows_to_host(E, *all_rows, landed);
+        } else if (err == hipSuccess) {
             err = hipStreamSynchronize(E->stream);
+            if (err == hipSuccess)
+                landed();
+        }
         E->meta_launches += metadata_launches(n, E->max_pages);
         E->copies += 3 + placed + (logits != nullptr);
         E->host_waits += 1;
@@ -415,7 +428,7 @@ int step(Engine* E, int n, const int* ids, const int* counts, const uint16_t* to
     const bool placed = placed_fits(E, n, h_ctx, h_q);
     if (!st)
         st = attempt(placed);
-    if (!st && placed && decode_head_status(E->h_out + kHostHead) != 0) {
+    if (!st && !merged) {
         // A fused merge's premise failed (a session's items did not meet in one L2: this
         // device does not dispatch as probed).  Stop placing, clear the workspace head
         // (status and merge counters) and run the step again through the two-launch path;
@@ -785,21 +798,14 @@ int mla_engine_forward(void* engine, int batch, int sequence, const uint16_t* id
             for (int i = 0; i < nb; ++i)
                 std::memcpy(toks.data() + (size_t)i * cnt,
                             ids + (size_t)(b0 + i) * sequence + off, (size_t)cnt * 2);
-            int st = step(E, nb, temp.data(), counts.data(), toks.data(), nullptr, nullptr,
-                          "mla_engine_forward", true);
-            if (st && st != MLA_ERR_NUMERICAL) {
-                release_all();
-                return st;
-            }
             std::vector<RowRun> runs;
             const size_t run = (size_t)cnt * c.vocab_size;
             for (int i = 0; i < nb; ++i)
                 runs.push_back({i * run, logits + ((size_t)(b0 + i) * sequence + off) * c.vocab_size,
                                 run});
-            if (const int copy = gpu_status(rows_to_host(E, runs), "mla_engine_forward"))
-                st = copy;
-            if (st) {  // a non-finite logit: the rows are out, the error stands
-                release_all();
+            if (const int st = step(E, nb, temp.data(), counts.data(), toks.data(), nullptr, nullptr,
+                                    "mla_engine_forward", &runs)) {
+                release_all();  // after a non-finite logit, the rows are out and the error stands
                 return st;
             }
             off += cnt;

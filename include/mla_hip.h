@@ -306,9 +306,11 @@ int mla_decode_attention_noalloc(void* stream, int B, int n_heads, int kv_rank, 
  * rows must already be appended (mla_append_latent with the metadata's
  * slot_mapping).  Arguments as for mla_decode_attention, plus cu_seqlens_k from
  * the same mla_build_metadata call and max_q_len >= every session's q_len (rows
- * of a longer session past max_q_len are not written).  Rows of sessions with
- * q_len <= 1 are not written (mla_decode_attention covers them).  flags:
- * MLA_DECODE_FORCE_GENERIC selects the portable VALU kernel.  No workspace. */
+ * of a longer session past max_q_len are not written).  The page kernel (kv_rank 128,
+ * rope_dim 16, 64-token pages, n_heads <= 16) works in units of 32 keys: there an infinite or
+ * NaN latent of a later token of the chunk can make the queries before it in its unit NaN.
+ * Rows of sessions with q_len <= 1 are not written (mla_decode_attention covers them).
+ * flags: MLA_DECODE_FORCE_GENERIC selects the portable VALU kernel.  No workspace. */
 int mla_prefill_attention(void* stream, int B, int n_heads, int kv_rank, int rope_dim,
                           int page_size, int dtype, float scale, const int32_t* cu_seqlens_q,
                           const int32_t* cu_seqlens_k, const int32_t* page_table, int max_pages,
@@ -489,7 +491,8 @@ int mla_engine_set_banned(void* engine, const uint16_t* ids, size_t n);
 int mla_engine_update_weights(void* engine, const float* params);
 /* Execution::stats (include/mini_mla/execution.hpp:25-27,33), engine-wide counters since
  * creation: stats[6] = {model forwards submitted (graph_submissions), host waits on the
- * engine's stream (host_waits), kernels launched (metal_kernel_submissions), copies
+ * engine's stream (host_waits: one for each model forward; the rows of mla_engine_forward
+ * are moved on piece by piece within it), kernels launched (metal_kernel_submissions), copies
  * issued, weight revision, steps rerun through the two-launch decode because a fused
  * merge's check failed (after the first such step the engine stops placing work)}. */
 int mla_engine_stats(void* engine, uint64_t* stats);
