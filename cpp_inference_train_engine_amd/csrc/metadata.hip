@@ -178,65 +178,30 @@ __device__ __forceinline__ long long placed_slots(const Placement& p, int n) {
 // ------------------------------------------------------------- larger batches ----
 // One workgroup did all of this before: filling a table of 64 K entries with a division per
 // entry, and a binary search per work item and row, took 69 us at 500 sessions of up to 8,192
-// tokens (16 of them with 256 new rows) and 29 us at 200 placed decode sessions.  Now the plan
-// takes 6.3 and 10.6 us (two scans and, placed, the deal; latency of one workgroup) and the fill
-// 4.3 and 4.1 us.  Up to kMetaSmallPt entries the single launch stays (7-11 us).
-// Work items of a session of kl keys with q new rows.
-__device__ __forceinline__ long long item_count(long long kl, long long q, long long page_size,
-                                                long long split) {
-    return q > 0 ? ceil_div_nn(ceil_div_nn(kl, page_size), split) : 0;
-}
+// tokens (16 of them with 256 new rows) and 26 us at 200 placed decode sessions.  Plan and fill take
+// 9.4 and 13.5 us (two scans and, placed, the deal; latency of one workgroup), and 8.5 us for one
+// session of 15,626 pages (27 by one workgroup, 42 while a session had one wave and one workgroup of
+// these).  Up to kMetaSmallPt entries the single launch stays (7-13 us): with room for 14,336
+// entries it took 11.2 us at 64 sessions of 188 pages, against 8.2, and 20.2 at 200 placed ones of up
+// to 66, against 13.5.  A host that waits for nothing pays 2.7 us for the second launch.
 
 // One workgroup: page-id and length checks, cu_seqlens_q / k, num_splits, cu_splits and info.  On
 // an error info says so, and fill_metadata_kernel empties the work list.
 __global__ __launch_bounds__(kMetaThreads) void plan_metadata_kernel(MetadataArgs a) {
     __shared__ long long lds[3 * kMetaWaves];
-    __shared__ int err;
+    __shared__ int err, bad_list, bad_id;
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int lo = a.cu_pages[0], hi = a.cu_pages[a.B];
     if (tid == 0) {
         err = INT_MAX;
+        bad_list = bad_id = 0;
         a.cu_seqlens_q[0] = a.cu_seqlens_k[0] = a.cu_splits[0] = 0;
     }
     __syncthreads();
-    // Page ids: each wave checks the lists of its share of the sessions, 64 sessions at a time,
-    // as one flat run (consecutive lists are adjacent), kIds loads of a lane in flight.  Only when
-    // that finds a bad id, or a list is too long or negative (then only its first max_pages ids
-    // may be read), the group is walked session by session to name the first bad one.
-    constexpr int kIds = 16;
-    const int per_wave = (a.B + kMetaWaves - 1) / kMetaWaves;
-    const int b_end = min(a.B, (wave + 1) * per_wave);
-    for (int base = wave * per_wave; base < b_end; base += 64) {
-        const int mine = min(base + lane, a.B - 1), sessions = min(64, b_end - base);
-        const int my_first = a.cu_pages[mine], my_pages = a.cu_pages[mine + 1] - my_first;
-        bool walk = __ballot(my_pages < 0 || my_pages > a.max_pages) != 0;
-        if (!walk) {
-            const int lo = __builtin_amdgcn_readlane(my_first, 0);
-            const int hi = __builtin_amdgcn_readlane(my_first + my_pages, sessions - 1);
-            bool bad = false;
-            for (int e0 = lo; e0 < hi; e0 += 64 * kIds) {
-                int32_t id[kIds];
-#pragma unroll
-                for (int k = 0; k < kIds; ++k)
-                    id[k] = a.page_ids[min(e0 + 64 * k + lane, hi - 1)];
-#pragma unroll
-                for (int k = 0; k < kIds; ++k)
-                    bad |= id[k] < 0 || id[k] >= a.num_pool_pages;
-            }
-            walk = __ballot(bad) != 0;
-        }
-        if (walk)
-            for (int u = 0; u < sessions; ++u) {
-                const int first = __builtin_amdgcn_readlane(my_first, u);
-                const int count = min(__builtin_amdgcn_readlane(my_pages, u), a.max_pages);
-                for (int j = lane; j < count; j += 64) {
-                    const int32_t id = a.page_ids[first + j];
-                    if (id < 0 || id >= a.num_pool_pages)
-                        atomicMin(&err, base + u);
-                }
-            }
-    }
-    // Cumulative rows and keys, and the pages that sessions with new rows read.
-    long long total[3] = {0, 0, 0};
+    // Cumulative rows and keys, and the pages that sessions with new rows read.  What the later
+    // phases need of the first sessions stays in registers and LDS (the page ids pass between).
+    __shared__ int32_t s_q[kPlaceMaxSessions], s_ctx[kPlaceMaxSessions];
+    long long first_pages = 0, total[3] = {0, 0, 0};
     for (int base = 0; base < a.B; base += kMetaThreads) {
         const int b = base + tid;
         long long v[3] = {0, 0, 0}, tot[3];
@@ -245,10 +210,18 @@ __global__ __launch_bounds__(kMetaThreads) void plan_metadata_kernel(MetadataArg
             const long long q = a.q_len[b], ctx = a.ctx_len[b], kl = ctx + q;
             const long long npages = (long long)a.cu_pages[b + 1] - a.cu_pages[b];
             const long long need = kl < 0 ? 0 : ceil_div_nn(kl, a.page_size);
+            if (npages < 0 || npages > a.max_pages)
+                bad_list = 1;
             bad = q < 0 || ctx < 0 || npages < 0 || npages > a.max_pages || need > npages;
             v[0] = q;
             v[1] = kl;
             v[2] = q > 0 ? need : 0;
+            if (base == 0)
+                first_pages = v[2];
+            if (b < kPlaceMaxSessions) {
+                s_q[b] = (int32_t)q;
+                s_ctx[b] = (int32_t)ctx;
+            }
         }
         block_scan<3>(v, tot, lds);
         if (b < a.B) {
@@ -262,6 +235,36 @@ __global__ __launch_bounds__(kMetaThreads) void plan_metadata_kernel(MetadataArg
         for (int k = 0; k < 3; ++k)
             total[k] += tot[k];
     }
+    __syncthreads();
+    // Page ids: consecutive lists are adjacent, so all threads check them as one flat run, kIds loads
+    // of a lane in flight (wave by session, one session of 15,626 pages took 26 us more).  Only when
+    // that finds a bad id, or a list is too long or negative (then only its first max_pages ids may
+    // be read), each wave walks every 16th session to name the first bad one.
+    constexpr int kIds = 16;
+    if (!bad_list) {
+        for (int e0 = lo; e0 < hi; e0 += kMetaThreads * kIds) {
+            int32_t id[kIds];
+#pragma unroll
+            for (int k = 0; k < kIds; ++k)
+                id[k] = a.page_ids[min(e0 + kMetaThreads * k + tid, hi - 1)];
+            bool bad = false;
+#pragma unroll
+            for (int k = 0; k < kIds; ++k)
+                bad |= id[k] < 0 || id[k] >= a.num_pool_pages;
+            if (bad)
+                bad_id = 1;
+        }
+    }
+    __syncthreads();
+    if (bad_list || bad_id)
+        for (int b = wave; b < a.B; b += kMetaWaves) {
+            const int first = a.cu_pages[b], count = min(a.cu_pages[b + 1] - first, a.max_pages);
+            for (int j = lane; j < count; j += 64) {
+                const int32_t id = a.page_ids[first + j];
+                if (id < 0 || id >= a.num_pool_pages)
+                    atomicMin(&err, b);
+            }
+        }
     __syncthreads();
     if (err != INT_MAX) {
         write_error_info(a, err);
@@ -281,8 +284,12 @@ __global__ __launch_bounds__(kMetaThreads) void plan_metadata_kernel(MetadataArg
     for (int base = 0; base < a.B; base += kMetaThreads) {
         const int b = base + tid;
         long long v[1] = {0}, tot[1];
-        if (b < a.B)
-            v[0] = item_count((long long)a.ctx_len[b] + a.q_len[b], a.q_len[b], a.page_size, split);
+        if (b < a.B) {
+            const long long q = base == 0 ? 0 : a.q_len[b];
+            const long long pages =
+                base == 0 ? first_pages : q > 0 ? ceil_div_nn(a.ctx_len[b] + q, a.page_size) : 0;
+            v[0] = ceil_div_nn(pages, split);
+        }
         const long long ns = v[0];
         block_scan<1>(v, tot, lds);
         if (b < a.B) {
@@ -302,9 +309,8 @@ __global__ __launch_bounds__(kMetaThreads) void plan_metadata_kernel(MetadataArg
     }
     __shared__ Placement place;
     if (a.placement > 0) {
-        place_sessions(a.B, a.placement, a.page_size, [&](int b) { return a.q_len[b]; },
-                                     [&](int b) { return a.ctx_len[b]; },
-                                     [&](int b) { return s_cus[b]; }, place);
+        place_sessions(a.B, a.placement, a.page_size, [&](int b) { return s_q[b]; },
+                       [&](int b) { return s_ctx[b]; }, [&](int b) { return s_cus[b]; }, place);
         if (placed_slots(place, a.placement) > a.max_work) {
             write_error_info(a, a.B);  // max_work cannot hold the placed work list
             return;
@@ -328,16 +334,20 @@ __global__ __launch_bounds__(kMetaThreads) void plan_metadata_kernel(MetadataArg
                                               : 0;
 }
 
-// Workgroup b < B writes session b's row of the page table, its work items and its slots; the
-// workgroups past B mark the empty slots of a work list in session order, kFillSlots each (all
-// slots after a failed plan).
+// Workgroups (b < B, y) write session b's row of the page table, its work items and its slots: one
+// workgroup a session where sessions are many, more for a few long ones (fill_slices).  Workgroups
+// (B .., 0) mark the empty slots of a work list in session order, kFillSlots each (all slots after
+// a failed plan).
 constexpr int kFillThreads = 256;
 constexpr int kFillSlots = 4096;
 
 __global__ __launch_bounds__(kFillThreads) void fill_metadata_kernel(MetadataArgs a) {
-    const int tid = threadIdx.x, b = blockIdx.x, n = a.placement;
+    const int tid = threadIdx.x, b = blockIdx.x, y = blockIdx.y, n = a.placement;
+    const int t0 = y * kFillThreads + tid, step = gridDim.y * kFillThreads;
     const int W = a.info[0];
     if (b >= a.B) {
+        if (y > 0)
+            return;
         const long long w0 = (long long)(b - a.B) * kFillSlots;
         for (long long w = w0 + tid; w < min(w0 + kFillSlots, (long long)a.max_work); w += kFillThreads)
             if (W < 0 || (n == 0 && w >= W))
@@ -346,16 +356,19 @@ __global__ __launch_bounds__(kFillThreads) void fill_metadata_kernel(MetadataArg
     }
     const int first = a.cu_pages[b], listed = min(a.cu_pages[b + 1] - first, a.max_pages);
     int32_t* row = a.page_table + (long long)b * a.max_pages;
-    const int slot0 = n > 0 ? row[0] : 0;  // placed: the session's first slot, from the plan
+    // placed: the session's first slot, from the plan; slice 0 writes the row's first entry, so it
+    // alone reads it, and writes the items
+    const bool items = n == 0 || y == 0;
+    const int slot0 = n > 0 && y == 0 ? row[0] : 0;
     __syncthreads();
-    for (int j = tid; j < a.max_pages; j += kFillThreads)
+    for (int j = t0; j < a.max_pages; j += step)
         row[j] = j < listed ? a.page_ids[first + j] : -1;
     if (W < 0)
         return;
     const int split = a.info[1], q = a.q_len[b], ctx = a.ctx_len[b], kl = ctx + q;
     const int q0 = a.cu_seqlens_q[b], u0 = a.cu_splits[b], ns = a.cu_splits[b + 1] - u0;
     const int need = (kl + a.page_size - 1) / a.page_size;
-    for (int sp = tid; sp < ns; sp += kFillThreads) {
+    for (int sp = n > 0 ? tid : t0; items && sp < ns; sp += n > 0 ? kFillThreads : step) {
         const int u = u0 + sp;
         const long long w = n > 0 ? slot0 + (long long)n * sp : u;
         int32_t* d = a.work_desc + w * kWorkDescInts;
@@ -375,7 +388,7 @@ __global__ __launch_bounds__(kFillThreads) void fill_metadata_kernel(MetadataArg
         for (int j = 0; j < kWorkPages; ++j)
             pg[j] = p0 + j < p1 ? a.page_ids[first + p0 + j] : -1;
     }
-    for (int i = tid; i < q; i += kFillThreads) {
+    for (int i = t0; i < q; i += step) {
         const int pos = ctx + i;
         a.slot_mapping[q0 + i] = (int32_t)(a.page_ids[first + pos / a.page_size] *
                                                (long long)a.page_size +
@@ -388,8 +401,10 @@ __global__ __launch_bounds__(kFillThreads) void fill_metadata_kernel(MetadataArg
 // page ids in LDS (one load round trip each); wave 0 alone runs both scans, 64 sessions
 // per pass with the running total carried between passes (a 6-step wave scan instead of
 // a 1024-thread block scan, whose 64-bit shuffles and barriers cost microseconds); then
-// all waves write every output, with no global store before the last barrier.  Outputs
-// are bit-identical to build_metadata_kernel's.
+// all waves write every output, with no global store before the last barrier.  A valid batch's
+// outputs are bit-identical to those of plan_metadata_kernel and fill_metadata_kernel; of a rejected
+// one, info and the emptied work list are (those two also leave a page table and cumulative
+// lengths, which nothing reads then).
 constexpr int kMetaSmallPt = 8192;
 
 __global__ __launch_bounds__(kMetaThreads) void build_metadata_lds_kernel(MetadataArgs a) {
@@ -602,6 +617,12 @@ int metadata_launches(int B, int max_pages) {
     return B <= kMetaLdsCap && (long long)B * max_pages <= kMetaSmallPt ? 1 : 2;
 }
 
+// Workgroups of a session: about one a CU in all, with 4 rows or table entries a thread or more.
+static int fill_slices(const MetadataArgs& a) {
+    const int most = std::max(a.max_pages, a.max_rows) / (4 * kFillThreads) + 1;
+    return std::max(1, std::min(256 / a.B, most));
+}
+
 hipError_t launch_build_metadata(const MetadataArgs& a, hipStream_t stream) {
     if (metadata_launches(a.B, a.max_pages) == 1)
         hipLaunchKernelGGL(build_metadata_lds_kernel, dim3(1), dim3(kMetaThreads), 0, stream, a);
@@ -611,7 +632,8 @@ hipError_t launch_build_metadata(const MetadataArgs& a, hipStream_t stream) {
         if (e != hipSuccess)
             return e;
         const int marks = (a.max_work + kFillSlots - 1) / kFillSlots;
-        hipLaunchKernelGGL(fill_metadata_kernel, dim3(a.B + marks), dim3(kFillThreads), 0, stream, a);
+        hipLaunchKernelGGL(fill_metadata_kernel, dim3(a.B + marks, fill_slices(a)),
+                           dim3(kFillThreads), 0, stream, a);
     }
     return hipGetLastError();
 }

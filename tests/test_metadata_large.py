@@ -67,3 +67,57 @@ def test_table_shapes(gpu, orc, B, longest):
                                   want["work_desc"][:W])
     np.testing.assert_array_equal(rb.slot_mapping[:int(want["info"][2])].cpu().numpy(),
                                   want["slot_mapping"][:int(want["info"][2])])
+
+
+def _long(need, q, ps=16):
+    """Sessions of `need` pages each, the last `q` tokens of each new."""
+    need, q = np.asarray(need), np.asarray(q)
+    cu_pages = np.concatenate([[0], np.cumsum(need)])
+    P = int(cu_pages[-1]) + 3
+    ids = np.random.default_rng(len(need)).permutation(P)[:cu_pages[-1]]
+    return need * ps - 5 - q, q, cu_pages, ids, P, int(need.max())
+
+
+@pytest.mark.parametrize("placed", [False, True])
+@pytest.mark.parametrize("need,q", [([8193], [1]), ([9000], [5000]), ([2800, 1, 2731], [1024, 1, 1023]),
+                                    ([700, 1100, 1, 2100], [1, 1, 0, 1]), ([70] * 127, [1] * 127)])
+def test_long_sessions(gpu, orc, need, q, placed):
+    """A session's row of the table and its slots are written by several workgroups when sessions
+    are few: every output against the oracle."""
+    import torch
+    from test_placement import _placed
+    ctx, q, cu_pages, ids, P, max_pages = _long(need, q)
+    B, n = len(q), gpu.xcd_count() if placed else 0
+    assert B * max_pages > 8192
+    max_work = 65535
+    want = orc.build_metadata(ctx, q, cu_pages, ids, 16, max_pages, P, 3, 512, max_work,
+                              placement_xcds=n) if placed else \
+        orc.build_metadata(ctx, q, cu_pages, ids, 16, max_pages, P, 3, 512, max_work)
+    _say(f"long sessions B={B} max_pages={max_pages} rows={q.sum()} placed={placed}")
+    rb = _placed(gpu, ctx, q, cu_pages, ids, 16, max_pages, P, 3, max_work, placement=placed)
+    torch.cuda.synchronize()
+    assert rb.read_info() == want["info"].tolist()
+    W, T = int(want["info"][0]), int(want["info"][2])
+    occ = want["occupied"] if placed else np.arange(max_work) < W
+    desc = rb.work_desc.cpu().numpy().reshape(-1, 8)[:max_work]
+    np.testing.assert_array_equal(desc[:, 0] >= 0, occ)
+    sel = (lambda x: x[occ]) if placed else (lambda x: x[:W])
+    np.testing.assert_array_equal(desc[occ], sel(want["work_desc"]))
+    np.testing.assert_array_equal(rb.work_pages.cpu().numpy().reshape(-1, 8)[:max_work][occ],
+                                  sel(want["work_pages"]))
+    np.testing.assert_array_equal(rb.page_table[:B * max_pages].cpu().numpy(),
+                                  want["page_table"].reshape(-1))
+    np.testing.assert_array_equal(rb.slot_mapping[:T].cpu().numpy(), want["slot_mapping"][:T])
+
+
+@pytest.mark.parametrize("where", [0, 1023, 1024, 16383, 16384, 20000, -1])
+@pytest.mark.parametrize("need", [[25001], [9000, 16001], [5000, 1, 20000]])
+def test_bad_id_of_a_long_session(gpu, where, need):
+    ctx, q, cu_pages, ids, P, max_pages = _long(need, [1] * len(need))
+    ids = ids.copy()
+    ids[where] = P if where % 2 else -1
+    session = int(np.searchsorted(cu_pages, where % len(ids), side="right")) - 1
+    _say(f"bad id {where} of sessions of {need} pages")
+    rb = _gpu_metadata(gpu, ctx, q, cu_pages, ids, 16, max_pages, P, 4, 512, 65535, len(need))
+    assert rb.info.cpu().numpy().tolist() == [-1, session, 0, 0, 0, 0, 0, 0]
+    assert np.all(rb.work_desc.cpu().numpy().reshape(-1, 8)[:, 0] == -1)
