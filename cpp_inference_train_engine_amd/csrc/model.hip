@@ -20,11 +20,12 @@
 //
 // Every projection is a skinny GEMM on v_mfma_f32_16x16x32_f16 (fp16 operands, fp32
 // accumulation).  A workgroup owns 16 rows (64 for the logits) and one to four 16-column
-// output tiles; its 8 waves split K.  Each wave fetches its weight tiles (fp16, TILED:
-// each wave load reads 1 KB contiguously) and its slice of the activation rows into
-// registers at kernel start, so a GEMM pays about one memory round trip, and the
-// partial sums meet in LDS.  Small row blocks keep the bytes each CU must pull low:
-// the load phase, not the arithmetic, is what these kernels wait on.
+// output tiles; its 8 waves split K and the partial sums meet in LDS (g2_kernel, a head a workgroup,
+// and g7_rows_kernel, 64 columns a wave, do not split K).  Each wave fetches its weight tiles (fp16,
+// TILED: each wave load reads 1 KB contiguously) and its slice of the activation rows into
+// registers at kernel start, so a GEMM pays about one memory round trip.  Small row blocks keep
+// the bytes each CU must pull low: the load phase, not the arithmetic, is what these kernels wait
+// on.
 //
 // RMSNorm (ops.cpp:33-45) is RMSNorm(x)_k = x_k * inv * w_k with inv = 1/rms(x) per row,
 // so RMSNorm(x).W = inv * ((x o w).W): the kernel that writes an activation x also

@@ -50,6 +50,47 @@ def test_tile_kernel_edges(gpu, orc, H, kv, rope, page, dtype):
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("H,kv,rope,page,dtype", [
+    (4, 32, 8, 16, 0), (16, 64, 16, 64, 1), (20, 128, 32, 32, 0), (32, 256, 32, 32, 1),
+    (16, 512, 64, 64, 0)])
+def test_scores_that_rise_and_fall_along_the_keys(gpu, orc, H, kv, rope, page, dtype):
+    """Scores between 0 and 40 log2 units, rising and falling along the keys: the reference maximum
+    of a wave is raised again, and its sums and accumulators rescaled, when a later unit passes the
+    first one's maximum by more than 8 units.  Bound: a score of 40 units (27.7 nats), summed in
+    fp32 from up to 576 products, carries about 27.7 * 2^-24 * sqrt(576) = 4e-5 into its weight, in
+    the oracle as well."""
+    from cpp_inference_train_engine_amd.ops import latent_word
+    from cpp_inference_train_engine_amd.workloads import to_bits
+    batch, scale = _batch(H, kv, rope, page, dtype, seed=11), 1.0 / np.sqrt(kv + rope)
+    rng = np.random.default_rng(12)
+    u = rng.standard_normal(kv, dtype=np.float32)
+    near = 0.02 * rng.standard_normal(batch.q_latent.shape, dtype=np.float32)
+    batch.q_latent[:] = to_bits(u + near, dtype)
+    batch.q_rope[:] = to_bits(0.1 * rng.standard_normal(batch.q_rope.shape, dtype=np.float32), dtype)
+    raised = 0
+    for b, n in enumerate(batch.k_len):
+        t = np.arange(int(n))
+        f = 40 * np.abs((t / 350 + b % 2) % 2 - 1)  # log2 units, peaks 700 keys apart
+        row = f[:, None] / (1.4427 * scale * (u @ u)) * u
+        bits = to_bits((row + 0.05 * rng.standard_normal((len(t), kv))).astype(np.float32), dtype)
+        pg = batch.page_ids[batch.cu_pages[b] + t // page]
+        batch.pages[0, pg[:, None],
+                    latent_word(t[:, None] % page, np.arange(kv)[None], page, kv, rope)] = bits
+        # split_pages = 4 pages an item for decode rows; wave w takes every 4th unit of 32 keys
+        span = 4 * page if batch.q_len[b] == 1 else int(n)
+        for first in range(0, int(n), span):
+            units = [f[i:min(i + 32, first + span)].max() for i in range(first, min(int(n), first + span), 32)]
+            raised += sum(max(units[w + 4::4], default=0) > units[w] + 9 for w in range(min(4, len(units))))
+    assert raised > 0
+    _say(f"tile kernel, rising scores H={H} kv={kv} dtype={dtype}: {raised} waves rescale")
+    want, want_lse = _oracle(orc, batch, scale=scale)
+    for flags in (0, 1):
+        got, lse = _run(gpu, batch, flags=flags, scale=scale)
+        np.testing.assert_allclose(got, want, rtol=1e-4, atol=1e-4, err_msg=f"flags={flags}")
+        np.testing.assert_allclose(lse, want_lse, rtol=1e-5, atol=1e-4)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("H,kv,rope,page,dtype", [
     (4, 32, 8, 16, 0), (17, 128, 16, 64, 1), (32, 256, 32, 32, 1), (16, 512, 64, 64, 0)])
 def test_nonfinite_latents_reach_only_the_rows_that_weigh_them(gpu, H, kv, rope, page, dtype):
     """Infinite and NaN latents of a chunk's token leave the queries before it alone, and make

@@ -258,13 +258,11 @@ def test_model_step_mla36m_matches_oracle(gpu, orc, B, max_ctx, seed):
 @pytest.mark.gpu
 @pytest.mark.parametrize("lengths", ["config3", "short"])
 def test_model_step_read_ahead_changes_no_bit(gpu, lengths):
-    """The L2 read-ahead of the attention's pages during qkv_kernel (default) against the
-    same placed step without it (MLA_STEP_NO_READ_AHEAD), on identical copies of the pools:
-    logits, greedy tokens and every page of every layer (the appended rows included) equal
-    bit for bit.  A read-ahead copy of the page being appended to would make the attention
-    miss the new token.  config3: 64 sessions of 128-4096 tokens; short: 64 sessions of
-    1-200 tokens, where an item's first page is often the page being appended to (the
-    read-ahead must skip it)."""
+    """MLA_STEP_NO_READ_AHEAD is accepted and changes nothing, and a placed step repeats itself:
+    the step with and without the flag, on identical copies of the pools, gives logits, greedy
+    tokens and every page of every layer (the appended rows included) equal bit for bit.  config3:
+    64 sessions of 128-4096 tokens; short: 64 sessions of 1-200 tokens, where an item's first page
+    is often the page being appended to."""
     import torch
     import oracle
     import cpp_inference_train_engine_amd as mla
@@ -292,7 +290,7 @@ def test_model_step_read_ahead_changes_no_bit(gpu, lengths):
                       np.stack([p.view(torch.int16).cpu().numpy() for p in pools]))
         del pools
     model.close()
-    _say(f"read-ahead vs none: max |logit diff| {np.abs(out[True][0] - out[False][0]).max():.3e}")
+    _say(f"with and without the flag: max |logit diff| {np.abs(out[True][0] - out[False][0]).max():.3e}")
     assert np.array_equal(out[True][0].view(np.uint32), out[False][0].view(np.uint32))
     assert np.array_equal(out[True][1], out[False][1])
     assert np.array_equal(out[True][2], out[False][2])
