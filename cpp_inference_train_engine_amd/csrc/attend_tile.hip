@@ -4,8 +4,8 @@
 // rope_dim % 8 == 0 up to 64, page_size % 16 == 0.
 //
 // Same math as decode_page_kernel and prefill_page_kernel (src/infer/inference.cpp:116-153;
-// src/model/ops.cpp:109-142), with the probabilities at fp32 precision: every other route of
-// these shapes (the portable kernels) keeps them in fp32.
+// src/model/ops.cpp:109-142), with the probabilities in 22 bits (fp16) or 24 (bf16): the other
+// route of these shapes, the portable kernels, keeps them in fp32.
 //
 // attend_tile_kernel -- a workgroup of 4 waves owns QT 16-row tiles of q-rows: 16 QT heads of
 //   one query (decode; one work item of the split-K list), or 16 QT consecutive (query, head)
@@ -24,14 +24,20 @@
 // holds, as in the portable kernels.  The product adds 0 times the latent, so an infinite or NaN
 // latent is zeroed in the slot first.  Such a latent makes the key's score non-finite in every row:
 // a row that sees the key is NaN through its probability, or weighs it 0 (a score of -inf).
-// One slot per wave and no second buffer: with two to five workgroups on a CU the other waves'
-// copies are in flight while one computes, and the LDS it would take halves that count.
+// One slot per wave and no second buffer: five, three and two workgroups fit a CU's LDS at kv_rank
+// up to 64, 128 and 256, so that other waves' copies are in flight while one computes, and a second
+// buffer would halve that count; above 256 one workgroup fits, whose four waves have only each other.
 // What bounds it: the latency of the copies, and for wide kv_rank the LDS reads (each row tile
 // reads the unit twice).  The portable kernels it replaces for these shapes are bound by 2-byte
-// loads and serial VALU sums.  Measured, call with merge: 32 sessions of ~1.8k tokens, 32 heads,
-// kv_rank 256, rope 32, 32-token pages, bf16: 30.8 us (1.06 TB/s) against 1546 us; 4 chunks of
-// 129 tokens on contexts up to 1000, 16 heads, kv_rank 64, rope 16, fp16: 15.1 us (64 TFLOP/s)
-// against 836 us.  Error against 64 bits 2.4e-7 and 1.7e-7 (portable: 2.8e-7 and 3.6e-7).
+// loads and serial VALU sums.  Measured, us against the portable kernels', and the error against 64
+// bits (portable in brackets): decode with merge, 32 sessions of ~1.8k tokens: 32 heads, kv_rank
+// 256, rope 32, 32-token pages, bf16 31.7 (1.03 TB/s) against 1543, 2.4e-7 (2.9e-7); 16 heads,
+// kv_rank 512, rope 64, bf16 61.7 against 1655, 3.6e-7 (4.8e-7), fp16 58.5 against 1526, 4.0e-7
+// (8.7e-7).  4 chunks of 129 tokens on contexts up to 1000, 16 heads: kv_rank 64, rope 16, fp16 15.5
+// (62 TFLOP/s) against 839, 1.7e-7 (3.5e-7); kv_rank 512, rope 64, bf16 101 against 4843, 3.8e-7
+// (5.2e-7).  Over kv_rank 32 to 512 and 2 to 1000 keys the error lies between 0.25 and 1.0 times
+// the portable kernels', but for 2 to 4 keys at kv_rank 32 (7.6e-8, 6.6e-8); a third fp16 part
+// changes none of these.
 #include "mla_common.hpp"
 #include "mla_internal.hpp"
 
@@ -404,7 +410,11 @@ hipError_t launch_one(const Args& a, dim3 grid, hipStream_t stream) {
 }
 
 // Rows of a workgroup: two row tiles share each copied unit up to kv_rank 128 when there are
-// rows for both.  Above it O^T and Q^T of two tiles exceed 256 registers (28-60 spilled), and
+// rows for both.  Two tiles against one in us: large calls 131.6 / 135.6 (250 sessions of ~4k
+// tokens, 32 heads, kv 128), 54.3 / 66.5 (the same, kv 32), 184 / 224 (8 chunks of 700, 16 heads,
+// kv 64); calls that leave the chip idle lose, since half as many workgroups share the work: 17.0 /
+// 15.3 (32 sessions of ~1.8k tokens, 32 heads, kv 128), 15.5 / 13.6 (4 chunks of 129, 16 heads, kv
+// 64).  Above kv_rank 128 O^T and Q^T of two tiles exceed 256 registers (28-60 spilled), and
 // the two tiles go to two workgroups that share an L2 instead: 33.4 us against 44.3 us at 32
 // heads and kv_rank 256 (41.8 us with one wave per SIMD and no spills), 30.8 us once the two
 // workgroups were placed on one XCD.
