@@ -79,12 +79,12 @@ constexpr int kStatusUnplaced = 2;  // fused flag over metadata not placed for t
 // Chunked-prefill attention (sessions with q_len > 1, causal within the chunk).
 struct PrefillArgs {
     int B, H, kv_rank, rope_dim, page_size, max_pages, num_pool_pages;
-    int max_q_len;     // rows of a longer session past it are not written (set by launch_prefill)
     float scale_log2;  // softmax scale * log2(e)
     const int32_t *cu_q, *cu_k, *page_table, *info;
     const uint16_t *pages, *q_latent, *q_rope;
     float *out, *lse;
     uint16_t* out16;  // as DecodeArgs::out16
+    int max_q_len;    // rows of a longer session past it are not written (set by launch_prefill)
 };
 
 // Launches of launch_build_metadata: 1, or 2 for a large page table or session count.

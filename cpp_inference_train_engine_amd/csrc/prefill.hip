@@ -91,7 +91,7 @@ void prefill_page_kernel(PrefillArgs a) {
     const int q0 = a.cu_q[b], q_len = a.cu_q[b + 1] - q0;
     const int k_len = a.cu_k[b + 1] - a.cu_k[b];
     const int H = a.H;
-    const int n_rows = min(q_len, a.max_q_len) * H;
+    const int n_rows = q_len * H;
     // Heavier workgroups (later queries see more keys) first.
     const int rb = (gridDim.x - 1 - blockIdx.x) * WG_ROWS;
     if (q_len < 2 || rb >= n_rows)
@@ -384,7 +384,7 @@ void prefill_page_kernel(PrefillArgs a) {
             o[gg] += *reinterpret_cast<const floatx4*>(xo + ((q * RT + rt) * 64 + gg * 16 + rn) * 4) * f;
     }
     const int row = rb + r;
-    if (row >= n_rows)
+    if (row >= min(n_rows, a.max_q_len * H))
         return;
     const long long fr = (long long)q0 * H + row;
     const float inv = L > 0.0f ? 1.0f / L : 0.0f;
