@@ -606,7 +606,7 @@ __global__ __launch_bounds__(64 * kG2Waves) void g2_kernel(StepArgs s, LayerWeig
 // qkv_kernel -- g1 and g2 in one launch for smaller batches: workgroup h < H computes head h's
 // queries, workgroup H the cache append.  Both start with g1's split-K GEMM over their column
 // range, so no other workgroup's output is waited for: each head workgroup recomputes the whole
-// cq row it needs for q_norm.  Each of the 9 workgroups (at 8 heads) of 16 rows then pulls 240 KB
+// cq row it needs for q_norm.  Each of the 9 workgroups (at 8 heads) of 16 rows then pulls 230 KB
 // of weights through one CU's load path, and one workgroup fills a CU; that costs less than a
 // second launch and its round trip until some XCD has more workgroups than CUs (an XCD runs the
 // columns of one residue, see l2_prefetch).  A step of sessions of 100 to 200 tokens, one launch /
